@@ -35,20 +35,19 @@ __global__ __launch_bounds__(256) void axpy_kernel(long N, T alpha, const T *__r
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += stride) y[i * incy] += alpha * x[i * incx];
 }
 
-// Unit strides, 16-byte aligned x and y: 16 bytes per thread per step.
+// Unit strides: 16 bytes per thread per step, at any element alignment.
 template <typename T>
 __global__ __launch_bounds__(256) void axpy_vec_kernel(long N, T alpha, const T *__restrict__ x, T *__restrict__ y) {
-    typedef typename Vec16<T, 16 / sizeof(T)>::type V;
-    constexpr int W = 16 / sizeof(T);
+    typedef typename Vec16<T>::type V;
+    constexpr int W = Vec16<T>::W;
     const long nv = N / W;
     const long stride = (long)gridDim.x * blockDim.x;
     const V *xv = reinterpret_cast<const V *>(x);
     V *yv = reinterpret_cast<V *>(y);
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < nv; i += stride) {
         V a = xv[i], b = yv[i];
-        T *pa = reinterpret_cast<T *>(&a), *pb = reinterpret_cast<T *>(&b);
 #pragma unroll
-        for (int j = 0; j < W; ++j) pb[j] = fma(alpha, pa[j], pb[j]);
+        for (int j = 0; j < W; ++j) b[j] = fma(alpha, a[j], b[j]);
         yv[i] = b;
     }
     // tail (fewer than W elements), one thread
@@ -160,7 +159,7 @@ int axpy(int N, T alpha, const T *x, int incx, T *y, int incy, hipStream_t s) {
     if (N == 0 || alpha == T(0)) return UGEMM_OK;
     if (!x || !y) return fail(UGEMM_ERR_ARG, "axpy: NULL vector");
     const int cus = device_cu_count();
-    if (incx == 1 && incy == 1 && ugemm_aligned16(x) && ugemm_aligned16(y)) {
+    if (incx == 1 && incy == 1) {
         // One 16-byte vector per thread (the grid-stride loop only matters
         // beyond 2^28 vectors): a grid capped at 8 blocks per CU looped
         // with two loads in flight per wave at a time.

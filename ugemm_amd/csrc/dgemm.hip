@@ -15,6 +15,8 @@
 // split-K call adds its partial slices in a fixed order (no atomics), so
 // repeated calls are bitwise identical.
 // Semantics as dgemm_cpu (ugemm.h:162-286) with the BLAS beta == 0 rule.
+#include <type_traits>
+
 #include "internal.h"
 #include "kernel_common.h"
 
@@ -32,7 +34,7 @@ struct DCfg {
 
 // Split-K (gridDim.y > 1): block (tile, z) multiplies K columns
 // [z*kc, min(K, (z+1)*kc)) into the partial slice ws + z*M*N (row length N).
-template <class CF, bool TA, bool TB, int VEC>
+template <class CF, bool TA, bool TB>
 __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) void dgemm_mfma_kernel(
     int M, int N, int K_, double alpha_, const double *__restrict__ A_, long lda, const double *__restrict__ B_,
     long ldb, double beta_, double *__restrict__ C_, long ldc_, int tiles_m, int tiles_n, int kc,
@@ -56,27 +58,34 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int wm = w >> 1, wn = w & 1;
 
-    using ARegs = TileRegs<double, TA ? BM : BK, TA ? BK : BM, NT, VEC>;
-    using BRegs = TileRegs<double, TB ? BK : BN, TB ? BN : BK, NT, VEC>;
+    using ARegs = TileRegs<double, TA ? BM : BK, TA ? BK : BM, NT>;
+    using BRegs = TileRegs<double, TB ? BK : BN, TB ? BN : BK, NT>;
     ARegs ra;
     BRegs rb;
     const bool interior = (m0 + BM <= M) && (n0 + BN <= N);
+    const bool wide_a = (TA ? M : K) >= 2, wide_b = (TB ? K : N) >= 2;
     const int ktiles = (K + BK - 1) / BK, kfull = K / BK;
 
-    auto load_tile = [&](int kt) {
+    // EDGE tiles reach past M, N or K.
+    auto load_tile = [&](int kt, auto edge) {
         const int k0 = kt * BK;
         const double *a0 = TA ? A + (long)k0 * lda + m0 : A + (long)m0 * lda + k0;
         const double *b0 = TB ? B + (long)n0 * ldb + k0 : B + (long)k0 * ldb + n0;
-        if (interior && kt < kfull) {
-            ra.template load<false>(a0, lda, t, 0, 0);
-            rb.template load<false>(b0, ldb, t, 0, 0);
+        if constexpr (!decltype(edge)::value) {
+            ra.load(a0, lda, t);
+            rb.load(b0, ldb, t);
         } else {
             const int mr = M - m0, nr = N - n0, kr = K - k0;
-            ra.template load<true>(a0, lda, t, TA ? mr : kr, TA ? kr : mr);
-            rb.template load<true>(b0, ldb, t, TB ? kr : nr, TB ? nr : kr);
+            ra.load_edge(a0, lda, t, TA ? mr : kr, TA ? kr : mr, wide_a);
+            rb.load_edge(b0, ldb, t, TB ? kr : nr, TB ? nr : kr, wide_b);
         }
     };
-    auto store_tile = [&](int buf) {
+    auto store_tile = [&](int kt, int buf, auto edge) {
+        if constexpr (decltype(edge)::value) {
+            const int mr = M - m0, nr = N - n0, kr = K - kt * BK;
+            ra.mask(t, TA ? mr : kr, TA ? kr : mr, wide_a);
+            rb.mask(t, TB ? kr : nr, TB ? nr : kr, wide_b);
+        }
         ra.template store<TA, LDA>(As + buf * BK * LDA, t);
         rb.template store<!TB, LDB>(Bs + buf * BK * LDB, t);
     };
@@ -87,17 +96,23 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = doublex4{0.0, 0.0, 0.0, 0.0};
 
-    if (ktiles > 0) {
-        load_tile(0);
-        store_tile(0);
+    // K tiles below nfast are loaded without bounds; the others (all of an
+    // edge tile's, and a K remainder) as edges, in a loop of their own.
+    const int nfast = interior ? kfull : 0;
+    if (nfast > 0) {
+        load_tile(0, std::false_type());
+        store_tile(0, 0, std::false_type());
+    } else if (ktiles > 0) {
+        load_tile(0, std::true_type());
+        store_tile(0, 0, std::true_type());
     }
     __syncthreads();
 
     const int frow = lane & 15, fk = lane >> 4;
-    for (int kt = 0; kt < ktiles; ++kt) {
+    auto step = [&](int kt, bool more, auto edge) {   // edge: of the next K tile
         const int buf = kt & 1;
-        const bool more = kt + 1 < ktiles;
-        if (more) load_tile(kt + 1);
+        if (more) load_tile(kt + 1, edge);
+        __builtin_amdgcn_sched_barrier(0);   // the loads stay in front of the multiplications
         const double *as = As + buf * BK * LDA + fk * LDA + wm * CF::WTM + frow;
         const double *bs = Bs + buf * BK * LDB + fk * LDB + wn * CF::WTN + frow;
 #pragma unroll
@@ -112,9 +127,13 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
                 for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i], fb[j], acc[i][j], 0, 0, 0);
         }
-        if (more) store_tile(buf ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) store_tile(kt + 1, buf ^ 1, edge);
         __syncthreads();
-    }
+    };
+    int kt = 0;
+    for (; kt + 1 < nfast; ++kt) step(kt, true, std::false_type());
+    for (; kt < ktiles; ++kt) step(kt, kt + 1 < ktiles, std::true_type());
 
     // C values of one fragment row are loaded before any is stored (a load
     // cannot pass a possibly aliasing store: one latency per row, not per element).
@@ -157,7 +176,6 @@ int launch_cfg(const Gemm<double> &g, hipStream_t s) {
     const int tiles_m = (g.M + CF::BM - 1) / CF::BM, tiles_n = (g.N + CF::BN - 1) / CF::BN;
     const long nblk = (long)tiles_m * tiles_n;
     if (nblk > 0x7fffffffL) return fail(UGEMM_ERR_ARG, "dgemm: too many tiles (%ld)", nblk);
-    const bool vec = ugemm_aligned16(g.A) && ugemm_aligned16(g.B) && (g.lda % 2 == 0) && (g.ldb % 2 == 0);
     int kc = g.K;
     const int splits = split_count(g.splits, nblk, g.K, 64, &kc, 2);
     double *ws = nullptr;
@@ -166,21 +184,14 @@ int launch_cfg(const Gemm<double> &g, hipStream_t s) {
         if (rc) return rc;
     }
     dim3 grid((unsigned)nblk, (unsigned)splits), block(CF::NT);
-#define UGEMM_L(TA, TB, VEC)                                                                                \
-    hipLaunchKernelGGL((dgemm_mfma_kernel<CF, TA, TB, VEC>), grid, block, 0, s, g.M, g.N, g.K, g.alpha, g.A, \
+#define UGEMM_L(TA, TB) \
+    hipLaunchKernelGGL((dgemm_mfma_kernel<CF, TA, TB>), grid, block, 0, s, g.M, g.N, g.K, g.alpha, g.A, \
                        g.lda, g.B, g.ldb, g.beta, g.C, g.ldc, tiles_m, tiles_n, kc, ws)
     timing_begin(s);
-    if (vec) {
-        if (!g.ta && !g.tb) UGEMM_L(false, false, 2);
-        else if (!g.ta && g.tb) UGEMM_L(false, true, 2);
-        else if (g.ta && !g.tb) UGEMM_L(true, false, 2);
-        else UGEMM_L(true, true, 2);
-    } else {
-        if (!g.ta && !g.tb) UGEMM_L(false, false, 1);
-        else if (!g.ta && g.tb) UGEMM_L(false, true, 1);
-        else if (g.ta && !g.tb) UGEMM_L(true, false, 1);
-        else UGEMM_L(true, true, 1);
-    }
+    if (!g.ta && !g.tb) UGEMM_L(false, false);
+    else if (!g.ta && g.tb) UGEMM_L(false, true);
+    else if (g.ta && !g.tb) UGEMM_L(true, false);
+    else UGEMM_L(true, true);
     timing_end(s);
 #undef UGEMM_L
     hipError_t e = hipGetLastError();

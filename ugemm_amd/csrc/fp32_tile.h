@@ -13,6 +13,8 @@
 // C = alpha * acc + beta * C, C is not read when beta == 0 (sgemm_ocl2.h:86-88).
 #pragma once
 
+#include <type_traits>
+
 #include "internal.h"
 #include "kernel_common.h"
 
@@ -21,15 +23,31 @@ namespace {
 
 constexpr int LDS_PAD = 4;   // floats; keeps rows 16-byte aligned
 
-// Empty register constraints on the accumulators: the FMAs of one k-step
-// must complete before the next step's code, which bounds live ranges.
+// Empty register constraints on the accumulators.  They end a k-step: its
+// FMAs must complete before the next step's code, which bounds live ranges.
+// And they hold four columns j .. j + 3 of a row in one register quad rotated
+// by one, column j + 3 first.  A v_fmac_f32 whose three operands lie in one
+// register bank (number modulo 4) takes twice as long (measured with fixed
+// registers: 63-75 against 123-141 TF/s for any other assignment).  Quads
+// start at even registers, the fragments' as well as these, so a(i), b(j) and
+// acc(i, j) could share a bank only if one quad started an odd distance from
+// another in j: the rotation rules that out.  Left to the register allocator,
+// 1-13% of the FMAs of a kernel had the conflict, and any change of the code
+// around the loop moved that share.
 template <int TM, int TN>
 __device__ __forceinline__ void pin_step(float (&acc)[TM][TN]) {
+    typedef float quad __attribute__((ext_vector_type(4)));
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; j += 4)
-            asm volatile("" : "+v"(acc[i][j]), "+v"(acc[i][j + 1]), "+v"(acc[i][j + 2]), "+v"(acc[i][j + 3]));
+        for (int j = 0; j < TN; j += 4) {
+            quad q = {acc[i][j + 3], acc[i][j], acc[i][j + 1], acc[i][j + 2]};
+            asm volatile("" : "+v"(q));
+            acc[i][j + 3] = q[0];
+            acc[i][j] = q[1];
+            acc[i][j + 1] = q[2];
+            acc[i][j + 2] = q[3];
+        }
 }
 
 // MINB_: workgroups per CU the kernel is compiled for (register budget).
@@ -45,19 +63,16 @@ struct Fp32Cfg {
 
 // One workgroup computes the C tile at (m0, n0) of g; shared by the plain and
 // the grouped (persistent) kernels. lds must hold 2*(BK*LDA + BK*LDB) floats.
-// aligned == false (with VEC == 4) reads A and B with scalar loads: the
-// grouped kernel mixes problems whose operands allow 128-bit loads with
-// problems whose operands do not.
 // CONV: opB is the implicit im2col matrix of cd (B and TB unused): every
 // thread keeps one column n of the B tile, so the pixel's origin is computed
 // once per tile and each element costs one table read and two compares.
 // epi: bias and activation after alpha/beta (Epilogue, internal.h).
-template <class CF, bool TA, bool TB, int VEC, bool CONV = false>
+template <class CF, bool TA, bool TB, bool CONV = false>
 __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K, const float alpha,
                                           const float *__restrict__ A, const long lda,
                                           const float *__restrict__ B, const long ldb, const float beta,
                                           float *__restrict__ C, const long ldc, const int m0, const int n0,
-                                          float *lds, const bool aligned = true, const Epilogue &epi = Epilogue(),
+                                          float *lds, const Epilogue &epi = Epilogue(),
                                           const ConvDesc &cd = ConvDesc()) {
     constexpr int BM = CF::BM, BN = CF::BN, BK = CF::BK, TM = CF::TM, TN = CF::TN, NT = CF::NT;
     constexpr int LDA = CF::LDA, LDB = CF::LDB;
@@ -71,12 +86,13 @@ __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K,
     const int ty = (lane >> 3) + 8 * (w / WX);
 
     // A tile: TA -> stored K x M (contiguous m); else M x K (contiguous k).
-    using ARegs = TileRegs<float, TA ? BM : BK, TA ? BK : BM, NT, VEC>;
-    using BRegs = TileRegs<float, TB ? BK : BN, TB ? BN : BK, NT, VEC>;
+    using ARegs = TileRegs<float, TA ? BM : BK, TA ? BK : BM, NT>;
+    using BRegs = TileRegs<float, TB ? BK : BN, TB ? BN : BK, NT>;
     ARegs ra;
     BRegs rb;
 
     const bool interior = (m0 + BM <= M) && (n0 + BN <= N);
+    const bool wide_a = (TA ? M : K) >= 4, wide_b = (TB ? K : N) >= 4;
     const int ktiles = (K + BK - 1) / BK;
     const int kfull = K / BK;   // tiles with no K tail
 
@@ -97,11 +113,19 @@ __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K,
         c_base = (long)c_h0 * cd.W + c_w0;
     }
 
-    auto load_tile = [&](int kt) {
+    // EDGE tiles reach past M, N or K.
+    auto load_tile = [&](int kt, auto edge) {
         const int k0 = kt * BK;
         const float *a0 = TA ? A + (long)k0 * lda + m0 : A + (long)m0 * lda + k0;
-        if (interior && kt < kfull && aligned) ra.template load<false>(a0, lda, t, 0, 0);
-        else ra.template load<true>(a0, lda, t, TA ? M - m0 : K - k0, TA ? K - k0 : M - m0, aligned);
+        const float *b0 = TB ? B + (long)n0 * ldb + k0 : B + (long)k0 * ldb + n0;
+        if constexpr (!decltype(edge)::value) {
+            ra.load(a0, lda, t);
+            if constexpr (!CONV) rb.load(b0, ldb, t);
+        } else {
+            const int mr = M - m0, nr = N - n0, kr = K - k0;
+            ra.load_edge(a0, lda, t, TA ? mr : kr, TA ? kr : mr, wide_a);
+            if constexpr (!CONV) rb.load_edge(b0, ldb, t, TB ? kr : nr, TB ? nr : kr, wide_b);
+        }
         if constexpr (CONV) {
 #pragma unroll
             for (int i = 0; i < CONV_N; ++i) {
@@ -116,13 +140,14 @@ __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K,
                 }
                 cvals[i] = v;
             }
-        } else {
-            const float *b0 = TB ? B + (long)n0 * ldb + k0 : B + (long)k0 * ldb + n0;
-            if (interior && kt < kfull && aligned) rb.template load<false>(b0, ldb, t, 0, 0);
-            else rb.template load<true>(b0, ldb, t, TB ? K - k0 : N - n0, TB ? N - n0 : K - k0, aligned);
         }
     };
-    auto store_tile = [&](int buf) {
+    auto store_tile = [&](int kt, int buf, auto edge) {
+        if constexpr (decltype(edge)::value) {
+            const int mr = M - m0, nr = N - n0, kr = K - kt * BK;
+            ra.mask(t, TA ? mr : kr, TA ? kr : mr, wide_a);
+            if constexpr (!CONV) rb.mask(t, TB ? kr : nr, TB ? nr : kr, wide_b);
+        }
         ra.template store<TA, LDA>(As + buf * BK * LDA, t);
         if constexpr (CONV) {
 #pragma unroll
@@ -138,16 +163,22 @@ __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K,
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = 0.0f;
 
-    if (ktiles > 0) {
-        load_tile(0);
-        store_tile(0);
+    // K tiles below nfast are loaded without bounds; the others (all of an
+    // edge tile's, and a K remainder) as edges, in a loop of their own.
+    const int nfast = interior ? kfull : 0;
+    if (nfast > 0) {
+        load_tile(0, std::false_type());
+        store_tile(0, 0, std::false_type());
+    } else if (ktiles > 0) {
+        load_tile(0, std::true_type());
+        store_tile(0, 0, std::true_type());
     }
     __syncthreads();
 
-    for (int kt = 0; kt < ktiles; ++kt) {
+    auto step = [&](int kt, bool more, auto edge) {   // edge: of the next K tile
         const int buf = kt & 1;
-        const bool more = kt + 1 < ktiles;
-        if (more) load_tile(kt + 1);
+        if (more) load_tile(kt + 1, edge);
+        __builtin_amdgcn_sched_barrier(0);   // the loads stay in front of the multiplications
         const float *as = As + buf * BK * LDA + ty * 4;
         const float *bs = Bs + buf * BK * LDB + tx * 4;
         // Register double-buffering of the k-step fragments: the LDS reads
@@ -175,15 +206,18 @@ __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K,
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) acc[i][j] = fmaf(fa[i], fb[j], acc[i][j]);
+                for (int j = 0; j < TN; ++j) asm("v_fmac_f32 %0, %1, %2" : "+v"(acc[i][j]) : "v"(fa[i]), "v"(fb[j]));
             pin_step(acc);
         }
-        if (more) store_tile(buf ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) store_tile(kt + 1, buf ^ 1, edge);
         __syncthreads();
-    }
+    };
+    int kt = 0;
+    for (; kt + 1 < nfast; ++kt) step(kt, true, std::false_type());
+    for (; kt < ktiles; ++kt) step(kt, kt + 1 < ktiles, std::true_type());
 
     // Epilogue: C = alpha * acc (+ beta * C), then bias and activation.
-    const bool vec_c = interior && ((ldc & 3) == 0) && ((((uintptr_t)C) & 15) == 0);
     const bool has_epi = epi.active();
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
@@ -192,15 +226,15 @@ __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K,
         for (int g = 0; g < TN / 4; ++g) {
             const int n = n0 + g * CF::TX * 4 + tx * 4;
             float *cp = C + (long)m * ldc + n;
-            if (vec_c) {
-                float4 o;
+            const f32x4u q = {acc[i][g * 4], acc[i][g * 4 + 1], acc[i][g * 4 + 2], acc[i][g * 4 + 3]};
+            if (interior) {
+                f32x4u o;
                 if (beta == 0.0f) {
-                    o = make_float4(alpha * acc[i][g * 4 + 0], alpha * acc[i][g * 4 + 1],
-                                    alpha * acc[i][g * 4 + 2], alpha * acc[i][g * 4 + 3]);
+                    o = alpha * q;
                 } else {
-                    const float4 c = *reinterpret_cast<const float4 *>(cp);
-                    o = make_float4(fmaf(alpha, acc[i][g * 4 + 0], beta * c.x), fmaf(alpha, acc[i][g * 4 + 1], beta * c.y),
-                                    fmaf(alpha, acc[i][g * 4 + 2], beta * c.z), fmaf(alpha, acc[i][g * 4 + 3], beta * c.w));
+                    const f32x4u c = *reinterpret_cast<const f32x4u *>(cp);
+                    o = f32x4u{fmaf(alpha, q.x, beta * c.x), fmaf(alpha, q.y, beta * c.y),
+                               fmaf(alpha, q.z, beta * c.z), fmaf(alpha, q.w, beta * c.w)};
                 }
                 if (has_epi) {
                     o.x = apply_epilogue(epi, o.x, m, n);
@@ -208,12 +242,12 @@ __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K,
                     o.z = apply_epilogue(epi, o.z, m, n + 2);
                     o.w = apply_epilogue(epi, o.w, m, n + 3);
                 }
-                *reinterpret_cast<float4 *>(cp) = o;
+                *reinterpret_cast<f32x4u *>(cp) = o;
             } else if (m < M) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     if (n + j < N) {
-                        float r = (beta == 0.0f) ? alpha * acc[i][g * 4 + j] : fmaf(alpha, acc[i][g * 4 + j], beta * cp[j]);
+                        float r = (beta == 0.0f) ? alpha * q[j] : fmaf(alpha, q[j], beta * cp[j]);
                         if (has_epi) r = apply_epilogue(epi, r, m, n + j);
                         cp[j] = r;
                     }

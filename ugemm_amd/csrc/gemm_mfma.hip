@@ -141,17 +141,16 @@ __device__ __forceinline__ long blocked_offset(int r, int k, int rows_pad) {
 // (chunk f of the rows_pad x k_pad/8 chunks).
 // FMT::SCALED: row r is multiplied by 2^-row_exp(amax[r]) before splitting.
 template <int NP, class FMT>
-__device__ __forceinline__ void prep_kcont_chunk(const float *__restrict__ X, long ld, int rows, int K, bool vec,
-                                                 typename FMT::E *__restrict__ out, long plane_stride, int rows_pad,
+__device__ __forceinline__ void prep_kcont_chunk(const float *__restrict__ X, long ld, int rows, int K, typename FMT::E *__restrict__ out, long plane_stride, int rows_pad,
                                                  int k_pad, const unsigned *__restrict__ amax, long f) {
     const long chunks_per_row = k_pad / 8;
     const int r = (int)(f / chunks_per_row);
     const int k = (int)(f - (long)r * chunks_per_row) * 8;
     float x[8];
     const float *p = X + (long)r * ld + k;
-    if (r < rows && k + 8 <= K && vec) {
-        const float4 a = *reinterpret_cast<const float4 *>(p);
-        const float4 b = *reinterpret_cast<const float4 *>(p + 4);
+    if (r < rows && k + 8 <= K) {
+        const f32x4u a = *reinterpret_cast<const f32x4u *>(p);
+        const f32x4u b = *reinterpret_cast<const f32x4u *>(p + 4);
         x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
     } else {
 #pragma unroll
@@ -167,12 +166,12 @@ __device__ __forceinline__ void prep_kcont_chunk(const float *__restrict__ X, lo
 
 template <int NP, class FMT>
 __global__ __launch_bounds__(256) void split_prep_kcont(const float *__restrict__ X, long ld, int rows, int K,
-                                                        bool vec, typename FMT::E *__restrict__ out,
+                                                        typename FMT::E *__restrict__ out,
                                                         long plane_stride, int rows_pad, int k_pad,
                                                         const unsigned *__restrict__ amax) {
     const long total = (long)rows_pad * (k_pad / 8);
     for (long f = (long)blockIdx.x * blockDim.x + threadIdx.x; f < total; f += (long)gridDim.x * blockDim.x)
-        prep_kcont_chunk<NP, FMT>(X, ld, rows, K, vec, out, plane_stride, rows_pad, k_pad, amax, f);
+        prep_kcont_chunk<NP, FMT>(X, ld, rows, K, out, plane_stride, rows_pad, k_pad, amax, f);
 }
 
 // k-contiguous source, 2-D blocks: block (bx, by) covers rows [64 bx, +64)
@@ -183,8 +182,7 @@ __global__ __launch_bounds__(256) void split_prep_kcont(const float *__restrict_
 // a row-major walk stored sixteen 64-byte pieces per instruction.  All four
 // chunks are loaded before any is split.
 template <int NP, class FMT>
-__device__ __forceinline__ void prep_kcont_tile(const float *__restrict__ X, long ld, int rows, int K, bool vec,
-                                                typename FMT::E *__restrict__ out, long plane_stride, int rows_pad,
+__device__ __forceinline__ void prep_kcont_tile(const float *__restrict__ X, long ld, int rows, int K, typename FMT::E *__restrict__ out, long plane_stride, int rows_pad,
                                                 int k_pad, const unsigned *__restrict__ amax, int r0, int k0) {
     const int t = threadIdx.x;
     // Scaled formats: the row maxima are loaded first, so that their latency
@@ -199,9 +197,9 @@ __device__ __forceinline__ void prep_kcont_tile(const float *__restrict__ X, lon
     for (int i = 0; i < 4; ++i) {
         const int f = t + 256 * i, r = r0 + (f >> 4), k = k0 + (f & 15) * 8;
         const float *p = X + (long)r * ld + k;
-        if (r < rows && k + 8 <= K && vec) {
-            const float4 a = *reinterpret_cast<const float4 *>(p);
-            const float4 b = *reinterpret_cast<const float4 *>(p + 4);
+        if (r < rows && k + 8 <= K) {
+            const f32x4u a = *reinterpret_cast<const f32x4u *>(p);
+            const f32x4u b = *reinterpret_cast<const f32x4u *>(p + 4);
             x[i][0] = a.x; x[i][1] = a.y; x[i][2] = a.z; x[i][3] = a.w;
             x[i][4] = b.x; x[i][5] = b.y; x[i][6] = b.z; x[i][7] = b.w;
         } else {
@@ -224,10 +222,10 @@ __device__ __forceinline__ void prep_kcont_tile(const float *__restrict__ X, lon
 
 template <int NP, class FMT>
 __global__ __launch_bounds__(256) void split_prep_kcont_tiles(const float *__restrict__ X, long ld, int rows, int K,
-                                                              bool vec, typename FMT::E *__restrict__ out,
+                                                              typename FMT::E *__restrict__ out,
                                                               long plane_stride, int rows_pad, int k_pad,
                                                               const unsigned *__restrict__ amax) {
-    prep_kcont_tile<NP, FMT>(X, ld, rows, K, vec, out, plane_stride, rows_pad, k_pad, amax, blockIdx.x * 64,
+    prep_kcont_tile<NP, FMT>(X, ld, rows, K, out, plane_stride, rows_pad, k_pad, amax, blockIdx.x * 64,
                              blockIdx.y * 128);
 }
 
@@ -245,7 +243,7 @@ __global__ __launch_bounds__(256) void split_prep_kcont_tiles(const float *__res
 // keep bit 2 of the lane fixed), then over the waves.
 template <int NP, class FMT>
 __device__ __forceinline__ void prep_kcont_rowscaled_pair(const float *__restrict__ X, long ld, int rows, int K,
-                                                          bool vec, typename FMT::E *__restrict__ out,
+                                                          typename FMT::E *__restrict__ out,
                                                           long plane_stride, int rows_pad, int k_pad,
                                                           unsigned *__restrict__ amax, int r0) {
     static_assert(FMT::SCALED, "row scales");
@@ -259,9 +257,9 @@ __device__ __forceinline__ void prep_kcont_rowscaled_pair(const float *__restric
     for (int i = 0; i < PASSES; ++i) {
         const int kt = i * 32 + ktl, k = kt * 32 + cc * 8;
         const float *p = X + (long)r * ld + k;
-        if (kt < ktiles && r < rows && k + 8 <= K && vec) {
-            const float4 a = *reinterpret_cast<const float4 *>(p);
-            const float4 c = *reinterpret_cast<const float4 *>(p + 4);
+        if (kt < ktiles && r < rows && k + 8 <= K) {
+            const f32x4u a = *reinterpret_cast<const f32x4u *>(p);
+            const f32x4u c = *reinterpret_cast<const f32x4u *>(p + 4);
             x[i][0] = a.x; x[i][1] = a.y; x[i][2] = a.z; x[i][3] = a.w;
             x[i][4] = c.x; x[i][5] = c.y; x[i][6] = c.z; x[i][7] = c.w;
         } else {
@@ -295,18 +293,17 @@ __device__ __forceinline__ void prep_kcont_rowscaled_pair(const float *__restric
 
 template <int NP, class FMT>
 __global__ __launch_bounds__(256) void split_prep_kcont_rowscaled(const float *__restrict__ X, long ld, int rows,
-                                                                  int K, bool vec, typename FMT::E *__restrict__ out,
+                                                                  int K, typename FMT::E *__restrict__ out,
                                                                   long plane_stride, int rows_pad, int k_pad,
                                                                   unsigned *__restrict__ amax) {
-    prep_kcont_rowscaled_pair<NP, FMT>(X, ld, rows, K, vec, out, plane_stride, rows_pad, k_pad, amax,
+    prep_kcont_rowscaled_pair<NP, FMT>(X, ld, rows, K, out, plane_stride, rows_pad, k_pad, amax,
                                        (int)blockIdx.x * 2);
 }
 
 // Row-contiguous source (X[k*ld + r]): the 64 x 64 tile (rows r0.., k k0..)
 // transposed through LDS (tile[64][65], 256 threads).
 template <int NP, class FMT>
-__device__ __forceinline__ void prep_rcont_tile(const float *__restrict__ X, long ld, int rows, int K, bool vec,
-                                                typename FMT::E *__restrict__ out, long plane_stride, int rows_pad,
+__device__ __forceinline__ void prep_rcont_tile(const float *__restrict__ X, long ld, int rows, int K, typename FMT::E *__restrict__ out, long plane_stride, int rows_pad,
                                                 int k_pad, const unsigned *__restrict__ amax, int r0, int k0,
                                                 float (*tile)[65]) {
     const int t = threadIdx.x;
@@ -327,8 +324,8 @@ __device__ __forceinline__ void prep_rcont_tile(const float *__restrict__ X, lon
         const int k = k0 + kk, r = r0 + rr;
         const float *p = X + (long)k * ld + r;
         float v[4];
-        if (k < K && r + 4 <= rows && vec) {
-            const float4 a = *reinterpret_cast<const float4 *>(p);
+        if (k < K && r + 4 <= rows) {
+            const f32x4u a = *reinterpret_cast<const f32x4u *>(p);
             v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
         } else {
 #pragma unroll
@@ -359,11 +356,11 @@ __device__ __forceinline__ void prep_rcont_tile(const float *__restrict__ X, lon
 
 template <int NP, class FMT>
 __global__ __launch_bounds__(256) void split_prep_rcont(const float *__restrict__ X, long ld, int rows, int K,
-                                                        bool vec, typename FMT::E *__restrict__ out,
+                                                        typename FMT::E *__restrict__ out,
                                                         long plane_stride, int rows_pad, int k_pad,
                                                         const unsigned *__restrict__ amax) {
     __shared__ float tile[64][65];
-    prep_rcont_tile<NP, FMT>(X, ld, rows, K, vec, out, plane_stride, rows_pad, k_pad, amax, blockIdx.x * 64,
+    prep_rcont_tile<NP, FMT>(X, ld, rows, K, out, plane_stride, rows_pad, k_pad, amax, blockIdx.x * 64,
                              blockIdx.y * 64, tile);
 }
 
@@ -384,7 +381,7 @@ __global__ __launch_bounds__(256) void grouped_split_prep(const PrepJob *__restr
     if constexpr (FMT::SCALED) {
         if (j.kcont == kPrepRowScaled) {
             // The maxima buffer is the plan's own device memory, written here.
-            prep_kcont_rowscaled_pair<NP, FMT>(j.X, j.ld, j.rows, j.K, j.vec != 0, out, j.plane_stride, j.rows_pad,
+            prep_kcont_rowscaled_pair<NP, FMT>(j.X, j.ld, j.rows, j.K, out, j.plane_stride, j.rows_pad,
                                                j.k_pad, const_cast<unsigned *>(j.amax), lb * 2);
             return;
         }
@@ -392,12 +389,12 @@ __global__ __launch_bounds__(256) void grouped_split_prep(const PrepJob *__restr
     const int r0 = (lb % j.nbx) * 64, kb = (lb / j.nbx) * kPrepSpan;
     if (j.kcont) {
         for (int s = 0; s < kPrepSpan && (kb + s) * 128 < j.k_pad; ++s)
-            prep_kcont_tile<NP, FMT>(j.X, j.ld, j.rows, j.K, j.vec != 0, out, j.plane_stride, j.rows_pad, j.k_pad,
+            prep_kcont_tile<NP, FMT>(j.X, j.ld, j.rows, j.K, out, j.plane_stride, j.rows_pad, j.k_pad,
                                      j.amax, r0, (kb + s) * 128);
     } else {
         for (int s = 0; s < kPrepSpan && (kb + s) * 64 < j.k_pad; ++s) {
             if (s > 0) __syncthreads();   // the previous tile's reads of the LDS tile are done
-            prep_rcont_tile<NP, FMT>(j.X, j.ld, j.rows, j.K, j.vec != 0, out, j.plane_stride, j.rows_pad, j.k_pad,
+            prep_rcont_tile<NP, FMT>(j.X, j.ld, j.rows, j.K, out, j.plane_stride, j.rows_pad, j.k_pad,
                                      j.amax, r0, (kb + s) * 64, tile);
         }
     }
@@ -419,10 +416,10 @@ __global__ __launch_bounds__(256) void split_prep_pair(PrepJob a, PrepJob b) {
     typename FMT::E *out = static_cast<typename FMT::E *>(j.out);
     const int r0 = (lb % j.nbx) * 64;
     if (j.kcont)
-        prep_kcont_tile<NP, FMT>(j.X, j.ld, j.rows, j.K, j.vec != 0, out, j.plane_stride, j.rows_pad, j.k_pad,
+        prep_kcont_tile<NP, FMT>(j.X, j.ld, j.rows, j.K, out, j.plane_stride, j.rows_pad, j.k_pad,
                                  nullptr, r0, (lb / j.nbx) * 128);
     else
-        prep_rcont_tile<NP, FMT>(j.X, j.ld, j.rows, j.K, j.vec != 0, out, j.plane_stride, j.rows_pad, j.k_pad,
+        prep_rcont_tile<NP, FMT>(j.X, j.ld, j.rows, j.K, out, j.plane_stride, j.rows_pad, j.k_pad,
                                  nullptr, r0, (lb / j.nbx) * 64, tile);
 }
 
@@ -434,15 +431,14 @@ __global__ void fill_zero_u32(unsigned *__restrict__ p, long n) {
 }
 
 // k-contiguous source: block b covers row b / kchunks, k in [2048 * (b % kchunks), +2048).
-__device__ __forceinline__ void row_amax_kcont_block(const float *__restrict__ X, long ld, int rows, int K, bool vec,
-                                                     long kchunks, unsigned *__restrict__ amax, long b) {
+__device__ __forceinline__ void row_amax_kcont_block(const float *__restrict__ X, long ld, int rows, int K, long kchunks, unsigned *__restrict__ amax, long b) {
     const int r = (int)(b / kchunks);
     const int k = (int)(b % kchunks) * 2048 + threadIdx.x * 8;
     const float *p = X + (long)r * ld + k;
     float m = 0.0f;
-    if (k + 8 <= K && vec) {
-        const float4 a = *reinterpret_cast<const float4 *>(p);
-        const float4 c = *reinterpret_cast<const float4 *>(p + 4);
+    if (k + 8 <= K) {
+        const f32x4u a = *reinterpret_cast<const f32x4u *>(p);
+        const f32x4u c = *reinterpret_cast<const f32x4u *>(p + 4);
         m = fmaxf(fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))),
                   fmaxf(fmaxf(fabsf(c.x), fabsf(c.y)), fmaxf(fabsf(c.z), fabsf(c.w))));
     } else {
@@ -462,8 +458,8 @@ __device__ __forceinline__ void row_amax_kcont_block(const float *__restrict__ X
 }
 
 __global__ __launch_bounds__(256) void row_amax_kcont(const float *__restrict__ X, long ld, int rows, int K,
-                                                      bool vec, long kchunks, unsigned *__restrict__ amax) {
-    row_amax_kcont_block(X, ld, rows, K, vec, kchunks, amax, blockIdx.x);
+                                                      long kchunks, unsigned *__restrict__ amax) {
+    row_amax_kcont_block(X, ld, rows, K, kchunks, amax, blockIdx.x);
 }
 
 // Row-contiguous source (X[k*ld + r]): block b covers columns r in
@@ -473,8 +469,7 @@ __global__ __launch_bounds__(256) void row_amax_kcont(const float *__restrict__ 
 // segments (blocks that shared columns and differed only in k read addresses
 // a power-of-two multiple of the row pitch apart, which crowd the same HBM
 // channels).
-__device__ __forceinline__ void row_amax_rcont_block(const float *__restrict__ X, long ld, int rows, int K, bool vec,
-                                                     long kblocks, unsigned *__restrict__ amax, long b) {
+__device__ __forceinline__ void row_amax_rcont_block(const float *__restrict__ X, long ld, int rows, int K, long kblocks, unsigned *__restrict__ amax, long b) {
     const long cblocks = (rows + 255) / 256;
     constexpr int SPAN = kAmaxRcontSpan;
     const int c0 = (int)(b % cblocks) * 256, k0 = (int)(b / cblocks) * SPAN;
@@ -482,15 +477,15 @@ __device__ __forceinline__ void row_amax_rcont_block(const float *__restrict__ X
     const int cg = threadIdx.x & 63, kp = threadIdx.x >> 6;
     const int c = c0 + cg * 4;
     float m[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (vec && c + 4 <= rows && k0 + SPAN <= K) {
+    if (c + 4 <= rows && k0 + SPAN <= K) {
         // Whole block: SPAN/4 independent 16-byte loads per thread, issued 16 at
         // a time into registers before any is used (the compiler otherwise
         // waits after every second load, which leaves HBM idle).
         const float *p = X + (long)(k0 + kp) * ld + c;
         for (int kb = 0; kb < SPAN / 4; kb += 16) {
-            float4 v[16];
+            f32x4u v[16];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = *reinterpret_cast<const float4 *>(p + (long)(kb + i) * 4 * ld);
+            for (int i = 0; i < 16; ++i) v[i] = *reinterpret_cast<const f32x4u *>(p + (long)(kb + i) * 4 * ld);
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 m[0] = fmaxf(m[0], fabsf(v[i].x)); m[1] = fmaxf(m[1], fabsf(v[i].y));
@@ -500,8 +495,8 @@ __device__ __forceinline__ void row_amax_rcont_block(const float *__restrict__ X
     } else {
         for (int kk = kp; kk < SPAN && k0 + kk < K; kk += 4) {
             const float *p = X + (long)(k0 + kk) * ld + c;
-            if (vec && c + 4 <= rows) {
-                const float4 a = *reinterpret_cast<const float4 *>(p);
+            if (c + 4 <= rows) {
+                const f32x4u a = *reinterpret_cast<const f32x4u *>(p);
                 m[0] = fmaxf(m[0], fabsf(a.x)); m[1] = fmaxf(m[1], fabsf(a.y));
                 m[2] = fmaxf(m[2], fabsf(a.z)); m[3] = fmaxf(m[3], fabsf(a.w));
             } else {
@@ -521,8 +516,8 @@ __device__ __forceinline__ void row_amax_rcont_block(const float *__restrict__ X
 }
 
 __global__ __launch_bounds__(256) void row_amax_rcont(const float *__restrict__ X, long ld, int rows, int K,
-                                                      bool vec, long kblocks, unsigned *__restrict__ amax) {
-    row_amax_rcont_block(X, ld, rows, K, vec, kblocks, amax, blockIdx.x);
+                                                      long kblocks, unsigned *__restrict__ amax) {
+    row_amax_rcont_block(X, ld, rows, K, kblocks, amax, blockIdx.x);
 }
 
 // Row maxima of the operands of a grouped FP16X3 plan: job j (PrepJob with
@@ -536,13 +531,13 @@ __global__ __launch_bounds__(256) void row_amax_rcont(const float *__restrict__ 
 // next of A.
 template <int NP, class FMT>
 __global__ __launch_bounds__(256) void split_prep_rowscaled_a_amax_b(
-    const float *__restrict__ A, long lda, int rows_a, int K, bool vec_a, typename FMT::E *__restrict__ out_a,
+    const float *__restrict__ A, long lda, int rows_a, int K, typename FMT::E *__restrict__ out_a,
     long plane_a, int rows_pad_a, int k_pad, unsigned *__restrict__ amax_a, const float *__restrict__ B, long ldb,
-    int rows_b, bool vec_b, long kblocks_b, unsigned *__restrict__ amax_b, int b_blocks) {
+    int rows_b, long kblocks_b, unsigned *__restrict__ amax_b, int b_blocks) {
     if ((int)blockIdx.x < b_blocks)
-        row_amax_rcont_block(B, ldb, rows_b, K, vec_b, kblocks_b, amax_b, blockIdx.x);
+        row_amax_rcont_block(B, ldb, rows_b, K, kblocks_b, amax_b, blockIdx.x);
     else
-        prep_kcont_rowscaled_pair<NP, FMT>(A, lda, rows_a, K, vec_a, out_a, plane_a, rows_pad_a, k_pad, amax_a,
+        prep_kcont_rowscaled_pair<NP, FMT>(A, lda, rows_a, K, out_a, plane_a, rows_pad_a, k_pad, amax_a,
                                            ((int)blockIdx.x - b_blocks) * 2);
 }
 
@@ -551,8 +546,8 @@ __global__ __launch_bounds__(256) void grouped_row_amax(const PrepJob *__restric
     const PrepJob j = jobs[block_job[blockIdx.x]];
     const long lb = (long)blockIdx.x - j.block0;
     unsigned *amax = static_cast<unsigned *>(j.out);
-    if (j.kcont) row_amax_kcont_block(j.X, j.ld, j.rows, j.K, j.vec != 0, j.nbx, amax, lb);
-    else row_amax_rcont_block(j.X, j.ld, j.rows, j.K, j.vec != 0, j.nbx, amax, lb);
+    if (j.kcont) row_amax_kcont_block(j.X, j.ld, j.rows, j.K, j.nbx, amax, lb);
+    else row_amax_rcont_block(j.X, j.ld, j.rows, j.K, j.nbx, amax, lb);
 }
 
 // Implicit im2col operand of a convolution (ConvDesc): element (n, k) of the
@@ -730,7 +725,7 @@ __global__ __launch_bounds__(CF::NT) void split_nt_core(int M_, int N_, int Kp_,
                                                        const unsigned *__restrict__ amax_b_, Epilogue epi,
                                                        const float *__restrict__ Af, long lda,
                                                        const float *__restrict__ Bf_, long ldb_, int K_,
-                                                       int vec_ab_, int kt_per, float *__restrict__ ws,
+                                                       int kt_per, float *__restrict__ ws,
                                                        const GroupedSplitProblem *__restrict__ gprobs,
                                                        const GroupedSplitTile *__restrict__ gtiles) {
     using FMT = typename CF::FMT;
@@ -753,7 +748,6 @@ __global__ __launch_bounds__(CF::NT) void split_nt_core(int M_, int N_, int Kp_,
     const float *__restrict__ Bf = GR ? gp->Bf : Bf_;
     const long ldb = GR ? gp->ldb : ldb_;
     const int K = GR ? gp->K : K_;
-    const int vec_ab = GR ? (gp->vec_b ? 2 : 0) : vec_ab_;
     constexpr int BM = CF::BM, BN = CF::BN, BK = CF::BK, NP = CF::NP, FM = CF::FM, FN = CF::FN;
     constexpr int CPR = CF::CPR, STAGE = CF::STAGE, STAGES = CF::STAGES, PER_T = CF::PER_T;
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -784,16 +778,15 @@ __global__ __launch_bounds__(CF::NT) void split_nt_core(int M_, int N_, int Kp_,
     float fa[FA ? FA_CH : 1][8], fb[FB ? FB_CH : 1][8];
     // Row-contiguous source: rows [r, r+RW) of k-lines k .. k+7 into v[i][j]
     // (row r+i, k+j); zeros outside rows x K.  RW is 1 or 2 (stage rows per
-    // thread); vec: 8-byte loads allowed (RW == 2).  full: the whole stage
-    // lies inside rows x K and vector loads are allowed (uniform over the
+    // thread).  full: the whole stage lies inside rows x K (uniform over the
     // block): unguarded loads, no per-element branches.
-    auto load_rc = [&](const float *X, long ld, int rows, int r, int k, bool vec, auto &v, bool full) {
+    auto load_rc = [&](const float *X, long ld, int rows, int r, int k, auto &v, bool full) {
         constexpr int RW = std::extent<std::remove_reference_t<decltype(v)>>::value;
         if (full) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 if constexpr (RW == 2) {
-                    const float2 x = *reinterpret_cast<const float2 *>(X + (long)(k + j) * ld + r);
+                    const f32x2u x = *reinterpret_cast<const f32x2u *>(X + (long)(k + j) * ld + r);
                     v[0][j] = x.x;
                     v[1][j] = x.y;
                 } else {
@@ -806,8 +799,8 @@ __global__ __launch_bounds__(CF::NT) void split_nt_core(int M_, int N_, int Kp_,
         for (int j = 0; j < 8; ++j) {
             const float *p = X + (long)(k + j) * ld + r;
             if constexpr (RW == 2) {
-                if (k + j < K && r + 2 <= rows && vec) {
-                    const float2 x = *reinterpret_cast<const float2 *>(p);
+                if (k + j < K && r + 2 <= rows) {
+                    const f32x2u x = *reinterpret_cast<const f32x2u *>(p);
                     v[0][j] = x.x;
                     v[1][j] = x.y;
                 } else {
@@ -820,11 +813,11 @@ __global__ __launch_bounds__(CF::NT) void split_nt_core(int M_, int N_, int Kp_,
         }
     };
     // 8 floats of row `row`, k in [k, k+8), zeros outside rows x K.
-    auto load8 = [&](const float *X, long ld, int rows, int row, int k, bool vec, float (&v)[8], bool full) {
+    auto load8 = [&](const float *X, long ld, int rows, int row, int k, float (&v)[8], bool full) {
         const float *p = X + (long)row * ld + k;
-        if (full || (row < rows && k + 8 <= K && vec)) {
-            const float4 x0 = *reinterpret_cast<const float4 *>(p);
-            const float4 x1 = *reinterpret_cast<const float4 *>(p + 4);
+        if (full || (row < rows && k + 8 <= K)) {
+            const f32x4u x0 = *reinterpret_cast<const f32x4u *>(p);
+            const f32x4u x1 = *reinterpret_cast<const f32x4u *>(p + 4);
             v[0] = x0.x; v[1] = x0.y; v[2] = x0.z; v[3] = x0.w; v[4] = x1.x; v[5] = x1.y; v[6] = x1.z; v[7] = x1.w;
         } else {
 #pragma unroll
@@ -853,28 +846,28 @@ __global__ __launch_bounds__(CF::NT) void split_nt_core(int M_, int N_, int Kp_,
         const int k0 = kt * BK;
         const bool kin = k0 + BK <= K;
         if constexpr (FA == FUSE_RCONT) {
-            load_rc(Af, lda, M, m0 + (t % (BM / FA_CH)) * FA_CH, k0 + (t / (BM / FA_CH)) * 8, vec_ab & 1, fa,
-                    kin && (FA_CH == 1 || (vec_ab & 1)) && m0 + BM <= M);
+            load_rc(Af, lda, M, m0 + (t % (BM / FA_CH)) * FA_CH, k0 + (t / (BM / FA_CH)) * 8, fa,
+                    kin && m0 + BM <= M);
         } else if constexpr (FA == FUSE_KCONT) {
-            const bool full = kin && (vec_ab & 1) && m0 + BM <= M;
+            const bool full = kin && m0 + BM <= M;
 #pragma unroll
             for (int i = 0; i < FA_CH; ++i) {
                 const int f = t + CF::NT * i, r = f >> 2, c = (f & 3) ^ ((r >> 1) & 3);
-                load8(Af, lda, M, m0 + r, k0 + c * 8, vec_ab & 1, fa[i], full);
+                load8(Af, lda, M, m0 + r, k0 + c * 8, fa[i], full);
             }
         } else {
 #pragma unroll
             for (int i = 0; i < A_CH; ++i) load_chunk(kt, i);
         }
         if constexpr (FB == FUSE_RCONT) {
-            load_rc(Bf, ldb, N, n0 + (t % (BN / FB_CH)) * FB_CH, k0 + (t / (BN / FB_CH)) * 8, (vec_ab & 2) != 0, fb,
-                    kin && (FB_CH == 1 || (vec_ab & 2)) && n0 + BN <= N);
+            load_rc(Bf, ldb, N, n0 + (t % (BN / FB_CH)) * FB_CH, k0 + (t / (BN / FB_CH)) * 8, fb,
+                    kin && n0 + BN <= N);
         } else if constexpr (FB == FUSE_KCONT) {
-            const bool full = kin && (vec_ab & 2) && n0 + BN <= N;
+            const bool full = kin && n0 + BN <= N;
 #pragma unroll
             for (int i = 0; i < FB_CH; ++i) {
                 const int f = t + CF::NT * i, r = f >> 2, c = (f & 3) ^ ((r >> 1) & 3);
-                load8(Bf, ldb, N, n0 + r, k0 + c * 8, (vec_ab & 2) != 0, fb[i], full);
+                load8(Bf, ldb, N, n0 + r, k0 + c * 8, fb[i], full);
             }
         } else {
 #pragma unroll
@@ -1314,13 +1307,12 @@ static long round_up(long x, long a) { return (x + a - 1) / a * a; }
 template <int NP, class FMT>
 int prep_operand(const float *X, long ld, bool kcont, int rows, int K, typename FMT::E *out, long plane_stride,
                  int rows_pad, int k_pad, unsigned *amax, hipStream_t s, bool split = true, bool amax_done = false) {
-    const bool vec = ugemm_aligned16(X) && (ld % 4 == 0);
     if constexpr (FMT::SCALED) {
         if (amax_done) goto planes;   // the row maxima were computed by an earlier launch
         if (split && kcont && rows > 0 && K > 0 && k_pad <= 8192 && rows_pad % 2 == 0) {
             // Row maxima and planes in one pass (one block per two padded rows).
             hipLaunchKernelGGL((split_prep_kcont_rowscaled<NP, FMT>), dim3((unsigned)(rows_pad / 2)), dim3(256), 0, s, X,
-                               ld, rows, K, vec, out, plane_stride, rows_pad, k_pad, amax);
+                               ld, rows, K, out, plane_stride, rows_pad, k_pad, amax);
             UGEMM_HIP_TRY(hipGetLastError());
             return UGEMM_OK;
         }
@@ -1328,11 +1320,11 @@ int prep_operand(const float *X, long ld, bool kcont, int rows, int K, typename 
             if (kcont) {
                 const long kchunks = (K + 2047) / 2048;
                 hipLaunchKernelGGL(row_amax_kcont, dim3((unsigned)(rows * kchunks)), dim3(256), 0, s, X, ld, rows, K,
-                                   vec, kchunks, amax);
+                                   kchunks, amax);
             } else {
                 const long kblocks = (K + kAmaxRcontSpan - 1) / kAmaxRcontSpan, cblocks = (rows + 255) / 256;
                 hipLaunchKernelGGL(row_amax_rcont, dim3((unsigned)(cblocks * kblocks)), dim3(256), 0, s, X, ld, rows,
-                                   K, vec, kblocks, amax);
+                                   K, kblocks, amax);
             }
         }
     }
@@ -1343,7 +1335,7 @@ int prep_operand(const float *X, long ld, bool kcont, int rows, int K, typename 
 planes:
     if (kcont && rows_pad % 64 == 0 && (k_pad + 127) / 128 < 65536) {
         dim3 grid((unsigned)(rows_pad / 64), (unsigned)((k_pad + 127) / 128));
-        hipLaunchKernelGGL((split_prep_kcont_tiles<NP, FMT>), grid, dim3(256), 0, s, X, ld, rows, K, vec, out,
+        hipLaunchKernelGGL((split_prep_kcont_tiles<NP, FMT>), grid, dim3(256), 0, s, X, ld, rows, K, out,
                            plane_stride, rows_pad, k_pad, (const unsigned *)amax);
     } else if (kcont) {
         const long total = (long)rows_pad * (k_pad / 8);
@@ -1352,11 +1344,11 @@ planes:
         // 13% slower at 8192^3 (fewer loads in flight).
         long blocks = (total + 255) / 256;
         if (blocks > (1L << 20)) blocks = 1L << 20;
-        hipLaunchKernelGGL((split_prep_kcont<NP, FMT>), dim3((unsigned)blocks), dim3(256), 0, s, X, ld, rows, K, vec,
+        hipLaunchKernelGGL((split_prep_kcont<NP, FMT>), dim3((unsigned)blocks), dim3(256), 0, s, X, ld, rows, K,
                            out, plane_stride, rows_pad, k_pad, (const unsigned *)amax);
     } else {
         dim3 grid((unsigned)((rows_pad + 63) / 64), (unsigned)((k_pad + 63) / 64));
-        hipLaunchKernelGGL((split_prep_rcont<NP, FMT>), grid, dim3(256), 0, s, X, ld, rows, K, vec, out, plane_stride,
+        hipLaunchKernelGGL((split_prep_rcont<NP, FMT>), grid, dim3(256), 0, s, X, ld, rows, K, out, plane_stride,
                            rows_pad, k_pad, (const unsigned *)amax);
     }
     UGEMM_HIP_TRY(hipGetLastError());
@@ -1381,16 +1373,10 @@ int launch_core(const Gemm<float> &g, const typename CF::FMT::E *Ap, long a_plan
     static const hipError_t attr = hipFuncSetAttribute((const void *)kern,
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, CF::LDS_BYTES);
     if (attr != hipSuccess) return hip_fail(attr, "hipFuncSetAttribute");
-    // Vector loads of a fused operand: 16 bytes (k-contiguous) or 8 bytes (row-contiguous).
-    auto vec_ok = [](const float *X, long ld, int fuse) {
-        return fuse == FUSE_RCONT ? ((reinterpret_cast<uintptr_t>(X) & 7) == 0 && ld % 2 == 0)
-                                  : (ugemm_aligned16(X) && ld % 4 == 0);
-    };
-    const int vec_ab = (vec_ok(g.A, g.lda, FA) ? 1 : 0) | (vec_ok(g.B, g.ldb, FB) ? 2 : 0);
     timing_begin(s);
     hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n), (unsigned)splits), dim3(CF::NT), CF::LDS_BYTES, s,
                        g.M, g.N, Kp, Ap, a_plane, Mp, Bp, b_plane, Np, g.alpha, g.beta, g.C, g.ldc, tiles_m, tiles_n,
-                       amax_a, amax_b, g.epi, g.A, g.lda, g.B, g.ldb, g.K, vec_ab, kc / CF::BK, ws,
+                       amax_a, amax_b, g.epi, g.A, g.lda, g.B, g.ldb, g.K, kc / CF::BK, ws,
                        (const GroupedSplitProblem *)nullptr, (const GroupedSplitTile *)nullptr);
     timing_end(s);
     hipError_t e = hipGetLastError();
@@ -1460,10 +1446,9 @@ int run_cfg(const Gemm<float> &g, hipStream_t s) {
     if constexpr (FMT::SCALED) {
         if (!fa && !fb && !g.ta && !g.tb && g.M > 0 && g.N > 0 && g.K > 0 && Kp <= 8192) {
             const long kblocks = (g.K + kAmaxRcontSpan - 1) / kAmaxRcontSpan, cblocks = (g.N + 255) / 256;
-            const bool vec_a = ugemm_aligned16(g.A) && g.lda % 4 == 0, vec_b = ugemm_aligned16(g.B) && g.ldb % 4 == 0;
             hipLaunchKernelGGL((split_prep_rowscaled_a_amax_b<NP, FMT>), dim3((unsigned)(cblocks * kblocks + Mp / 2)),
-                               dim3(256), 0, s, g.A, g.lda, g.M, g.K, vec_a, Ap, a_plane, (int)Mp, (int)Kp, amax_a,
-                               g.B, g.ldb, g.N, vec_b, kblocks, amax_b, (int)(cblocks * kblocks));
+                               dim3(256), 0, s, g.A, g.lda, g.M, g.K, Ap, a_plane, (int)Mp, (int)Kp, amax_a,
+                               g.B, g.ldb, g.N, kblocks, amax_b, (int)(cblocks * kblocks));
             const hipError_t e = hipGetLastError();
             rc = e == hipSuccess ? UGEMM_OK : hip_fail(e, "split preparation");
             if (!rc) rc = prep_operand<NP, FMT>(g.B, g.ldb, false, g.N, g.K, Bp, b_plane, (int)Np, (int)Kp, amax_b, s,
@@ -1486,7 +1471,6 @@ int run_cfg(const Gemm<float> &g, hipStream_t s) {
                 j.rows_pad = (int)rows_pad;
                 j.k_pad = (int)Kp;
                 j.kcont = kcont;
-                j.vec = ugemm_aligned16(X) && ld % 4 == 0;
                 j.block0 = block0;
                 j.nbx = (int)(rows_pad / 64);
                 j.amax = nullptr;
@@ -1694,7 +1678,7 @@ int grouped_core(const PrepJob *jobs, const int *block_job, int prep_blocks, con
     hipLaunchKernelGGL(kern, dim3((unsigned)ntiles), dim3(CF::NT), CF::LDS_BYTES, s, 0, 0, 0,
                        (const typename FMT::E *)nullptr, 0L, 0, (const typename FMT::E *)nullptr, 0L, 0, 0.0f, 0.0f,
                        (float *)nullptr, 0L, 0, 0, (const unsigned *)nullptr, (const unsigned *)nullptr, Epilogue(),
-                       (const float *)nullptr, 0L, (const float *)nullptr, 0L, 0, 0, 0, (float *)nullptr, probs, tiles);
+                       (const float *)nullptr, 0L, (const float *)nullptr, 0L, 0, 0, (float *)nullptr, probs, tiles);
     timing_end(s);
     e = hipGetLastError();
     return e == hipSuccess ? UGEMM_OK : hip_fail(e, "grouped split-form core");

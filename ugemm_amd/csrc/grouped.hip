@@ -21,8 +21,7 @@
 // which workgroup took it: replays are bitwise identical.  The heads are
 // cleared by a kernel, not a memset, so the pair can be captured in a graph.
 // Kernel body: the plain FP32 tile (fp32_tile.h), dispatched on the
-// problem's layout; 128-bit operand loads are used for the problems whose A
-// and B allow them.
+// problem's layout.
 // A plan's launches must not overlap in time (the queue heads belong to the
 // plan): run one plan from one stream, or order the streams.
 // Used for convolution-as-GEMM batches (the conv -> GEMM shape mapping of
@@ -45,8 +44,8 @@ struct DevProblem {
     long lda, ldb, ldc;
     int M, N, K;          // K is 0 when alpha == 0 (A and B are then not read)
     float alpha, beta;
-    int layout;           // bit 0: A transposed, bit 1: B transposed, bit 2: A and B allow 128-bit
-                          // loads, bit 3: B is the implicit im2col operand cd (convolution)
+    int layout;           // bit 0: A transposed, bit 1: B transposed, bit 3: B is the implicit im2col operand cd
+                          // (convolution)
     Epilogue epi;         // bias + activation (convolutions)
     ConvDesc cd;
 };
@@ -64,49 +63,48 @@ __global__ void grouped_reset_heads(int *heads) {
 // One tile of problem p at (m0, n0), dispatched on the problem's layout.
 template <class CF, bool CONV>
 __device__ __forceinline__ void grouped_tile(const DevProblem &p, int m0, int n0, float *lds) {
-    const bool aligned = (p.layout & 4) != 0;
     if constexpr (IsM32<CF>::value && CONV) {   // FP32-MFMA convolution plans
-        m32_tile<CF, false, false, 4, true>(p.M, p.N, p.K, p.alpha, p.A, p.lda, nullptr, 0, p.beta, p.C, p.ldc, m0,
-                                            n0, lds, aligned, p.epi, p.cd);
+        m32_tile<CF, false, false, true>(p.M, p.N, p.K, p.alpha, p.A, p.lda, nullptr, 0, p.beta, p.C, p.ldc, m0,
+                                            n0, lds, p.epi, p.cd);
     } else if constexpr (IsM32<CF>::value) {   // FP32-MFMA GEMM plans
         switch (p.layout & 3) {
             case 0:
-                m32_tile<CF, false, false, 4>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
-                                              n0, lds, aligned);
+                m32_tile<CF, false, false>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
+                                              n0, lds);
                 break;
             case 1:
-                m32_tile<CF, true, false, 4>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
-                                             n0, lds, aligned);
+                m32_tile<CF, true, false>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
+                                             n0, lds);
                 break;
             case 2:
-                m32_tile<CF, false, true, 4>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
-                                             n0, lds, aligned);
+                m32_tile<CF, false, true>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
+                                             n0, lds);
                 break;
             default:
-                m32_tile<CF, true, true, 4>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
-                                            n0, lds, aligned);
+                m32_tile<CF, true, true>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
+                                            n0, lds);
                 break;
         }
     } else if constexpr (CONV) {
-        fp32_tile<CF, false, false, 4, true>(p.M, p.N, p.K, p.alpha, p.A, p.lda, nullptr, 0, p.beta, p.C, p.ldc, m0,
-                                             n0, lds, aligned, p.epi, p.cd);
+        fp32_tile<CF, false, false, true>(p.M, p.N, p.K, p.alpha, p.A, p.lda, nullptr, 0, p.beta, p.C, p.ldc, m0,
+                                             n0, lds, p.epi, p.cd);
     } else {
         switch (p.layout & 3) {
             case 0:
-                fp32_tile<CF, false, false, 4>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
-                                               n0, lds, aligned);
+                fp32_tile<CF, false, false>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
+                                               n0, lds);
                 break;
             case 1:
-                fp32_tile<CF, true, false, 4>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
-                                              n0, lds, aligned);
+                fp32_tile<CF, true, false>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
+                                              n0, lds);
                 break;
             case 2:
-                fp32_tile<CF, false, true, 4>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
-                                              n0, lds, aligned);
+                fp32_tile<CF, false, true>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
+                                              n0, lds);
                 break;
             default:
-                fp32_tile<CF, true, true, 4>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
-                                             n0, lds, aligned);
+                fp32_tile<CF, true, true>(p.M, p.N, p.K, p.alpha, p.A, p.lda, p.B, p.ldb, p.beta, p.C, p.ldc, m0,
+                                             n0, lds);
                 break;
         }
     }
@@ -451,7 +449,6 @@ int build_split_schedule(ugemm_grouped_plan *p, int v) {
         j.rows = rows;
         j.K = K;
         j.kcont = kcont ? 1 : 0;
-        j.vec = (K > 0 && ugemm_aligned16(X) && ld % 4 == 0) ? 1 : 0;
         j.block0 = (int)ablocks;
         j.nbx = kcont ? (K + 2047) / 2048 : (K + kAmaxRcontSpan - 1) / kAmaxRcontSpan;
         ablocks += kcont ? (long)rows * j.nbx : (long)((rows + 255) / 256) * j.nbx;
@@ -478,7 +475,6 @@ int build_split_schedule(ugemm_grouped_plan *p, int v) {
         j.rows_pad = rows_pad;
         j.k_pad = k_pad;
         j.kcont = row_scaled ? kPrepRowScaled : (kcont ? 1 : 0);
-        j.vec = (K > 0 && ugemm_aligned16(X) && ld % 4 == 0) ? 1 : 0;
         j.block0 = (int)blocks;
         j.nbx = rows_pad / 64;
         const long ktiles = kcont ? (k_pad + 127) / 128 : k_pad / 64;
@@ -512,8 +508,6 @@ int build_split_schedule(ugemm_grouped_plan *p, int v) {
             g.Bf = q.B;
             g.ldb = q.ldb;
             g.K = q.K;
-            g.vec_b = tb ? (q.K > 0 && ugemm_aligned16(q.B) && q.ldb % 4 == 0)
-                         : ((reinterpret_cast<uintptr_t>(q.B) & 7) == 0 && q.ldb % 2 == 0);
         }
         g.amax_a = scaled ? (const unsigned *)(intptr_t)am_a : nullptr;
         g.amax_b = scaled ? (const unsigned *)(intptr_t)am_b : nullptr;
@@ -707,9 +701,8 @@ int ugemm_hip_grouped_plan_create(ugemm_grouped_plan_t **plan, int count, const 
             delete p;
             return fail(UGEMM_ERR_ARG, "grouped: problem %d: NULL operand", i);
         }
-        const bool vec = ugemm_aligned16(q.A) && ugemm_aligned16(q.B) && q.lda % 4 == 0 && q.ldb % 4 == 0;
         DevProblem d{q.A, q.B, q.C, q.lda, q.ldb, q.ldc, q.M, q.N, reads_ab ? q.K : 0, q.alpha, q.beta,
-                     (ta ? 1 : 0) | (tb ? 2 : 0) | (vec ? 4 : 0)};
+                     (ta ? 1 : 0) | (tb ? 2 : 0)};
         p->probs.push_back(d);
         p->flops += 2.0 * q.M * q.N * q.K;
     }
@@ -775,7 +768,7 @@ int ugemm_hip_conv_grouped_plan_create_mode(ugemm_grouped_plan_t **plan, int cou
         d.K = K;
         d.alpha = 1.0f;
         d.beta = 0.0f;
-        d.layout = 8 | ((ugemm_aligned16(c.weights) && K % 4 == 0) ? 4 : 0);
+        d.layout = 8;
         d.epi.bias = c.bias;
         d.epi.bias_rows = 1;
         d.epi.act = c.act;

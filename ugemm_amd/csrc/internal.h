@@ -50,10 +50,10 @@ struct GroupedSplitProblem {
     long ldc;
     const unsigned *amax_a, *amax_b;   // FP16X3: per-row maxima (Mp, Np entries)
     // Variants that split B in the core (no B planes): B's FP32 source, its
-    // leading dimension, the true K, and whether vector loads are allowed.
+    // leading dimension and the true K.
     const float *Bf;
     long ldb;
-    int K, vec_b;
+    int K;
 };
 struct GroupedSplitTile {
     int problem, m0, n0, pad;
@@ -74,7 +74,7 @@ struct PrepJob {
     void *out;
     long plane_stride;
     int rows, K, rows_pad, k_pad;
-    int kcont, vec;
+    int kcont;
     int block0, nbx;
     const unsigned *amax;   // FP16X3: the operand's row maxima (row scales), else null
 };

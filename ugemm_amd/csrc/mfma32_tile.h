@@ -64,19 +64,18 @@ __device__ __forceinline__ m32_floatx4 m32_frag4(const float *L, int row, int k)
 }
 
 // C[m0:m0+BM, n0:n0+BN] = alpha * op(A) op(B) + beta * C, then the epilogue.
-// A and B point at the operands' origins (k = 0); vec_ok == false (VEC 4
-// only): the operands are not 16-byte aligned, every chunk is read with
-// scalar loads.  lds: CF::kLdsFloats floats, 16-byte aligned.
+// A and B point at the operands' origins (k = 0).  lds: CF::kLdsFloats
+// floats, 16-byte aligned.
 // CONV: op(B) is the implicit im2col matrix of cd (B and TB unused; the
 // gather of sgemm_gl1.h:166-190): every thread keeps one column n of the B
 // tile, so the pixel's origin is computed once per tile and each element
 // costs one table read and two compares; the B stage is [k][n].
-template <class CF, bool TA, bool TB, int VEC, bool CONV = false>
+template <class CF, bool TA, bool TB, bool CONV = false>
 __device__ __forceinline__ void m32_tile(const int M, const int N, const int K, const float alpha,
                                          const float *__restrict__ A, const long lda, const float *__restrict__ B,
                                          const long ldb, const float beta, float *__restrict__ C, const long ldc,
-                                         const int m0, const int n0, float *lds, const bool vec_ok = true,
-                                         const Epilogue &epi = Epilogue(), const ConvDesc &cd = ConvDesc()) {
+                                         const int m0, const int n0, float *lds, const Epilogue &epi = Epilogue(),
+                                         const ConvDesc &cd = ConvDesc()) {
     constexpr bool KCA = !TA, KCB = TB;
     constexpr int BM = CF::BM, BN = CF::BN, BK = CF::BK, NT = CF::NT, FM = CF::FM, FN = CF::FN;
     constexpr int LDA = CF::template ld<KCA, BM>(), LDB = CF::template ld<KCB, BN>();
@@ -88,12 +87,12 @@ __device__ __forceinline__ void m32_tile(const int M, const int N, const int K, 
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int wm = w / CF::WGN, wn = w % CF::WGN;
 
-    using ARegs = TileRegs<float, KCA ? BK : BM, KCA ? BM : BK, NT, VEC>;
-    using BRegs = TileRegs<float, KCB ? BK : BN, KCB ? BN : BK, NT, VEC>;
+    using ARegs = TileRegs<float, KCA ? BK : BM, KCA ? BM : BK, NT>;
+    using BRegs = TileRegs<float, KCB ? BK : BN, KCB ? BN : BK, NT>;
     ARegs ra;
     BRegs rb;
     const bool interior = (m0 + BM <= M) && (n0 + BN <= N);
-    const bool fast = interior && vec_ok;
+    const bool wide_a = (TA ? M : K) >= 4, wide_b = (TB ? K : N) >= 4;
     const int ktiles = (K + BK - 1) / BK, kfull = K / BK;
 
     static_assert(!CONV || (!TB && NT % BN == 0 && BN % 64 == 0), "implicit operand layout");
@@ -111,12 +110,19 @@ __device__ __forceinline__ void m32_tile(const int M, const int N, const int K, 
         c_base = (long)c_h0 * cd.W + c_w0;
     }
 
-    auto load_tile = [&](int kt) {
+    // EDGE tiles reach past M, N or K.
+    auto load_tile = [&](int kt, auto edge) {
         const int k0 = kt * BK;
         const float *a0 = TA ? A + (long)k0 * lda + m0 : A + (long)m0 * lda + k0;
-        const int mr = M - m0, nr = N - n0, kr = K - k0;
-        if (fast && kt < kfull) ra.template load<false>(a0, lda, t, 0, 0);
-        else ra.template load<true>(a0, lda, t, KCA ? kr : mr, KCA ? mr : kr, vec_ok);
+        const float *b0 = TB ? B + (long)n0 * ldb + k0 : B + (long)k0 * ldb + n0;
+        if constexpr (!decltype(edge)::value) {
+            ra.load(a0, lda, t);
+            if constexpr (!CONV) rb.load(b0, ldb, t);
+        } else {
+            const int mr = M - m0, nr = N - n0, kr = K - k0;
+            ra.load_edge(a0, lda, t, KCA ? kr : mr, KCA ? mr : kr, wide_a);
+            if constexpr (!CONV) rb.load_edge(b0, ldb, t, KCB ? kr : nr, KCB ? nr : kr, wide_b);
+        }
         if constexpr (CONV) {
 #pragma unroll
             for (int i = 0; i < CONV_N; ++i) {
@@ -131,13 +137,14 @@ __device__ __forceinline__ void m32_tile(const int M, const int N, const int K, 
                 }
                 cvals[i] = v;
             }
-        } else {
-            const float *b0 = TB ? B + (long)n0 * ldb + k0 : B + (long)k0 * ldb + n0;
-            if (fast && kt < kfull) rb.template load<false>(b0, ldb, t, 0, 0);
-            else rb.template load<true>(b0, ldb, t, KCB ? kr : nr, KCB ? nr : kr, vec_ok);
         }
     };
-    auto store_tile = [&](int buf) {
+    auto store_tile = [&](int kt, int buf, auto edge) {
+        if constexpr (decltype(edge)::value) {
+            const int mr = M - m0, nr = N - n0, kr = K - kt * BK;
+            ra.mask(t, KCA ? kr : mr, KCA ? mr : kr, wide_a);
+            if constexpr (!CONV) rb.mask(t, KCB ? kr : nr, KCB ? nr : kr, wide_b);
+        }
         ra.template store<true, LDA>(As + buf * SA, t);
         if constexpr (CONV) {
 #pragma unroll
@@ -153,17 +160,23 @@ __device__ __forceinline__ void m32_tile(const int M, const int N, const int K, 
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = m32_floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    if (ktiles > 0) {
-        load_tile(0);
-        store_tile(0);
+    // K tiles below nfast are loaded without bounds; the others (all of an
+    // edge tile's, and a K remainder) as edges, in a loop of their own.
+    const int nfast = interior ? kfull : 0;
+    if (nfast > 0) {
+        load_tile(0, std::false_type());
+        store_tile(0, 0, std::false_type());
+    } else if (ktiles > 0) {
+        load_tile(0, std::true_type());
+        store_tile(0, 0, std::true_type());
     }
     __syncthreads();
 
     const int frow = lane & 15, g4 = (lane >> 4) * 4;
-    for (int kt = 0; kt < ktiles; ++kt) {
+    auto step = [&](int kt, bool more, auto edge) {   // edge: of the next K tile
         const int buf = kt & 1;
-        const bool more = kt + 1 < ktiles;
-        if (more) load_tile(kt + 1);
+        if (more) load_tile(kt + 1, edge);
+        __builtin_amdgcn_sched_barrier(0);   // the loads stay in front of the multiplications
         const float *as = As + buf * SA, *bs = Bs + buf * SB;
 #pragma unroll
         for (int s = 0; s < BK / 16; ++s) {
@@ -180,9 +193,13 @@ __device__ __forceinline__ void m32_tile(const int M, const int N, const int K, 
                     for (int j = 0; j < FN; ++j)
                         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i][q], fb[j][q], acc[i][j], 0, 0, 0);
         }
-        if (more) store_tile(buf ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) store_tile(kt + 1, buf ^ 1, edge);
         __syncthreads();
-    }
+    };
+    int kt = 0;
+    for (; kt + 1 < nfast; ++kt) step(kt, true, std::false_type());
+    for (; kt < ktiles; ++kt) step(kt, kt + 1 < ktiles, std::true_type());
 
     // C values of one fragment row are loaded before any is stored (a load
     // cannot pass a possibly aliasing store: one latency per row, not per element).

@@ -9,7 +9,7 @@ namespace {
 
 // Split-K (gridDim.y > 1): block (tile, z) multiplies K columns
 // [z*kc, min(K, (z+1)*kc)) into the partial slice ws + z*M*N (row length N).
-template <class CF, bool TA, bool TB, int VEC>
+template <class CF, bool TA, bool TB>
 __global__ __launch_bounds__(CF::NT, CF::MINB) void sgemm_fp32_kernel(int M, int N, int K, float alpha,
                                                             const float *__restrict__ A, long lda,
                                                             const float *__restrict__ B, long ldb, float beta,
@@ -18,16 +18,12 @@ __global__ __launch_bounds__(CF::NT, CF::MINB) void sgemm_fp32_kernel(int M, int
     __shared__ __attribute__((aligned(16))) float lds[2 * CF::BK * (CF::LDA + CF::LDB)];
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
-    if (gridDim.y > 1) {
-        const int k0 = blockIdx.y * kc, kz = min(kc, K - k0);
-        const float *Az = TA ? A + (long)k0 * lda : A + k0;
-        const float *Bz = TB ? B + k0 : B + (long)k0 * ldb;
-        fp32_tile<CF, TA, TB, VEC>(M, N, kz, 1.0f, Az, lda, Bz, ldb, 0.0f, ws + (long)blockIdx.y * M * N, N,
-                                   tm * CF::BM, tn * CF::BN, lds, true, Epilogue());
-    } else {
-        fp32_tile<CF, TA, TB, VEC>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tm * CF::BM, tn * CF::BN, lds, true,
-                                   epi);
-    }
+    const bool part = gridDim.y > 1;
+    const int k0 = part ? (int)blockIdx.y * kc : 0;
+    fp32_tile<CF, TA, TB>(M, N, part ? min(kc, K - k0) : K, part ? 1.0f : alpha, TA ? A + (long)k0 * lda : A + k0, lda,
+                          TB ? B + k0 : B + (long)k0 * ldb, ldb, part ? 0.0f : beta,
+                          part ? ws + (long)blockIdx.y * M * N : C, part ? (long)N : ldc, tm * CF::BM, tn * CF::BN, lds,
+                          part ? Epilogue() : epi);
 }
 
 // Implicit-GEMM convolution: C (M = output channels x N = output pixels) =
@@ -35,7 +31,7 @@ __global__ __launch_bounds__(CF::NT, CF::MINB) void sgemm_fp32_kernel(int M, int
 // epilogue.  The column matrix is gathered in the tile loader (ConvDesc).
 // Split-K as in sgemm_fp32_kernel: the chunk's rows of the offset table
 // (absolute image offsets) and its weight columns.
-template <class CF, bool TA, int VEC>
+template <class CF>
 __global__ __launch_bounds__(CF::NT) void conv_fp32_kernel(int M, int N, int K, float alpha,
                                                            const float *__restrict__ A, long lda, float beta,
                                                            float *__restrict__ C, long ldc, int tiles_m, int tiles_n,
@@ -43,17 +39,13 @@ __global__ __launch_bounds__(CF::NT) void conv_fp32_kernel(int M, int N, int K, 
     __shared__ __attribute__((aligned(16))) float lds[2 * CF::BK * (CF::LDA + CF::LDB)];
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
-    if (gridDim.y > 1) {
-        const int k0 = blockIdx.y * kc, kz = min(kc, K - k0);
-        ConvDesc cz = cd;
-        cz.ktab = cd.ktab + k0;
-        const float *Az = TA ? A + (long)k0 * lda : A + k0;
-        fp32_tile<CF, TA, false, VEC, true>(M, N, kz, 1.0f, Az, lda, nullptr, 0, 0.0f, ws + (long)blockIdx.y * M * N,
-                                            N, tm * CF::BM, tn * CF::BN, lds, true, Epilogue(), cz);
-    } else {
-        fp32_tile<CF, TA, false, VEC, true>(M, N, K, alpha, A, lda, nullptr, 0, beta, C, ldc, tm * CF::BM,
-                                            tn * CF::BN, lds, true, epi, cd);
-    }
+    const bool part = gridDim.y > 1;
+    const int k0 = part ? (int)blockIdx.y * kc : 0;
+    ConvDesc cz = cd;
+    cz.ktab = cd.ktab + k0;
+    fp32_tile<CF, false, false, true>(M, N, part ? min(kc, K - k0) : K, part ? 1.0f : alpha, A + k0, lda, nullptr, 0,
+                                      part ? 0.0f : beta, part ? ws + (long)blockIdx.y * M * N : C,
+                                      part ? (long)N : ldc, tm * CF::BM, tn * CF::BN, lds, part ? Epilogue() : epi, cz);
 }
 
 // ---------------------------------------------------------------------------
@@ -62,8 +54,8 @@ using V0 = Fp32Cfg<128, 128, 16, 8, 8>;
 using V1 = Fp32Cfg<64, 64, 16, 4, 4>;
 using V2 = Fp32Cfg<128, 64, 16, 8, 4>;
 using V3 = Fp32Cfg<64, 128, 16, 4, 8>;
-using V4 = Fp32Cfg<256, 128, 16, 16, 8>;
-using V5 = Fp32Cfg<128, 256, 16, 8, 16>;
+using V4 = Fp32Cfg<256, 128, 16, 16, 8, 2>;
+using V5 = Fp32Cfg<128, 256, 16, 8, 16, 2>;
 
 const char *kNames[] = {"fp32_128x128x16_t8x8", "fp32_64x64x16_t4x4", "fp32_128x64x16_t8x4",
                         "fp32_64x128x16_t4x8", "fp32_256x128x16_t16x8", "fp32_128x256x16_t8x16"};
@@ -75,9 +67,6 @@ int launch_cfg(const Gemm<float> &g, hipStream_t s) {
     const int tiles_n = (g.N + CF::BN - 1) / CF::BN;
     const long nblk = (long)tiles_m * tiles_n;
     if (nblk > 0x7fffffffL) return fail(UGEMM_ERR_ARG, "sgemm: too many tiles (%ld)", nblk);
-    // 128-bit loads need 16-byte aligned bases and leading dimensions that are multiples of 4
-    // (split-K chunk offsets are multiples of 64 columns, which keeps that).
-    const bool vec = ugemm_aligned16(g.A) && ugemm_aligned16(g.B) && (g.lda % 4 == 0) && (g.ldb % 4 == 0);
     int kc = g.K;
     const int splits = split_count(g.splits, nblk, g.K, 64, &kc, 2);
     float *ws = nullptr;
@@ -86,21 +75,14 @@ int launch_cfg(const Gemm<float> &g, hipStream_t s) {
         if (rc) return rc;
     }
     dim3 grid((unsigned)nblk, (unsigned)splits), block(CF::NT);
-#define UGEMM_L(TA, TB, VEC)                                                                             \
-    hipLaunchKernelGGL((sgemm_fp32_kernel<CF, TA, TB, VEC>), grid, block, 0, s, g.M, g.N, g.K, g.alpha, g.A, \
+#define UGEMM_L(TA, TB) \
+    hipLaunchKernelGGL((sgemm_fp32_kernel<CF, TA, TB>), grid, block, 0, s, g.M, g.N, g.K, g.alpha, g.A, \
                        g.lda, g.B, g.ldb, g.beta, g.C, g.ldc, tiles_m, tiles_n, g.epi, kc, ws)
     timing_begin(s);
-    if (vec) {
-        if (!g.ta && !g.tb) UGEMM_L(false, false, 4);
-        else if (!g.ta && g.tb) UGEMM_L(false, true, 4);
-        else if (g.ta && !g.tb) UGEMM_L(true, false, 4);
-        else UGEMM_L(true, true, 4);
-    } else {
-        if (!g.ta && !g.tb) UGEMM_L(false, false, 1);
-        else if (!g.ta && g.tb) UGEMM_L(false, true, 1);
-        else if (g.ta && !g.tb) UGEMM_L(true, false, 1);
-        else UGEMM_L(true, true, 1);
-    }
+    if (!g.ta && !g.tb) UGEMM_L(false, false);
+    else if (!g.ta && g.tb) UGEMM_L(false, true);
+    else if (g.ta && !g.tb) UGEMM_L(true, false);
+    else UGEMM_L(true, true);
     timing_end(s);
 #undef UGEMM_L
     hipError_t e = hipGetLastError();
@@ -119,7 +101,6 @@ int launch_conv_cfg(const Gemm<float> &g, const ConvDesc &cd, hipStream_t s) {
     const int tiles_n = (g.N + CF::BN - 1) / CF::BN;
     const long nblk = (long)tiles_m * tiles_n;
     if (nblk > 0x7fffffffL) return fail(UGEMM_ERR_ARG, "conv: too many tiles (%ld)", nblk);
-    const bool vec = ugemm_aligned16(g.A) && (g.lda % 4 == 0);
     int kc = g.K;
     const int splits = split_count(g.splits, nblk, g.K, 64, &kc, 2);
     float *ws = nullptr;
@@ -129,15 +110,8 @@ int launch_conv_cfg(const Gemm<float> &g, const ConvDesc &cd, hipStream_t s) {
     }
     dim3 grid((unsigned)nblk, (unsigned)splits), block(CF::NT);
     timing_begin(s);
-    if (vec && !g.ta)
-        hipLaunchKernelGGL((conv_fp32_kernel<CF, false, 4>), grid, block, 0, s, g.M, g.N, g.K, g.alpha, g.A, g.lda,
-                           g.beta, g.C, g.ldc, tiles_m, tiles_n, g.epi, cd, kc, ws);
-    else if (!g.ta)
-        hipLaunchKernelGGL((conv_fp32_kernel<CF, false, 1>), grid, block, 0, s, g.M, g.N, g.K, g.alpha, g.A, g.lda,
-                           g.beta, g.C, g.ldc, tiles_m, tiles_n, g.epi, cd, kc, ws);
-    else
-        hipLaunchKernelGGL((conv_fp32_kernel<CF, true, 1>), grid, block, 0, s, g.M, g.N, g.K, g.alpha, g.A, g.lda,
-                           g.beta, g.C, g.ldc, tiles_m, tiles_n, g.epi, cd, kc, ws);
+    hipLaunchKernelGGL((conv_fp32_kernel<CF>), grid, block, 0, s, g.M, g.N, g.K, g.alpha, g.A, g.lda, g.beta, g.C,
+                       g.ldc, tiles_m, tiles_n, g.epi, cd, kc, ws);
     timing_end(s);
     hipError_t e = hipGetLastError();
     int rc = e == hipSuccess ? UGEMM_OK : hip_fail(e, "conv launch");

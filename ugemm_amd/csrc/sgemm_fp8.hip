@@ -67,7 +67,7 @@ __device__ __forceinline__ int pack4_e4m3(float a, float b, float c, float d) {
 struct Fp8Operand {
     const float *X;
     long ld;
-    int rows, K, vec, kcont;
+    int rows, K, kcont;
     unsigned char *out;
     int rows_pad, rblocks;
     int *exps;
@@ -102,8 +102,8 @@ __device__ __forceinline__ void fp8_quantise_block(const Fp8Operand &op, int rb,
         const int r = KCONT ? r0 + line : r0 + cl, k = KCONT ? k0 + cl : k0 + line;
         const float *p = KCONT ? X + (long)r * ld + k : X + (long)k * ld + r;
         const bool full = KCONT ? (r < rows && k + 4 <= K) : (k < K && r + 4 <= rows);
-        if (full && op.vec) {
-            const float4 x = *reinterpret_cast<const float4 *>(p);
+        if (full) {
+            const f32x4u x = *reinterpret_cast<const f32x4u *>(p);
             v[q * 4 + 0] = x.x; v[q * 4 + 1] = x.y; v[q * 4 + 2] = x.z; v[q * 4 + 3] = x.w;
         } else {
 #pragma unroll
@@ -372,7 +372,7 @@ long round_up(long x, long a) { return (x + a - 1) / a * a; }
 
 Fp8Operand operand(const float *X, long ld, bool kcont, int rows, int K, unsigned char *out, int rows_pad,
                    int *exps) {
-    return Fp8Operand{X, ld, rows, K, (ugemm_aligned16(X) && ld % 4 == 0) ? 1 : 0, kcont ? 1 : 0, out, rows_pad,
+    return Fp8Operand{X, ld, rows, K, kcont ? 1 : 0, out, rows_pad,
                       rows_pad / SB, exps};
 }
 

@@ -18,7 +18,7 @@
 namespace ugemm {
 namespace {
 
-template <class CF, bool TA, bool TB, int VEC>
+template <class CF, bool TA, bool TB>
 __global__ __launch_bounds__(CF::NT, CF::MINB) void sgemm_mfma32_kernel(
     int M, int N, int K_, float alpha_, const float *__restrict__ A_, long lda, const float *__restrict__ B_,
     long ldb, float beta_, float *__restrict__ C_, long ldc_, int tiles_m, int tiles_n, Epilogue epi, int kc,
@@ -33,12 +33,9 @@ __global__ __launch_bounds__(CF::NT, CF::MINB) void sgemm_mfma32_kernel(
     const float *B = TB ? B_ + kz0 : B_ + (long)kz0 * ldb;
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
-    if (part)
-        m32_tile<CF, TA, TB, VEC>(M, N, K, 1.0f, A, lda, B, ldb, 0.0f, ws + (long)blockIdx.y * M * N, (long)N,
-                                  tm * CF::BM, tn * CF::BN, lds);
-    else
-        m32_tile<CF, TA, TB, VEC>(M, N, K, alpha_, A, lda, B, ldb, beta_, C_, ldc_, tm * CF::BM, tn * CF::BN, lds,
-                                  true, epi);
+    m32_tile<CF, TA, TB>(M, N, K, part ? 1.0f : alpha_, A, lda, B, ldb, part ? 0.0f : beta_,
+                         part ? ws + (long)blockIdx.y * M * N : C_, part ? (long)N : ldc_, tm * CF::BM, tn * CF::BN, lds,
+                         part ? Epilogue() : epi);
 }
 
 // Implicit-GEMM convolution on the FP32 matrix cores: C (M = output
@@ -49,22 +46,18 @@ __global__ __launch_bounds__(CF::NT, CF::MINB) void sgemm_mfma32_kernel(
 template <class CF>
 __global__ __launch_bounds__(CF::NT, CF::MINB) void conv_mfma32_kernel(
     int M, int N, int K_, const float *__restrict__ A_, long lda, float *__restrict__ C_, long ldc_, int tiles_m,
-    int tiles_n, Epilogue epi, ConvDesc cd, bool vec, int kc, float *__restrict__ ws) {
+    int tiles_n, Epilogue epi, ConvDesc cd, int kc, float *__restrict__ ws) {
     constexpr int kLds = 2 * (CF::template stage<true, CF::BM>() + CF::template stage<false, CF::BN>());
     __shared__ __attribute__((aligned(16))) float lds[kLds];
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
-    if (gridDim.y > 1) {
-        const int k0 = blockIdx.y * kc, kz = min(kc, K_ - k0);
-        ConvDesc cz = cd;
-        cz.ktab = cd.ktab + k0;
-        m32_tile<CF, false, false, 4, true>(M, N, kz, 1.0f, A_ + k0, lda, nullptr, 0, 0.0f,
-                                            ws + (long)blockIdx.y * M * N, (long)N, tm * CF::BM, tn * CF::BN, lds, vec,
-                                            Epilogue(), cz);
-    } else {
-        m32_tile<CF, false, false, 4, true>(M, N, K_, 1.0f, A_, lda, nullptr, 0, 0.0f, C_, ldc_, tm * CF::BM,
-                                            tn * CF::BN, lds, vec, epi, cd);
-    }
+    const bool part = gridDim.y > 1;
+    const int k0 = part ? (int)blockIdx.y * kc : 0;
+    ConvDesc cz = cd;
+    cz.ktab = cd.ktab + k0;
+    m32_tile<CF, false, false, true>(M, N, part ? min(kc, K_ - k0) : K_, 1.0f, A_ + k0, lda, nullptr, 0, 0.0f,
+                                     part ? ws + (long)blockIdx.y * M * N : C_, part ? (long)N : ldc_, tm * CF::BM,
+                                     tn * CF::BN, lds, part ? Epilogue() : epi, cz);
 }
 
 using V0 = M32Cfg<128, 128, 16, 2, 2, 2>;
@@ -82,7 +75,6 @@ int launch_cfg(const Gemm<float> &g, hipStream_t s) {
     const int tiles_m = (g.M + CF::BM - 1) / CF::BM, tiles_n = (g.N + CF::BN - 1) / CF::BN;
     const long nblk = (long)tiles_m * tiles_n;
     if (nblk > 0x7fffffffL) return fail(UGEMM_ERR_ARG, "sgemm fp32 mfma: too many tiles (%ld)", nblk);
-    const bool vec = ugemm_aligned16(g.A) && ugemm_aligned16(g.B) && (g.lda % 4 == 0) && (g.ldb % 4 == 0);
     int kc = g.K;
     const int splits = split_count(g.splits, nblk, g.K, 64, &kc, 2);
     float *ws = nullptr;
@@ -91,21 +83,14 @@ int launch_cfg(const Gemm<float> &g, hipStream_t s) {
         if (rc) return rc;
     }
     dim3 grid((unsigned)nblk, (unsigned)splits), block(CF::NT);
-#define UGEMM_L(TA, TB, VEC)                                                                                   \
-    hipLaunchKernelGGL((sgemm_mfma32_kernel<CF, TA, TB, VEC>), grid, block, 0, s, g.M, g.N, g.K, g.alpha, g.A, \
+#define UGEMM_L(TA, TB) \
+    hipLaunchKernelGGL((sgemm_mfma32_kernel<CF, TA, TB>), grid, block, 0, s, g.M, g.N, g.K, g.alpha, g.A, \
                        g.lda, g.B, g.ldb, g.beta, g.C, g.ldc, tiles_m, tiles_n, g.epi, kc, ws)
     timing_begin(s);
-    if (vec) {
-        if (!g.ta && !g.tb) UGEMM_L(false, false, 4);
-        else if (!g.ta && g.tb) UGEMM_L(false, true, 4);
-        else if (g.ta && !g.tb) UGEMM_L(true, false, 4);
-        else UGEMM_L(true, true, 4);
-    } else {
-        if (!g.ta && !g.tb) UGEMM_L(false, false, 1);
-        else if (!g.ta && g.tb) UGEMM_L(false, true, 1);
-        else if (g.ta && !g.tb) UGEMM_L(true, false, 1);
-        else UGEMM_L(true, true, 1);
-    }
+    if (!g.ta && !g.tb) UGEMM_L(false, false);
+    else if (!g.ta && g.tb) UGEMM_L(false, true);
+    else if (g.ta && !g.tb) UGEMM_L(true, false);
+    else UGEMM_L(true, true);
     timing_end(s);
 #undef UGEMM_L
     hipError_t e = hipGetLastError();
@@ -123,7 +108,6 @@ int launch_conv_cfg(const Gemm<float> &g, const ConvDesc &cd, hipStream_t s) {
     const int tiles_m = (g.M + CF::BM - 1) / CF::BM, tiles_n = (g.N + CF::BN - 1) / CF::BN;
     const long nblk = (long)tiles_m * tiles_n;
     if (nblk > 0x7fffffffL) return fail(UGEMM_ERR_ARG, "conv fp32 mfma: too many tiles (%ld)", nblk);
-    const bool vec = ugemm_aligned16(g.A) && (g.lda % 4 == 0);
     int kc = g.K;
     const int splits = split_count(g.splits, nblk, g.K, 64, &kc, 2);
     float *ws = nullptr;
@@ -133,7 +117,7 @@ int launch_conv_cfg(const Gemm<float> &g, const ConvDesc &cd, hipStream_t s) {
     }
     timing_begin(s);
     hipLaunchKernelGGL((conv_mfma32_kernel<CF>), dim3((unsigned)nblk, (unsigned)splits), dim3(CF::NT), 0, s, g.M,
-                       g.N, g.K, g.A, g.lda, g.C, g.ldc, tiles_m, tiles_n, g.epi, cd, vec, kc, ws);
+                       g.N, g.K, g.A, g.lda, g.C, g.ldc, tiles_m, tiles_n, g.epi, cd, kc, ws);
     timing_end(s);
     hipError_t e = hipGetLastError();
     int rc = e == hipSuccess ? UGEMM_OK : hip_fail(e, "conv fp32 mfma launch");
