@@ -15,6 +15,7 @@
 // split-K call adds its partial slices in a fixed order (no atomics), so
 // repeated calls are bitwise identical.
 // Semantics as dgemm_cpu (ugemm.h:162-286) with the BLAS beta == 0 rule.
+#include <algorithm>
 #include <type_traits>
 
 #include "internal.h"
@@ -25,17 +26,23 @@ namespace {
 
 typedef double doublex4 __attribute__((ext_vector_type(4)));
 
-template <int BM_, int BN_>
+// WG x WG waves to a tile.  KG: groups of them in a workgroup, each with its
+// own LDS stages; group g multiplies K tiles g, g + KG, ... and the groups'
+// sums are added through LDS in group order (small grids, launch_small).
+// WEU: waves per SIMD the kernel is compiled for.
+template <int BM_, int BN_, int WG_ = 2, int KG_ = 1, int WEU_ = 2>
 struct DCfg {
-    static constexpr int BM = BM_, BN = BN_, BK = 16, NT = 256;
-    static constexpr int WTM = BM / 2, WTN = BN / 2, FM = WTM / 16, FN = WTN / 16;
+    static constexpr int BM = BM_, BN = BN_, BK = 16, WG = WG_, NT = 64 * WG * WG, KG = KG_, WEU = WEU_;
+    static constexpr int WTM = BM / WG, WTN = BN / WG, FM = WTM / 16, FN = WTN / 16;
     static constexpr int LDA = BM + 2, LDB = BN + 2;   // doubles; +2 keeps 16-byte alignment
+    static constexpr int kStage = 2 * BK * (LDA + LDB);   // doubles: two stages of a group
+    static_assert(KG == 1 || BM * BN <= kStage, "the groups' sums fit their stages");
 };
 
 // Split-K (gridDim.y > 1): block (tile, z) multiplies K columns
 // [z*kc, min(K, (z+1)*kc)) into the partial slice ws + z*M*N (row length N).
 template <class CF, bool TA, bool TB>
-__global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) void dgemm_mfma_kernel(
+__global__ __launch_bounds__(CF::NT * CF::KG) __attribute__((amdgpu_waves_per_eu(CF::WEU))) void dgemm_mfma_kernel(
     int M, int N, int K_, double alpha_, const double *__restrict__ A_, long lda, const double *__restrict__ B_,
     long ldb, double beta_, double *__restrict__ C_, long ldc_, int tiles_m, int tiles_n, int kc,
     double *__restrict__ ws) {
@@ -49,14 +56,16 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
     const double alpha = part ? 1.0 : alpha_, beta = part ? 0.0 : beta_;
     constexpr int BM = CF::BM, BN = CF::BN, BK = CF::BK, NT = CF::NT, FM = CF::FM, FN = CF::FN;
     constexpr int LDA = CF::LDA, LDB = CF::LDB;
-    __shared__ __attribute__((aligned(16))) double lds[2 * BK * (LDA + LDB)];
-    double *As = lds, *Bs = lds + 2 * BK * LDA;
+    constexpr int KG = CF::KG;
+    __shared__ __attribute__((aligned(16))) double lds[KG * CF::kStage];
+    const int grp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
+    double *As = lds + grp * CF::kStage, *Bs = As + 2 * BK * LDA;
 
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int wm = w >> 1, wn = w & 1;
+    const int t = KG == 1 ? threadIdx.x : threadIdx.x % NT, lane = t & 63, w = t >> 6;
+    const int wm = w / CF::WG, wn = w % CF::WG;
 
     using ARegs = TileRegs<double, TA ? BM : BK, TA ? BK : BM, NT>;
     using BRegs = TileRegs<double, TB ? BK : BN, TB ? BN : BK, NT>;
@@ -99,19 +108,18 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
     // K tiles below nfast are loaded without bounds; the others (all of an
     // edge tile's, and a K remainder) as edges, in a loop of their own.
     const int nfast = interior ? kfull : 0;
-    if (nfast > 0) {
-        load_tile(0, std::false_type());
-        store_tile(0, 0, std::false_type());
-    } else if (ktiles > 0) {
-        load_tile(0, std::true_type());
-        store_tile(0, 0, std::true_type());
+    if (grp < nfast) {
+        load_tile(grp, std::false_type());
+        store_tile(grp, 0, std::false_type());
+    } else if (grp < ktiles) {
+        load_tile(grp, std::true_type());
+        store_tile(grp, 0, std::true_type());
     }
     __syncthreads();
 
     const int frow = lane & 15, fk = lane >> 4;
-    auto step = [&](int kt, bool more, auto edge) {   // edge: of the next K tile
-        const int buf = kt & 1;
-        if (more) load_tile(kt + 1, edge);
+    auto step = [&](int kt, int buf, bool more, auto edge) {   // edge: of the group's next K tile
+        if (more) load_tile(kt + KG, edge);
         __builtin_amdgcn_sched_barrier(0);   // the loads stay in front of the multiplications
         const double *as = As + buf * BK * LDA + fk * LDA + wm * CF::WTM + frow;
         const double *bs = Bs + buf * BK * LDB + fk * LDB + wn * CF::WTN + frow;
@@ -128,12 +136,45 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(2))) voi
                 for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i], fb[j], acc[i][j], 0, 0, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
-        if (more) store_tile(kt + 1, buf ^ 1, edge);
+        if (more) store_tile(kt + KG, buf ^ 1, edge);
         __syncthreads();
     };
-    int kt = 0;
-    for (; kt + 1 < nfast; ++kt) step(kt, true, std::false_type());
-    for (; kt < ktiles; ++kt) step(kt, kt + 1 < ktiles, std::true_type());
+    int kt = grp, buf = 0;
+    for (; kt + KG < nfast; kt += KG, buf ^= 1) step(kt, buf, true, std::false_type());
+    for (; kt < ktiles; kt += KG, buf ^= 1) step(kt, buf, kt + KG < ktiles, std::true_type());
+    if constexpr (KG > 1) {
+        // Groups with one K tile less join the last step's barrier.
+        if (ktiles % KG != 0 && grp >= ktiles % KG) __syncthreads();
+    }
+
+    if constexpr (KG > 1) {
+        // The groups' sums into LDS (their stages are free: every step ends
+        // with a barrier), then group g adds up fragments g, g + KG, ... in
+        // group order and finishes them.
+        doublex4 *red = reinterpret_cast<doublex4 *>(lds);
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) red[((grp * FM + i) * FN + j) * NT + t] = acc[i][j];
+        __syncthreads();
+#pragma unroll 1
+        for (int q = grp; q < FM * FN; q += KG) {
+            doublex4 sum = red[q * NT + t];
+#pragma unroll
+            for (int h = 1; h < KG; ++h) sum += red[(h * FM * FN + q) * NT + t];
+            const int mb = m0 + wm * CF::WTM + (q / FN) * 16 + (lane >> 4);
+            const int n = n0 + wn * CF::WTN + (q % FN) * 16 + (lane & 15);
+            double cv[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                cv[r] = (beta != 0.0 && mb + 4 * r < M && n < N) ? C[(long)(mb + 4 * r) * ldc + n] : 0.0;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (mb + 4 * r < M && n < N)
+                    C[(long)(mb + 4 * r) * ldc + n] = (beta == 0.0) ? alpha * sum[r] : fma(alpha, sum[r], beta * cv[r]);
+        }
+        return;
+    }
 
     // C values of one fragment row are loaded before any is stored (a load
     // cannot pass a possibly aliasing store: one latency per row, not per element).
@@ -168,6 +209,9 @@ using D0 = DCfg<128, 128>;
 using D1 = DCfg<64, 64>;
 using D2 = DCfg<128, 64>;
 using D3 = DCfg<64, 128>;
+// Small grids (launch_small): K dealt to groups of one workgroup.
+using D1K4 = DCfg<64, 64, 2, 4, 4>;
+using D1S8 = DCfg<32, 32, 1, 8, 2>;
 const char *kNames[] = {"f64_mfma_128x128x16", "f64_mfma_64x64x16", "f64_mfma_128x64x16", "f64_mfma_64x128x16"};
 constexpr int kNum = 4;
 
@@ -183,7 +227,7 @@ int launch_cfg(const Gemm<double> &g, hipStream_t s) {
         const int rc = stream_alloc((void **)&ws, (size_t)splits * g.M * g.N * sizeof(double), s);
         if (rc) return rc;
     }
-    dim3 grid((unsigned)nblk, (unsigned)splits), block(CF::NT);
+    dim3 grid((unsigned)nblk, (unsigned)splits), block(CF::NT * CF::KG);
 #define UGEMM_L(TA, TB) \
     hipLaunchKernelGGL((dgemm_mfma_kernel<CF, TA, TB>), grid, block, 0, s, g.M, g.N, g.K, g.alpha, g.A, \
                        g.lda, g.B, g.ldb, g.beta, g.C, g.ldc, tiles_m, tiles_n, kc, ws)
@@ -204,6 +248,25 @@ int launch_cfg(const Gemm<double> &g, hipStream_t s) {
     return rc;
 }
 
+// Variant 1 with the automatic split count: K dealt to groups of a workgroup
+// where the grid leaves a CU one wave a SIMD (the reasons stand at the FP32
+// kernel's launch_small; here 139 KB of LDS leave room for one workgroup of 8
+// groups of 32x32 or of 4 groups of 64x64).  us a call, 64x64x1 / 64x64x4 / 32x32x8:
+//   128x96x200 19.8 / 15.2 / 8.6;  512x512x512 29.8 / 25.5 / 12.1;  36x64x971 73 / 47 / 20;
+//   1023x1000x1023 89 / 53 / 78;  58x16704x512 (261 of 64x64) 54 / 57 / 69.
+int launch_small(const Gemm<double> &g, hipStream_t s) {
+    const long cus = device_cu_count();
+    const long t32 = (long)((g.M + 31) / 32) * ((g.N + 31) / 32), t64 = (long)((g.M + 63) / 64) * ((g.N + 63) / 64);
+    if (g.splits != 0 || t64 > 4 * cus) return launch_cfg<D1>(g, s);
+    Gemm<double> h = g;
+    h.splits = 1;
+    if (t32 <= cus && t32 * g.K <= cus * 2048) {
+        if (g.K > 1200) h.splits = (int)std::max(1L, std::min({cus / t32, g.K / 512L, 16L}));
+        return launch_cfg<D1S8>(h, s);
+    }
+    return deal_k(t64, g.K, 38.0, 1, &h.splits) ? (h.splits = 1, launch_cfg<D1K4>(h, s)) : launch_cfg<D1>(h, s);
+}
+
 }  // namespace
 
 int dgemm_variant_count() { return kNum; }
@@ -214,15 +277,17 @@ int dgemm_pick_variant(const Gemm<double> &g) {
     const long t128 = (long)((g.M + 127) / 128) * ((g.N + 127) / 128);
     if (t128 >= 2 * cus) return 0;
     const long t64 = (long)((g.M + 63) / 64) * ((g.N + 63) / 64);
-    if (g.M >= 4L * g.N && t64 >= cus) return 2;
-    if (g.N >= 4L * g.M && t64 >= cus) return 3;
+    if (t64 > 4 * cus) {
+        if (g.M >= 4L * g.N) return 2;
+        if (g.N >= 4L * g.M) return 3;
+    }
     return 1;
 }
 
 int launch_dgemm(const Gemm<double> &g, int variant, hipStream_t s) {
     switch (variant) {
         case 0: return launch_cfg<D0>(g, s);
-        case 1: return launch_cfg<D1>(g, s);
+        case 1: return launch_small(g, s);
         case 2: return launch_cfg<D2>(g, s);
         case 3: return launch_cfg<D3>(g, s);
         default: return fail(UGEMM_ERR_ARG, "dgemm: no variant %d", variant);

@@ -50,19 +50,25 @@ __device__ __forceinline__ void pin_step(float (&acc)[TM][TN]) {
         }
 }
 
-// MINB_: workgroups per CU the kernel is compiled for (register budget).
-template <int BM_, int BN_, int BK_, int TM_, int TN_, int MINB_ = 1>
+// MINB_: waves per SIMD the kernel is compiled for (register budget).
+// KG_: groups of NT threads in a workgroup, each with its own LDS stages.
+// Group g multiplies K tiles g, g + KG, ...; the groups' sums are added
+// through LDS in group order.  For grids that leave CUs short of waves: one
+// wave a SIMD hides no latency of its K steps.
+template <int BM_, int BN_, int BK_, int TM_, int TN_, int MINB_ = 1, int KG_ = 1>
 struct Fp32Cfg {
     static constexpr int BM = BM_, BN = BN_, BK = BK_, TM = TM_, TN = TN_, MINB = MINB_;
     static constexpr int TX = BN / TN, TY = BM / TM;
-    static constexpr int NT = TX * TY;
+    static constexpr int NT = TX * TY, KG = KG_, THREADS = NT * KG;
     static_assert(TM % 4 == 0 && TN % 4 == 0, "micro-tile built from 4-wide groups");
     static_assert(TX % 8 == 0 && TY % 8 == 0 && NT % 64 == 0, "waves are 8x8 thread grids");
     static constexpr int LDA = BM + LDS_PAD, LDB = BN + LDS_PAD;
+    static constexpr int kStageFloats = 2 * BK * (LDA + LDB), kLdsFloats = KG * kStageFloats;   // two stages a group
+    static_assert(KG == 1 || BM * BN <= kStageFloats, "the groups' sums fit their stages");
 };
 
 // One workgroup computes the C tile at (m0, n0) of g; shared by the plain and
-// the grouped (persistent) kernels. lds must hold 2*(BK*LDA + BK*LDB) floats.
+// the grouped (persistent) kernels. lds must hold CF::kLdsFloats floats.
 // CONV: opB is the implicit im2col matrix of cd (B and TB unused): every
 // thread keeps one column n of the B tile, so the pixel's origin is computed
 // once per tile and each element costs one table read and two compares.
@@ -76,10 +82,12 @@ __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K,
                                           const ConvDesc &cd = ConvDesc()) {
     constexpr int BM = CF::BM, BN = CF::BN, BK = CF::BK, TM = CF::TM, TN = CF::TN, NT = CF::NT;
     constexpr int LDA = CF::LDA, LDB = CF::LDB;
-    float *As = lds;                    // [2][BK][LDA]
-    float *Bs = lds + 2 * BK * LDA;     // [2][BK][LDB]
+    constexpr int KG = CF::KG;
+    const int grp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);   // NT: whole waves
+    float *As = lds + grp * CF::kStageFloats;   // [2][BK][LDA]
+    float *Bs = As + 2 * BK * LDA;              // [2][BK][LDB]
 
-    const int t = threadIdx.x;
+    const int t = KG == 1 ? threadIdx.x : threadIdx.x % NT;
     const int lane = t & 63, w = t >> 6;
     constexpr int WX = CF::TX / 8;
     const int tx = (lane & 7) + 8 * (w % WX);
@@ -166,18 +174,17 @@ __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K,
     // K tiles below nfast are loaded without bounds; the others (all of an
     // edge tile's, and a K remainder) as edges, in a loop of their own.
     const int nfast = interior ? kfull : 0;
-    if (nfast > 0) {
-        load_tile(0, std::false_type());
-        store_tile(0, 0, std::false_type());
-    } else if (ktiles > 0) {
-        load_tile(0, std::true_type());
-        store_tile(0, 0, std::true_type());
+    if (grp < nfast) {
+        load_tile(grp, std::false_type());
+        store_tile(grp, 0, std::false_type());
+    } else if (grp < ktiles) {
+        load_tile(grp, std::true_type());
+        store_tile(grp, 0, std::true_type());
     }
     __syncthreads();
 
-    auto step = [&](int kt, bool more, auto edge) {   // edge: of the next K tile
-        const int buf = kt & 1;
-        if (more) load_tile(kt + 1, edge);
+    auto step = [&](int kt, int buf, bool more, auto edge) {   // edge: of the group's next K tile
+        if (more) load_tile(kt + KG, edge);
         __builtin_amdgcn_sched_barrier(0);   // the loads stay in front of the multiplications
         const float *as = As + buf * BK * LDA + ty * 4;
         const float *bs = Bs + buf * BK * LDB + tx * 4;
@@ -210,49 +217,78 @@ __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K,
             pin_step(acc);
         }
         __builtin_amdgcn_sched_barrier(0);
-        if (more) store_tile(kt + 1, buf ^ 1, edge);
+        if (more) store_tile(kt + KG, buf ^ 1, edge);
         __syncthreads();
     };
-    int kt = 0;
-    for (; kt + 1 < nfast; ++kt) step(kt, true, std::false_type());
-    for (; kt < ktiles; ++kt) step(kt, kt + 1 < ktiles, std::true_type());
+    int kt = grp, buf = 0;
+    for (; kt + KG < nfast; kt += KG, buf ^= 1) step(kt, buf, true, std::false_type());
+    for (; kt < ktiles; kt += KG, buf ^= 1) step(kt, buf, kt + KG < ktiles, std::true_type());
+    if constexpr (KG > 1) {
+        // Groups with one K tile less join the last step's barrier.
+        if (ktiles % KG != 0 && grp >= ktiles % KG) __syncthreads();
+    }
 
-    // Epilogue: C = alpha * acc (+ beta * C), then bias and activation.
+    // Epilogue: C = alpha * acc (+ beta * C), then bias and activation, of
+    // four columns n .. n + 3 of row m.
     const bool has_epi = epi.active();
+    auto finish = [&](int m, int n, const f32x4u &q) {
+        float *cp = C + (long)m * ldc + n;
+        if (interior) {
+            f32x4u o;
+            if (beta == 0.0f) {
+                o = alpha * q;
+            } else {
+                const f32x4u c = *reinterpret_cast<const f32x4u *>(cp);
+                o = f32x4u{fmaf(alpha, q.x, beta * c.x), fmaf(alpha, q.y, beta * c.y), fmaf(alpha, q.z, beta * c.z),
+                           fmaf(alpha, q.w, beta * c.w)};
+            }
+            if (has_epi) {
+                o.x = apply_epilogue(epi, o.x, m, n);
+                o.y = apply_epilogue(epi, o.y, m, n + 1);
+                o.z = apply_epilogue(epi, o.z, m, n + 2);
+                o.w = apply_epilogue(epi, o.w, m, n + 3);
+            }
+            *reinterpret_cast<f32x4u *>(cp) = o;
+        } else if (m < M) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-        const int m = m0 + (i / 4) * CF::TY * 4 + ty * 4 + (i % 4);
-#pragma unroll
-        for (int g = 0; g < TN / 4; ++g) {
-            const int n = n0 + g * CF::TX * 4 + tx * 4;
-            float *cp = C + (long)m * ldc + n;
-            const f32x4u q = {acc[i][g * 4], acc[i][g * 4 + 1], acc[i][g * 4 + 2], acc[i][g * 4 + 3]};
-            if (interior) {
-                f32x4u o;
-                if (beta == 0.0f) {
-                    o = alpha * q;
-                } else {
-                    const f32x4u c = *reinterpret_cast<const f32x4u *>(cp);
-                    o = f32x4u{fmaf(alpha, q.x, beta * c.x), fmaf(alpha, q.y, beta * c.y),
-                               fmaf(alpha, q.z, beta * c.z), fmaf(alpha, q.w, beta * c.w)};
-                }
-                if (has_epi) {
-                    o.x = apply_epilogue(epi, o.x, m, n);
-                    o.y = apply_epilogue(epi, o.y, m, n + 1);
-                    o.z = apply_epilogue(epi, o.z, m, n + 2);
-                    o.w = apply_epilogue(epi, o.w, m, n + 3);
-                }
-                *reinterpret_cast<f32x4u *>(cp) = o;
-            } else if (m < M) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if (n + j < N) {
-                        float r = (beta == 0.0f) ? alpha * q[j] : fmaf(alpha, q[j], beta * cp[j]);
-                        if (has_epi) r = apply_epilogue(epi, r, m, n + j);
-                        cp[j] = r;
-                    }
+            for (int j = 0; j < 4; ++j) {
+                if (n + j < N) {
+                    float r = (beta == 0.0f) ? alpha * q[j] : fmaf(alpha, q[j], beta * cp[j]);
+                    if (has_epi) r = apply_epilogue(epi, r, m, n + j);
+                    cp[j] = r;
                 }
             }
+        }
+    };
+    constexpr int TG = TN / 4;
+    if constexpr (KG == 1) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int g = 0; g < TG; ++g)
+                finish(m0 + (i / 4) * CF::TY * 4 + ty * 4 + (i % 4), n0 + g * CF::TX * 4 + tx * 4,
+                       f32x4u{acc[i][g * 4], acc[i][g * 4 + 1], acc[i][g * 4 + 2], acc[i][g * 4 + 3]});
+    } else {
+        // The groups' sums into LDS (their stages are free: every step ends
+        // with a barrier), then group g adds up quads g, g + KG, ... of every
+        // thread's micro-tile, in group order.
+        typedef float quad __attribute__((ext_vector_type(4)));
+        quad *red = reinterpret_cast<quad *>(lds);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int g = 0; g < TG; ++g)
+                red[(grp * TM * TG + i * TG + g) * NT + t] =
+                    quad{acc[i][g * 4], acc[i][g * 4 + 1], acc[i][g * 4 + 2], acc[i][g * 4 + 3]};
+        __syncthreads();
+#pragma unroll 1
+        for (int q = grp; q < TM * TG; q += KG) {
+            quad sum = red[q * NT + t];
+#pragma unroll
+            for (int h = 1; h < KG; ++h) sum += red[(h * TM * TG + q) * NT + t];
+            const int i = q / TG, g = q % TG;
+            finish(m0 + (i / 4) * CF::TY * 4 + ty * 4 + (i % 4), n0 + g * CF::TX * 4 + tx * 4,
+                   f32x4u{sum.x, sum.y, sum.z, sum.w});
         }
     }
 }

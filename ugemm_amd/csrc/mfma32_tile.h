@@ -32,11 +32,14 @@ namespace {
 
 typedef float m32_floatx4 __attribute__((ext_vector_type(4)));
 
-// MINB_: workgroups per CU the kernel is compiled for (register budget).
-template <int BM_, int BN_, int BK_, int WGM_, int WGN_, int MINB_ = 1>
+// MINB_: waves per SIMD the kernel is compiled for (register budget).
+// KG_: groups of WGM x WGN waves in a workgroup, each with its own LDS stages;
+// group g multiplies K tiles g, g + KG, ... and the groups' sums are added
+// through LDS in group order (small grids, as Fp32Cfg).
+template <int BM_, int BN_, int BK_, int WGM_, int WGN_, int MINB_ = 1, int KG_ = 1>
 struct M32Cfg {
     static constexpr int BM = BM_, BN = BN_, BK = BK_, WGM = WGM_, WGN = WGN_, MINB = MINB_;
-    static constexpr int NT = 64 * WGM * WGN;
+    static constexpr int NT = 64 * WGM * WGN, KG = KG_, THREADS = NT * KG;
     static constexpr int WTM = BM / WGM, WTN = BN / WGN, FM = WTM / 16, FN = WTN / 16;
     static_assert(BK % 16 == 0 && WTM % 16 == 0 && WTN % 16 == 0, "fragment-aligned tile");
     // LDS row length and stage size (floats) of an operand tile of ROWS rows.
@@ -45,13 +48,16 @@ struct M32Cfg {
     template <bool KC, int ROWS>
     static constexpr int stage() { return KC ? ROWS * (BK + 4) : BK * (ROWS + 4); }
     // LDS floats of the largest layout (both operands k-contiguous).
-    static constexpr int kLdsFloats = 2 * (BM + BN) * (BK + 4);
+    static constexpr int kLdsFloats = KG * 2 * (BM + BN) * (BK + 4);
+    // Of one layout (two stages of both operands a group).
+    template <bool TA, bool TB>
+    static constexpr int lds_floats() { return KG * 2 * (stage<!TA, BM>() + stage<TB, BN>()); }
 };
 
 template <class CF>
 struct IsM32 : std::false_type {};
-template <int BM, int BN, int BK, int WGM, int WGN, int MINB>
-struct IsM32<M32Cfg<BM, BN, BK, WGM, WGN, MINB>> : std::true_type {};
+template <int BM, int BN, int BK, int WGM, int WGN, int MINB, int KG>
+struct IsM32<M32Cfg<BM, BN, BK, WGM, WGN, MINB, KG>> : std::true_type {};
 
 // The lane's four k values (k .. k+3) of fragment row `row`.
 template <bool KC, int LD>
@@ -80,11 +86,14 @@ __device__ __forceinline__ void m32_tile(const int M, const int N, const int K, 
     constexpr int BM = CF::BM, BN = CF::BN, BK = CF::BK, NT = CF::NT, FM = CF::FM, FN = CF::FN;
     constexpr int LDA = CF::template ld<KCA, BM>(), LDB = CF::template ld<KCB, BN>();
     constexpr int SA = CF::template stage<KCA, BM>(), SB = CF::template stage<KCB, BN>();
-    static_assert(2 * (SA + SB) <= CF::kLdsFloats, "LDS budget");
-    float *As = lds, *Bs = lds + 2 * SA;
+    constexpr int KG = CF::KG;
+    static_assert(KG * 2 * (SA + SB) <= CF::kLdsFloats, "LDS budget");
+    static_assert(KG == 1 || BM * BN <= 2 * (SA + SB), "the groups' sums fit their stages");
+    const int grp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
+    float *As = lds + grp * 2 * (SA + SB), *Bs = As + 2 * SA;
     const bool has_epi = epi.active();
 
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int t = KG == 1 ? threadIdx.x : threadIdx.x % NT, lane = t & 63, w = t >> 6;
     const int wm = w / CF::WGN, wn = w % CF::WGN;
 
     using ARegs = TileRegs<float, KCA ? BK : BM, KCA ? BM : BK, NT>;
@@ -163,19 +172,18 @@ __device__ __forceinline__ void m32_tile(const int M, const int N, const int K, 
     // K tiles below nfast are loaded without bounds; the others (all of an
     // edge tile's, and a K remainder) as edges, in a loop of their own.
     const int nfast = interior ? kfull : 0;
-    if (nfast > 0) {
-        load_tile(0, std::false_type());
-        store_tile(0, 0, std::false_type());
-    } else if (ktiles > 0) {
-        load_tile(0, std::true_type());
-        store_tile(0, 0, std::true_type());
+    if (grp < nfast) {
+        load_tile(grp, std::false_type());
+        store_tile(grp, 0, std::false_type());
+    } else if (grp < ktiles) {
+        load_tile(grp, std::true_type());
+        store_tile(grp, 0, std::true_type());
     }
     __syncthreads();
 
     const int frow = lane & 15, g4 = (lane >> 4) * 4;
-    auto step = [&](int kt, bool more, auto edge) {   // edge: of the next K tile
-        const int buf = kt & 1;
-        if (more) load_tile(kt + 1, edge);
+    auto step = [&](int kt, int buf, bool more, auto edge) {   // edge: of the group's next K tile
+        if (more) load_tile(kt + KG, edge);
         __builtin_amdgcn_sched_barrier(0);   // the loads stay in front of the multiplications
         const float *as = As + buf * SA, *bs = Bs + buf * SB;
 #pragma unroll
@@ -194,12 +202,48 @@ __device__ __forceinline__ void m32_tile(const int M, const int N, const int K, 
                         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i][q], fb[j][q], acc[i][j], 0, 0, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
-        if (more) store_tile(kt + 1, buf ^ 1, edge);
+        if (more) store_tile(kt + KG, buf ^ 1, edge);
         __syncthreads();
     };
-    int kt = 0;
-    for (; kt + 1 < nfast; ++kt) step(kt, true, std::false_type());
-    for (; kt < ktiles; ++kt) step(kt, kt + 1 < ktiles, std::true_type());
+    int kt = grp, buf = 0;
+    for (; kt + KG < nfast; kt += KG, buf ^= 1) step(kt, buf, true, std::false_type());
+    for (; kt < ktiles; kt += KG, buf ^= 1) step(kt, buf, kt + KG < ktiles, std::true_type());
+    if constexpr (KG > 1) {
+        // Groups with one K tile less join the last step's barrier.
+        if (ktiles % KG != 0 && grp >= ktiles % KG) __syncthreads();
+    }
+
+    if constexpr (KG > 1) {
+        // The groups' sums into LDS (their stages are free: every step ends
+        // with a barrier), then group g adds up fragments g, g + KG, ... in
+        // group order and finishes them.
+        m32_floatx4 *red = reinterpret_cast<m32_floatx4 *>(lds);
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) red[((grp * FM + i) * FN + j) * NT + t] = acc[i][j];
+        __syncthreads();
+#pragma unroll 1
+        for (int q = grp; q < FM * FN; q += KG) {
+            m32_floatx4 sum = red[q * NT + t];
+#pragma unroll
+            for (int h = 1; h < KG; ++h) sum += red[(h * FM * FN + q) * NT + t];
+            const int mb = m0 + wm * CF::WTM + (q / FN) * 16 + 4 * (lane >> 4);
+            const int n = n0 + wn * CF::WTN + (q % FN) * 16 + (lane & 15);
+            float cv[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                cv[r] = (beta != 0.0f && mb + r < M && n < N) ? C[(long)(mb + r) * ldc + n] : 0.0f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (mb + r < M && n < N) {
+                    float v = (beta == 0.0f) ? alpha * sum[r] : fmaf(alpha, sum[r], beta * cv[r]);
+                    if (has_epi) v = apply_epilogue(epi, v, mb + r, n);
+                    C[(long)(mb + r) * ldc + n] = v;
+                }
+        }
+        return;
+    }
 
     // C values of one fragment row are loaded before any is stored (a load
     // cannot pass a possibly aliasing store: one latency per row, not per element).

@@ -1,6 +1,8 @@
 // Plain FP32 SGEMM for gfx950: vector FMA with FP32 accumulation, one
 // workgroup per C tile (tile body in fp32_tile.h).  Tiles are visited in the
 // XCD-aware order of tile_coords (kernel_common.h).
+#include <algorithm>
+
 #include "internal.h"
 #include "fp32_tile.h"
 
@@ -10,12 +12,12 @@ namespace {
 // Split-K (gridDim.y > 1): block (tile, z) multiplies K columns
 // [z*kc, min(K, (z+1)*kc)) into the partial slice ws + z*M*N (row length N).
 template <class CF, bool TA, bool TB>
-__global__ __launch_bounds__(CF::NT, CF::MINB) void sgemm_fp32_kernel(int M, int N, int K, float alpha,
+__global__ __launch_bounds__(CF::THREADS, CF::MINB) void sgemm_fp32_kernel(int M, int N, int K, float alpha,
                                                             const float *__restrict__ A, long lda,
                                                             const float *__restrict__ B, long ldb, float beta,
                                                             float *__restrict__ C, long ldc, int tiles_m, int tiles_n,
                                                             Epilogue epi, int kc, float *__restrict__ ws) {
-    __shared__ __attribute__((aligned(16))) float lds[2 * CF::BK * (CF::LDA + CF::LDB)];
+    __shared__ __attribute__((aligned(16))) float lds[CF::kLdsFloats];
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
     const bool part = gridDim.y > 1;
@@ -36,7 +38,7 @@ __global__ __launch_bounds__(CF::NT) void conv_fp32_kernel(int M, int N, int K, 
                                                            const float *__restrict__ A, long lda, float beta,
                                                            float *__restrict__ C, long ldc, int tiles_m, int tiles_n,
                                                            Epilogue epi, ConvDesc cd, int kc, float *__restrict__ ws) {
-    __shared__ __attribute__((aligned(16))) float lds[2 * CF::BK * (CF::LDA + CF::LDB)];
+    __shared__ __attribute__((aligned(16))) float lds[CF::kLdsFloats];
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
     const bool part = gridDim.y > 1;
@@ -57,6 +59,11 @@ using V3 = Fp32Cfg<64, 128, 16, 4, 8>;
 using V4 = Fp32Cfg<256, 128, 16, 16, 8, 2>;
 using V5 = Fp32Cfg<128, 256, 16, 8, 16, 2>;
 
+// Small grids (launch_small): K dealt to groups of one workgroup.
+using V1K4 = Fp32Cfg<64, 64, 16, 4, 4, 1, 4>;
+using V1S8 = Fp32Cfg<32, 32, 16, 4, 4, 1, 8>;
+using V1S16 = Fp32Cfg<32, 32, 16, 4, 4, 1, 16>;
+
 const char *kNames[] = {"fp32_128x128x16_t8x8", "fp32_64x64x16_t4x4", "fp32_128x64x16_t8x4",
                         "fp32_64x128x16_t4x8", "fp32_256x128x16_t16x8", "fp32_128x256x16_t8x16"};
 constexpr int kNumVariants = 6;
@@ -74,7 +81,7 @@ int launch_cfg(const Gemm<float> &g, hipStream_t s) {
         const int rc = stream_alloc((void **)&ws, (size_t)splits * g.M * g.N * sizeof(float), s);
         if (rc) return rc;
     }
-    dim3 grid((unsigned)nblk, (unsigned)splits), block(CF::NT);
+    dim3 grid((unsigned)nblk, (unsigned)splits), block(CF::THREADS);
 #define UGEMM_L(TA, TB) \
     hipLaunchKernelGGL((sgemm_fp32_kernel<CF, TA, TB>), grid, block, 0, s, g.M, g.N, g.K, g.alpha, g.A, \
                        g.lda, g.B, g.ldb, g.beta, g.C, g.ldc, tiles_m, tiles_n, g.epi, kc, ws)
@@ -93,6 +100,32 @@ int launch_cfg(const Gemm<float> &g, hipStream_t s) {
         if (!rc) rc = rc2;
     }
     return rc;
+}
+
+// Variant 1 with the automatic split count.  A grid of few tiles leaves a CU
+// one wave a SIMD and a serial chain of K steps of 1.2 us each; K is then
+// dealt to the groups of a workgroup instead of a second launch (which, with
+// its workspace, costs 14 us on top of a 7 us call).  us a call by tile and
+// groups, 64x64x1 / 64x64x4 / 32x32x8 / 32x32x16:
+//   128x96x200 (12 tiles of 32x32) 17.5 / 10.9 / 6.8 / 6.9;  512x512x512 (256) 27.5 / 16.9 / 8.7 / 8.8;
+//   28x768x1472 (24) 96 / 44 / 19.9 / 17.7;  700x700x2000 (484) 157 / 61 / 41.6 / 43.0;
+//   1023x1000x1023 (1024; 256 of 64x64) 82 / 37 / 44 / 50;  1400x1400x300 (484 of 64x64) 26.0 / 23.9 / 31 / 47;
+//   2720x1313x87 (903 of 64x64) 18.2 / 19.5 / 27 / 49.
+// 32x32 tiles in groups of 8 or 16 serve the smallest grids (at 7 us per 1000
+// of K; past 2048 the CUs that are left take chunks of it) while the product
+// is short of 4096 of K on every CU; deal_k chooses for the others.
+int launch_small(const Gemm<float> &g, hipStream_t s) {
+    const long cus = device_cu_count();
+    const long t32 = (long)((g.M + 31) / 32) * ((g.N + 31) / 32), t64 = (long)((g.M + 63) / 64) * ((g.N + 63) / 64);
+    if (g.splits != 0 || t64 > 4 * cus) return launch_cfg<V1>(g, s);
+    Gemm<float> h = g;
+    h.splits = 1;
+    if (t32 <= cus && t32 * g.K <= cus * 4096) {
+        if (g.K > 2048) h.splits = (int)std::max(1L, std::min({cus / t32, g.K / 1024L, 16L}));
+        return launch_cfg<V1S16>(h, s);
+    }
+    if (t32 <= 2 * cus && g.K <= 2048) return launch_cfg<V1S8>(h, s);
+    return deal_k(t64, g.K, 28.0, 2, &h.splits) ? (h.splits = 1, launch_cfg<V1K4>(h, s)) : launch_cfg<V1>(h, s);
 }
 
 template <class CF>
@@ -148,8 +181,10 @@ int fp32_pick_variant(const Gemm<float> &g) {
     if (t128 >= 2L * cus) return 0;
     if (2 * t128x256 >= cus && g.K >= 1024 && g.splits != 1) return 5;
     const long t64 = (long)((g.M + 63) / 64) * ((g.N + 63) / 64);
-    if (g.M >= 4 * g.N && t64 >= cus) return 2;
-    if (g.N >= 4 * g.M && t64 >= cus) return 3;
+    if (t64 > 2L * cus) {
+        if (g.M >= 4 * g.N) return 2;
+        if (g.N >= 4 * g.M) return 3;
+    }
     return 1;
 }
 
@@ -169,7 +204,7 @@ int launch_conv_fp32(const Gemm<float> &g, const ConvDesc &cd, int variant, hipS
 int launch_fp32(const Gemm<float> &g, int variant, hipStream_t s) {
     switch (variant) {
         case 0: return launch_cfg<V0>(g, s);
-        case 1: return launch_cfg<V1>(g, s);
+        case 1: return launch_small(g, s);
         case 2: return launch_cfg<V2>(g, s);
         case 3: return launch_cfg<V3>(g, s);
         case 4: return launch_cfg<V4>(g, s);

@@ -11,6 +11,8 @@
 // [z*kc, min(K, (z+1)*kc)) into the partial slice ws + z*M*N; the partials
 // are added in fixed order by the split-K reduction, which also applies
 // alpha, beta and the epilogue.  Repeated calls are bitwise identical.
+#include <algorithm>
+
 #include "internal.h"
 #include "kernel_common.h"
 #include "mfma32_tile.h"
@@ -19,13 +21,12 @@ namespace ugemm {
 namespace {
 
 template <class CF, bool TA, bool TB>
-__global__ __launch_bounds__(CF::NT, CF::MINB) void sgemm_mfma32_kernel(
+__global__ __launch_bounds__(CF::THREADS, CF::MINB) void sgemm_mfma32_kernel(
     int M, int N, int K_, float alpha_, const float *__restrict__ A_, long lda, const float *__restrict__ B_,
     long ldb, float beta_, float *__restrict__ C_, long ldc_, int tiles_m, int tiles_n, Epilogue epi, int kc,
     float *__restrict__ ws) {
     // This layout's two stages of both operands (at most CF::kLdsFloats).
-    constexpr int kLds = 2 * (CF::template stage<!TA, CF::BM>() + CF::template stage<TB, CF::BN>());
-    __shared__ __attribute__((aligned(16))) float lds[kLds];
+    __shared__ __attribute__((aligned(16))) float lds[CF::template lds_floats<TA, TB>()];
     const bool part = gridDim.y > 1;
     const int kz0 = part ? (int)blockIdx.y * kc : 0;
     const int K = part ? min(kc, K_ - kz0) : K_;
@@ -66,6 +67,11 @@ using V2 = M32Cfg<128, 256, 16, 2, 4>;
 using V3 = M32Cfg<64, 64, 16, 2, 2, 2>;
 using V4 = M32Cfg<256, 256, 16, 2, 4>;
 using V5 = M32Cfg<128, 128, 32, 2, 2, 2>;
+// Small grids (launch_small): K dealt to groups of one workgroup.
+using V3K4 = M32Cfg<64, 64, 16, 2, 2, 1, 4>;
+using V3S8 = M32Cfg<32, 32, 16, 1, 1, 1, 8>;
+using V3S16 = M32Cfg<32, 32, 16, 1, 1, 1, 16>;
+
 const char *kNames[] = {"f32_mfma_128x128x16_w2x2", "f32_mfma_256x128x16_w4x2", "f32_mfma_128x256x16_w2x4",
                         "f32_mfma_64x64x16_w2x2",   "f32_mfma_256x256x16_w2x4", "f32_mfma_128x128x32_w2x2"};
 constexpr int kNum = 6;
@@ -82,7 +88,7 @@ int launch_cfg(const Gemm<float> &g, hipStream_t s) {
         const int rc = stream_alloc((void **)&ws, (size_t)splits * g.M * g.N * sizeof(float), s);
         if (rc) return rc;
     }
-    dim3 grid((unsigned)nblk, (unsigned)splits), block(CF::NT);
+    dim3 grid((unsigned)nblk, (unsigned)splits), block(CF::THREADS);
 #define UGEMM_L(TA, TB) \
     hipLaunchKernelGGL((sgemm_mfma32_kernel<CF, TA, TB>), grid, block, 0, s, g.M, g.N, g.K, g.alpha, g.A, \
                        g.lda, g.B, g.ldb, g.beta, g.C, g.ldc, tiles_m, tiles_n, g.epi, kc, ws)
@@ -101,6 +107,25 @@ int launch_cfg(const Gemm<float> &g, hipStream_t s) {
         if (!rc) rc = rc2;
     }
     return rc;
+}
+
+// Variant 3 with the automatic split count: K dealt to groups of a workgroup
+// where the grid leaves a CU one wave a SIMD (the reasons stand at the FP32
+// kernel's launch_small).  us a call, 64x64x1 / 64x64x4 / 32x32x8 / 32x32x16:
+//   128x96x200 14.2 / 10.4 / 6.8 / 7.1;  512x512x512 18.8 / 15.8 / 8.6 / 8.9;  28x768x1472 65 / 41 / 18 / 17;
+//   700x700x2000 115 / 54 / 36 / 37;  1023x1000x1023 61 / 31 / 38 / 46;  2720x1313x87 17.1 / 18.7 / 30 / 52.
+int launch_small(const Gemm<float> &g, hipStream_t s) {
+    const long cus = device_cu_count();
+    const long t32 = (long)((g.M + 31) / 32) * ((g.N + 31) / 32), t64 = (long)((g.M + 63) / 64) * ((g.N + 63) / 64);
+    if (g.splits != 0 || t64 > 4 * cus) return launch_cfg<V3>(g, s);
+    Gemm<float> h = g;
+    h.splits = 1;
+    if (t32 <= cus && t32 * g.K <= cus * 4096) {
+        if (g.K > 2048) h.splits = (int)std::max(1L, std::min({cus / t32, g.K / 1024L, 16L}));
+        return launch_cfg<V3S16>(h, s);
+    }
+    if (t32 <= 2 * cus && g.K <= 2048) return launch_cfg<V3S8>(h, s);
+    return deal_k(t64, g.K, 21.0, 2, &h.splits) ? (h.splits = 1, launch_cfg<V3K4>(h, s)) : launch_cfg<V3>(h, s);
 }
 
 template <class CF>
@@ -165,7 +190,7 @@ int launch_m32(const Gemm<float> &g, int variant, hipStream_t s) {
         case 0: return launch_cfg<V0>(g, s);
         case 1: return launch_cfg<V1>(g, s);
         case 2: return launch_cfg<V2>(g, s);
-        case 3: return launch_cfg<V3>(g, s);
+        case 3: return launch_small(g, s);
         case 4: return launch_cfg<V4>(g, s);
         case 5: return launch_cfg<V5>(g, s);
         default: return fail(UGEMM_ERR_ARG, "sgemm fp32 mfma: no variant %d", variant);

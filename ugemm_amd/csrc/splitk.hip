@@ -1,6 +1,7 @@
 // Split-K support shared by the FP32, split-form and FP64 kernels: the split
 // count heuristic and the fixed-order reduction of the partial products.
 #include <algorithm>
+#include <cmath>
 
 #include "internal.h"
 
@@ -56,6 +57,32 @@ int split_count(int requested, long tiles, int K, int kalign, int *kc, int per_c
     S = std::max(1, (K + chunk - 1) / chunk);   // every split has a non-empty K range
     *kc = chunk;
     return S;
+}
+
+// The estimate behind the choice, fitted to sweeps of split counts 1-32 and of
+// the grouped kernel over 64..1600 square C and K 200..50176 (FP32, FP32-MFMA,
+// FP64; it is within 15% of the best measured choice there): the CU with the
+// most blocks sets the time; o blocks on a CU lose 0.3 / o of it to latency (a
+// workgroup of four groups counts as four); a chunk pays 64 of K for its first
+// loads and its epilogue; the partial sums cost 50 S / K of the products; and
+// a second launch with its workspace makes a call at least 21 us long.
+// 1400x1024x4096 FP32-MFMA: 205 us with the two-blocks-a-CU rule, 137 with
+// this; 1000x600x5000 FP32 143 and 106; 1024x1024x2048 FP64 95 and 82 (groups).
+bool deal_k(long tiles, int K, double us_per_k1000, int grouped, int *splits) {
+    const double cus = (double)device_cu_count(), t1 = us_per_k1000 * K / 1000.0;
+    const double groups = t1 * std::ceil(tiles / cus) * (1.0 + 0.3 / 4) + 3.0;
+    double best = 0;
+    *splits = 1;
+    for (int S = 1; S <= 32 && (S == 1 || K / S >= 256); ++S) {
+        const double most = std::ceil(tiles * S / cus), o = std::min(most, 5.0);
+        double t = t1 * most / S * (1.0 + 0.3 / o) * (1.0 + 64.0 * S / K);
+        if (S > 1) t = std::max(t * (1.0 + 50.0 * S / K) + 5.0, 21.0);
+        if (S == 1 || t < best) {
+            best = t;
+            *splits = S;
+        }
+    }
+    return tiles <= grouped * cus && groups <= best;
 }
 
 int launch_splitk_reduce_f32(int M, int N, int splits, float alpha, const float *ws, float beta, float *C, long ldc,
