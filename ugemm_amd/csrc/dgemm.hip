@@ -261,7 +261,7 @@ int launch_small(const Gemm<double> &g, hipStream_t s) {
     Gemm<double> h = g;
     h.splits = 1;
     if (t32 <= cus && t32 * g.K <= cus * 2048) {
-        if (g.K > 1200) h.splits = (int)std::max(1L, std::min({cus / t32, g.K / 512L, 16L}));
+        if (g.K > 640) h.splits = (int)std::max(1L, std::min({cus / t32, g.K / 256L, 16L}));
         return launch_cfg<D1S8>(h, s);
     }
     return deal_k(t64, g.K, 38.0, 1, &h.splits) ? (h.splits = 1, launch_cfg<D1K4>(h, s)) : launch_cfg<D1>(h, s);

@@ -104,15 +104,14 @@ int launch_cfg(const Gemm<float> &g, hipStream_t s) {
 
 // Variant 1 with the automatic split count.  A grid of few tiles leaves a CU
 // one wave a SIMD and a serial chain of K steps of 1.2 us each; K is then
-// dealt to the groups of a workgroup instead of a second launch (which, with
-// its workspace, costs 14 us on top of a 7 us call).  us a call by tile and
-// groups, 64x64x1 / 64x64x4 / 32x32x8 / 32x32x16:
+// dealt to the groups of a workgroup instead of chunks and a second launch (5
+// us on top of a 7 us call).  us a call by tile and groups, 64x64x1 / 64x64x4 / 32x32x8 / 32x32x16:
 //   128x96x200 (12 tiles of 32x32) 17.5 / 10.9 / 6.8 / 6.9;  512x512x512 (256) 27.5 / 16.9 / 8.7 / 8.8;
 //   28x768x1472 (24) 96 / 44 / 19.9 / 17.7;  700x700x2000 (484) 157 / 61 / 41.6 / 43.0;
 //   1023x1000x1023 (1024; 256 of 64x64) 82 / 37 / 44 / 50;  1400x1400x300 (484 of 64x64) 26.0 / 23.9 / 31 / 47;
 //   2720x1313x87 (903 of 64x64) 18.2 / 19.5 / 27 / 49.
 // 32x32 tiles in groups of 8 or 16 serve the smallest grids (at 7 us per 1000
-// of K; past 2048 the CUs that are left take chunks of it) while the product
+// of K; past 1024 the CUs that are left take chunks of it) while the product
 // is short of 4096 of K on every CU; deal_k chooses for the others.
 int launch_small(const Gemm<float> &g, hipStream_t s) {
     const long cus = device_cu_count();
@@ -121,7 +120,7 @@ int launch_small(const Gemm<float> &g, hipStream_t s) {
     Gemm<float> h = g;
     h.splits = 1;
     if (t32 <= cus && t32 * g.K <= cus * 4096) {
-        if (g.K > 2048) h.splits = (int)std::max(1L, std::min({cus / t32, g.K / 1024L, 16L}));
+        if (g.K > 1024) h.splits = (int)std::max(1L, std::min({cus / t32, g.K / 384L, 16L}));
         return launch_cfg<V1S16>(h, s);
     }
     if (t32 <= 2 * cus && g.K <= 2048) return launch_cfg<V1S8>(h, s);

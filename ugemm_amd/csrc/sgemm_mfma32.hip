@@ -121,7 +121,7 @@ int launch_small(const Gemm<float> &g, hipStream_t s) {
     Gemm<float> h = g;
     h.splits = 1;
     if (t32 <= cus && t32 * g.K <= cus * 4096) {
-        if (g.K > 2048) h.splits = (int)std::max(1L, std::min({cus / t32, g.K / 1024L, 16L}));
+        if (g.K > 1024) h.splits = (int)std::max(1L, std::min({cus / t32, g.K / 384L, 16L}));
         return launch_cfg<V3S16>(h, s);
     }
     if (t32 <= 2 * cus && g.K <= 2048) return launch_cfg<V3S8>(h, s);

@@ -64,8 +64,8 @@ int split_count(int requested, long tiles, int K, int kalign, int *kc, int per_c
 // FP64; it is within 15% of the best measured choice there): the CU with the
 // most blocks sets the time; o blocks on a CU lose 0.3 / o of it to latency (a
 // workgroup of four groups counts as four); a chunk pays 64 of K for its first
-// loads and its epilogue; the partial sums cost 50 S / K of the products; and
-// a second launch with its workspace makes a call at least 21 us long.
+// loads and its epilogue; the partial sums cost 50 S / K of the products and a
+// second launch 5 us.
 // 1400x1024x4096 FP32-MFMA: 205 us with the two-blocks-a-CU rule, 137 with
 // this; 1000x600x5000 FP32 143 and 106; 1024x1024x2048 FP64 95 and 82 (groups).
 bool deal_k(long tiles, int K, double us_per_k1000, int grouped, int *splits) {
@@ -76,7 +76,7 @@ bool deal_k(long tiles, int K, double us_per_k1000, int grouped, int *splits) {
     for (int S = 1; S <= 32 && (S == 1 || K / S >= 256); ++S) {
         const double most = std::ceil(tiles * S / cus), o = std::min(most, 5.0);
         double t = t1 * most / S * (1.0 + 0.3 / o) * (1.0 + 64.0 * S / K);
-        if (S > 1) t = std::max(t * (1.0 + 50.0 * S / K) + 5.0, 21.0);
+        if (S > 1) t = t * (1.0 + 50.0 * S / K) + 5.0;
         if (S == 1 || t < best) {
             best = t;
             *splits = S;
