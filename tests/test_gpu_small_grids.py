@@ -78,3 +78,17 @@ def test_epilogue_after_the_groups_sum(mode, M, N, K):
     scale = 1.25 * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64)) + 0.5 * np.abs(C0) + np.abs(bias)
     got = dC.download().astype(np.float64)
     assert np.all(np.abs(got - want) <= orc.tolerance(K + 2) * scale)
+
+
+@pytest.mark.parametrize("mode", [ug.MODE_FP32, ug.MODE_FP32_MFMA])
+@pytest.mark.parametrize("M,N,K", [(1984, 2048, 4096), (1000, 1024, 16384), (1400, 1400, 30000)])
+def test_partial_sums_fit_the_static_scratch(mode, M, N, K):
+    """The no-allocation entry takes these sizes: few enough tiles to split K,
+    but with chunks of it whose partial sums could pass 64 MiB."""
+    dA, dB = hip.DeviceArray((M, K), np.float32), hip.DeviceArray((K, N), np.float32)
+    for d in (dA, dB):
+        hip.check(hip.lib().hipMemset(d.ptr, 0, d.nbytes), "clear")
+    dC = hip.DeviceArray.from_host(np.ones((M, N), np.float32))
+    ug.sgemm_noalloc_dev("R", "N", "N", M, N, K, 1.0, dA, K, dB, N, 0.5, dC, N, mode=mode)
+    hip.synchronize()
+    assert np.all(dC.download() == 0.5)

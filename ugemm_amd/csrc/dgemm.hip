@@ -264,7 +264,7 @@ int launch_small(const Gemm<double> &g, hipStream_t s) {
         if (g.K > 640) h.splits = (int)std::max(1L, std::min({cus / t32, g.K / 256L, 16L}));
         return launch_cfg<D1S8>(h, s);
     }
-    return deal_k(t64, g.K, 38.0, 1, &h.splits) ? (h.splits = 1, launch_cfg<D1K4>(h, s)) : launch_cfg<D1>(h, s);
+    return deal_k(t64, g.K, 38.0, 1, sizeof(*g.C) * g.M * g.N, &h.splits) ? (h.splits = 1, launch_cfg<D1K4>(h, s)) : launch_cfg<D1>(h, s);
 }
 
 }  // namespace

@@ -203,8 +203,9 @@ int split_count(int requested, long tiles, int K, int kalign, int *kc, int per_c
 // deals out K: true for four groups inside each workgroup (one launch), false
 // for *splits chunks (1: none).  us_per_k1000: microseconds a busy CU takes
 // for one tile per 1000 of K; grouped: workgroups of four groups a CU holds
-// (no groups for more tiles than that on every CU).
-bool deal_k(long tiles, int K, double us_per_k1000, int grouped, int *splits);
+// (no groups for more tiles than that on every CU); c_bytes: of one chunk's
+// partial C.
+bool deal_k(long tiles, int K, double us_per_k1000, int grouped, size_t c_bytes, int *splits);
 int launch_splitk_reduce_f32(int M, int N, int splits, float alpha, const float *ws, float beta, float *C, long ldc,
                              const Epilogue &epi, hipStream_t s);
 int launch_splitk_reduce_f64(int M, int N, int splits, double alpha, const double *ws, double beta, double *C,

@@ -124,7 +124,7 @@ int launch_small(const Gemm<float> &g, hipStream_t s) {
         return launch_cfg<V1S16>(h, s);
     }
     if (t32 <= 2 * cus && g.K <= 2048) return launch_cfg<V1S8>(h, s);
-    return deal_k(t64, g.K, 28.0, 2, &h.splits) ? (h.splits = 1, launch_cfg<V1K4>(h, s)) : launch_cfg<V1>(h, s);
+    return deal_k(t64, g.K, 28.0, 2, sizeof(*g.C) * g.M * g.N, &h.splits) ? (h.splits = 1, launch_cfg<V1K4>(h, s)) : launch_cfg<V1>(h, s);
 }
 
 template <class CF>

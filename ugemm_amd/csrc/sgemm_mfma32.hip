@@ -125,7 +125,7 @@ int launch_small(const Gemm<float> &g, hipStream_t s) {
         return launch_cfg<V3S16>(h, s);
     }
     if (t32 <= 2 * cus && g.K <= 2048) return launch_cfg<V3S8>(h, s);
-    return deal_k(t64, g.K, 21.0, 2, &h.splits) ? (h.splits = 1, launch_cfg<V3K4>(h, s)) : launch_cfg<V3>(h, s);
+    return deal_k(t64, g.K, 21.0, 2, sizeof(*g.C) * g.M * g.N, &h.splits) ? (h.splits = 1, launch_cfg<V3K4>(h, s)) : launch_cfg<V3>(h, s);
 }
 
 template <class CF>

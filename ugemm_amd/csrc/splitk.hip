@@ -68,12 +68,13 @@ int split_count(int requested, long tiles, int K, int kalign, int *kc, int per_c
 // second launch 5 us.
 // 1400x1024x4096 FP32-MFMA: 205 us with the two-blocks-a-CU rule, 137 with
 // this; 1000x600x5000 FP32 143 and 106; 1024x1024x2048 FP64 95 and 82 (groups).
-bool deal_k(long tiles, int K, double us_per_k1000, int grouped, int *splits) {
+bool deal_k(long tiles, int K, double us_per_k1000, int grouped, size_t c_bytes, int *splits) {
     const double cus = (double)device_cu_count(), t1 = us_per_k1000 * K / 1000.0;
     const double groups = t1 * std::ceil(tiles / cus) * (1.0 + 0.3 / 4) + 3.0;
     double best = 0;
     *splits = 1;
-    for (int S = 1; S <= 32 && (S == 1 || K / S >= 256); ++S) {
+    // At most 32 MiB of partial sums: half the scratch of the no-allocation entry.
+    for (int S = 1; S <= 32 && (S == 1 || (K / S >= 256 && S * c_bytes <= (32u << 20))); ++S) {
         const double most = std::ceil(tiles * S / cus), o = std::min(most, 5.0);
         double t = t1 * most / S * (1.0 + 0.3 / o) * (1.0 + 64.0 * S / K);
         if (S > 1) t = t * (1.0 + 50.0 * S / K) + 5.0;
