@@ -16,6 +16,7 @@
 #include <type_traits>
 
 #include "internal.h"
+#include "conv_gather.h"
 #include "kernel_common.h"
 
 namespace ugemm {
@@ -69,9 +70,7 @@ struct Fp32Cfg {
 
 // One workgroup computes the C tile at (m0, n0) of g; shared by the plain and
 // the grouped (persistent) kernels. lds must hold CF::kLdsFloats floats.
-// CONV: opB is the implicit im2col matrix of cd (B and TB unused): every
-// thread keeps one column n of the B tile, so the pixel's origin is computed
-// once per tile and each element costs one table read and two compares.
+// CONV: opB is the implicit im2col matrix of cd (B and TB unused; ConvRegs).
 // epi: bias and activation after alpha/beta (Epilogue, internal.h).
 template <class CF, bool TA, bool TB, bool CONV = false>
 __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K, const float alpha,
@@ -104,22 +103,11 @@ __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K,
     const int ktiles = (K + BK - 1) / BK;
     const int kfull = K / BK;   // tiles with no K tail
 
-    // Implicit im2col: thread t always holds column nl = t % BN of the B
-    // tile (NT is a multiple of BN) and rows kl = t / BN + i * (NT / BN).
-    static_assert(!CONV || (NT % BN == 0 && BN % 64 == 0 && !TB), "implicit operand layout");
-    constexpr int CONV_N = CONV ? BK * BN / NT : 1;
-    float cvals[CONV_N];
-    long c_base = 0;
-    int c_h0 = 0, c_w0 = 0;
-    bool c_ncol = false;
-    if constexpr (CONV) {
-        const int n = n0 + t % BN;
-        c_ncol = n < N;
-        const int ho = c_ncol ? n / cd.wcol : 0, wo = c_ncol ? n - ho * cd.wcol : 0;
-        c_h0 = ho * cd.stride - cd.pad;
-        c_w0 = wo * cd.stride - cd.pad;
-        c_base = (long)c_h0 * cd.W + c_w0;
-    }
+    // Implicit im2col operand (columns past N and taps outside the image read zeros).
+    static_assert(!CONV || !TB, "implicit operand layout");
+    using CRegs = typename ConvRegsOf<CONV, BK, BN, NT>::type;
+    CRegs rc;
+    if constexpr (CONV) rc.init(cd, n0 + t % BN, N);
 
     // EDGE tiles reach past M, N or K.
     auto load_tile = [&](int kt, auto edge) {
@@ -134,21 +122,7 @@ __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K,
             ra.load_edge(a0, lda, t, TA ? mr : kr, TA ? kr : mr, wide_a);
             if constexpr (!CONV) rb.load_edge(b0, ldb, t, TB ? kr : nr, TB ? nr : kr, wide_b);
         }
-        if constexpr (CONV) {
-#pragma unroll
-            for (int i = 0; i < CONV_N; ++i) {
-                // k is the same for the 64 lanes of a wave (BN is a multiple
-                // of 64): one scalar load of the table entry per wave.
-                const int k = __builtin_amdgcn_readfirstlane(k0 + t / BN + i * (NT / BN));
-                float v = 0.0f;
-                if (c_ncol && k < K) {
-                    const int2 e = cd.ktab[k];
-                    const int hi = c_h0 + (e.y >> 16), wi = c_w0 + (e.y & 0xffff);
-                    if ((unsigned)hi < (unsigned)cd.H && (unsigned)wi < (unsigned)cd.W) v = cd.in[c_base + e.x];
-                }
-                cvals[i] = v;
-            }
-        }
+        if constexpr (CONV) rc.load(cd, k0, K, t);
     };
     auto store_tile = [&](int kt, int buf, auto edge) {
         if constexpr (decltype(edge)::value) {
@@ -158,8 +132,7 @@ __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K,
         }
         ra.template store<TA, LDA>(As + buf * BK * LDA, t);
         if constexpr (CONV) {
-#pragma unroll
-            for (int i = 0; i < CONV_N; ++i) Bs[buf * BK * LDB + (t / BN + i * (NT / BN)) * LDB + t % BN] = cvals[i];
+            rc.template store<LDB>(Bs + buf * BK * LDB, t);
         } else {
             rb.template store<!TB, LDB>(Bs + buf * BK * LDB, t);
         }
@@ -173,7 +146,7 @@ __device__ __forceinline__ void fp32_tile(const int M, const int N, const int K,
 
     // K tiles below nfast are loaded without bounds; the others (all of an
     // edge tile's, and a K remainder) as edges, in a loop of their own.
-    const int nfast = interior ? kfull : 0;
+    const int nfast = (CONV ? m0 + BM <= M : interior) ? kfull : 0;
     if (grp < nfast) {
         load_tile(grp, std::false_type());
         store_tile(grp, 0, std::false_type());

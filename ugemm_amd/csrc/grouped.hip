@@ -110,16 +110,10 @@ __device__ __forceinline__ void grouped_tile(const DevProblem &p, int m0, int n0
     }
 }
 
-template <class CF>
-constexpr int lds_floats() {
-    if constexpr (IsM32<CF>::value) return CF::kLdsFloats;
-    else return 2 * CF::BK * (CF::LDA + CF::LDB);
-}
-
 // Waves per SIMD the persistent kernel is compiled for (register budget).
 template <class CF>
 constexpr int grouped_waves() {
-    return IsM32<CF>::value ? 2 : 3;
+    return CF::KG > 1 ? CF::THREADS / 256 : IsM32<CF>::value ? 2 : 3;
 }
 
 // At least 3 waves per SIMD for the FP32 vector tiles (<= 168 VGPRs): the
@@ -129,11 +123,11 @@ constexpr int grouped_waves() {
 // CS: the tile of a mixed plan whose DevTile::shape is 1 (CF for shape 0);
 // the same as CF for a single-shape plan.  Both shapes have CF::NT threads.
 template <class CF, bool CONV, class CS = CF>
-__global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(grouped_waves<CF>()))) void grouped_fp32_kernel(
+__global__ __launch_bounds__(CF::THREADS) __attribute__((amdgpu_waves_per_eu(grouped_waves<CF>()))) void grouped_fp32_kernel(
     const DevProblem *__restrict__ probs, const DevTile *__restrict__ tiles, const int *__restrict__ q_begin,
     int *heads) {
-    static_assert(CS::NT == CF::NT, "the shapes of a mixed plan share the workgroup size");
-    constexpr int LDS_F = lds_floats<CF>() > lds_floats<CS>() ? lds_floats<CF>() : lds_floats<CS>();
+    static_assert(CS::THREADS == CF::THREADS, "the shapes of a mixed plan share the workgroup size");
+    constexpr int LDS_F = CF::kLdsFloats > CS::kLdsFloats ? CF::kLdsFloats : CS::kLdsFloats;
     __shared__ __attribute__((aligned(16))) float lds[LDS_F];
     __shared__ int s_tile;
     int q = blockIdx.x % kQueues;
@@ -144,7 +138,7 @@ __global__ __launch_bounds__(CF::NT) __attribute__((amdgpu_waves_per_eu(grouped_
             s_tile = i < size ? base + i : -1;
         }
         __syncthreads();
-        const int i = s_tile;
+        const int i = __builtin_amdgcn_readfirstlane(s_tile);   // uniform: the problem stays in scalar registers
         __syncthreads();   // every thread has read s_tile before it is written again
         if (i < 0) {
             q = (q + 1) % kQueues;
@@ -163,9 +157,11 @@ using G0 = Fp32Cfg<128, 128, 16, 8, 8>;
 using G1 = Fp32Cfg<64, 64, 16, 4, 4>;
 using G2 = Fp32Cfg<128, 64, 16, 8, 4>;
 using G3 = Fp32Cfg<64, 128, 16, 4, 8>;
-// Variant 4 ("mixed"): every problem gets the 128 x 128 tile (G0) or the
-// 64 x 128 tile (G3), whichever covers its rows with less padding (the
-// larger, more efficient tile when it pads at most 10% more).
+// Variant 1 of plans of few tiles: K dealt to the groups of a workgroup.
+using G1K4 = Fp32Cfg<64, 64, 16, 4, 4, 1, 4>;
+using G1K8 = Fp32Cfg<32, 64, 16, 4, 4, 1, 8>;
+// Variant 4 ("mixed"): 128 x 128 tiles (G0), and the 64 x 128 tile (G3) for a
+// problem's last rows where it covers them.
 constexpr int kNumVariants = 5, kMixed = 4;
 // The same five tile choices on the FP32 matrix cores (UGEMM_MODE_FP32_MFMA
 // plans), 4 waves each; variant 4 mixes GM0 and GM3 per problem.
@@ -173,10 +169,12 @@ using GM0 = M32Cfg<128, 128, 16, 2, 2>;
 using GM1 = M32Cfg<64, 64, 16, 2, 2>;
 using GM2 = M32Cfg<128, 64, 16, 2, 2>;
 using GM3 = M32Cfg<64, 128, 16, 2, 2>;
+using GM1K4 = M32Cfg<64, 64, 16, 2, 2, 1, 4>;
+using GM1K8 = M32Cfg<32, 64, 16, 1, 2, 1, 8>;
 
 struct VariantOps {
     int bm, bn, bk;          // shape 0
-    int bm1, bn1;            // shape 1 (mixed plans; equal to shape 0 otherwise)
+    int bm1, bn1;            // shape 1 (last rows of mixed plans; equal to shape 0 otherwise)
     const void *kern, *kern_conv;
     int nt;
 };
@@ -184,14 +182,15 @@ struct VariantOps {
 template <class CF, class CS = CF>
 VariantOps ops_of() {
     return VariantOps{CF::BM, CF::BN, CF::BK, CS::BM, CS::BN, (const void *)grouped_fp32_kernel<CF, false, CS>,
-                      (const void *)grouped_fp32_kernel<CF, true, CS>, CF::NT};
+                      (const void *)grouped_fp32_kernel<CF, true, CS>, CF::THREADS};
 }
 
-VariantOps variant_ops(int mode, int v) {
+// groups: of variant 1 (build_schedule).
+VariantOps variant_ops(int mode, int v, int groups) {
     if (mode == UGEMM_MODE_FP32_MFMA) {
         switch (v) {
             case 0: return ops_of<GM0>();
-            case 1: return ops_of<GM1>();
+            case 1: return groups == 8 ? ops_of<GM1K8>() : groups == 4 ? ops_of<GM1K4>() : ops_of<GM1>();
             case 2: return ops_of<GM2>();
             case 3: return ops_of<GM3>();
             default: return ops_of<GM0, GM3>();
@@ -199,7 +198,7 @@ VariantOps variant_ops(int mode, int v) {
     }
     switch (v) {
         case 0: return ops_of<G0>();
-        case 1: return ops_of<G1>();
+        case 1: return groups == 8 ? ops_of<G1K8>() : groups == 4 ? ops_of<G1K4>() : ops_of<G1>();
         case 2: return ops_of<G2>();
         case 3: return ops_of<G3>();
         default: return ops_of<G0, G3>();
@@ -210,13 +209,6 @@ const char *kGroupedNames[] = {"fp32_128x128x16_t8x8", "fp32_64x64x16_t4x4", "fp
                                "fp32_64x128x16_t4x8", "fp32_mixed_128x128_or_64x128_per_problem"};
 const char *kGroupedM32Names[] = {"f32_mfma_128x128x16_w2x2", "f32_mfma_64x64x16_w2x2", "f32_mfma_128x64x16_w2x2",
                                   "f32_mfma_64x128x16_w2x2", "f32_mfma_mixed_128x128_or_64x128_per_problem"};
-
-// Tile shape of problem rows M in a mixed plan: 0 (BM0 rows) unless its
-// padded rows exceed those of shape 1 (BM1 rows) by more than 10%.
-int mixed_shape(int M, int bm0, int bm1) {
-    const long r0 = (long)(M + bm0 - 1) / bm0 * bm0, r1 = (long)(M + bm1 - 1) / bm1 * bm1;
-    return (r0 * 10 <= r1 * 11) ? 0 : 1;
-}
 
 }  // namespace
 
@@ -237,6 +229,7 @@ struct ugemm_grouped_plan {
     double flops = 0;
     int mode = UGEMM_MODE_FP32;
     int variant = 0;
+    int groups = 1;   // of variant 1 (build_schedule)
     int grid = 0;
     int ntiles = 0;
     DevProblem *d_probs = nullptr;
@@ -245,7 +238,6 @@ struct ugemm_grouped_plan {
     int *d_heads = nullptr;    // kQueues queue heads (zeroed before every launch)
     bool capture = false;
     bool conv = false;          // a plan of convolutions (grouped_fp32_kernel<CF, true>)
-    int2 *d_ktab = nullptr;     // the convolutions' im2col offset tables, one block per problem
     // Split-form plans (BF16 forms): every problem's planes, prepared by one
     // job-table kernel, then one split-core block per tile.
     bool split = false;
@@ -306,7 +298,7 @@ int launch_plan_kernel(ugemm_grouped_plan *p, hipStream_t s) {
         return launch_mfma_grouped(p->mode, p->variant, p->b_kcont, p->d_jobs, p->d_block_job, p->prep_blocks,
                                    p->d_sprobs, p->d_stiles, p->ntiles, s, p->d_amax ? &sc : nullptr);
     }
-    const VariantOps ops = variant_ops(p->mode, p->variant);
+    const VariantOps ops = variant_ops(p->mode, p->variant, p->groups);
     hipLaunchKernelGGL(grouped_reset_heads, dim3(1), dim3(64), 0, s, p->d_heads);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "grouped queue reset");
@@ -325,7 +317,26 @@ int capture_plan(ugemm_grouped_plan *p);   // records the plan's launches in its
 int build_schedule(ugemm_grouped_plan *p, int v) {
     release_schedule(p);
     p->variant = v;
-    const VariantOps ops = variant_ops(p->mode, v);
+    // Variant 1: a plan of few tiles leaves CUs short of waves and then waits
+    // for its longest tile (288 K steps at K 4608); its K goes to 4 groups of a
+    // 64x64 tile or 8 of a 32x64 one.  us, one group / 4 / 8 by 64x64 tiles:
+    // 88 (convolutions, K to 4176) 440 / 185 / 129;  505 (K to 4464) 407 / 300 / 251;
+    // 930 (to 3213) 406 / 280 / 269;  1230 (convolutions, to 496) 160 / 109 / 143;
+    // 1777 (to 4203) 645 / 475 / 490;  2671 (convolutions, to 4608) 857 / 875 / 1142;
+    // 4310 (to 4446) 973 / 1035 / 1084.
+    p->groups = 1;
+    if (v == 1) {
+        long t64 = 0, t32 = 0;
+        int kmax = 0;
+        for (const DevProblem &q : p->probs) {
+            t64 += (long)((q.M + 63) / 64) * ((q.N + 63) / 64);
+            t32 += (long)((q.M + 31) / 32) * ((q.N + 63) / 64);
+            kmax = std::max(kmax, q.K);
+        }
+        const long cus = device_cu_count();
+        p->groups = t32 <= 4 * cus && kmax >= 1024 ? 8 : t64 <= 8 * cus ? 4 : 1;
+    }
+    const VariantOps ops = variant_ops(p->mode, v, p->groups);
     struct HostTile {
         DevTile t;
         long cost;
@@ -335,18 +346,23 @@ int build_schedule(ugemm_grouped_plan *p, int v) {
         const DevProblem &q = p->probs[i];
         if (q.M == 0 || q.N == 0) continue;
         if (q.K == 0 && q.beta == 1.0f) continue;   // nothing to do
-        // Shape of this problem's tiles; cost ~ k-steps x tile rows.
-        const int shape = (v == kMixed) ? mixed_shape(q.M, ops.bm, ops.bm1) : 0;
-        const int bm = shape ? ops.bm1 : ops.bm, bn = shape ? ops.bn1 : ops.bn;
-        const long cost = ((q.K + ops.bk - 1) / ops.bk + 2) * bm;
-        // Grouped order: GROUP_M tile-rows at a time, walked column by column.
+        // Row bands of the first shape's height; in a mixed plan the last band
+        // takes the second shape where that covers its rows.
+        const int tiles_n = (q.N + ops.bn - 1) / ops.bn;
+        struct Band {
+            int m0, shape;
+        };
+        std::vector<Band> bands;
+        for (int m0 = 0; m0 < q.M; m0 += ops.bm)
+            bands.push_back(Band{m0, v == kMixed && q.M - m0 <= ops.bm1 ? 1 : 0});
+        // Grouped order: GROUP_M bands at a time, walked column by column.
         constexpr int GROUP_M = 8;
-        const int tiles_m = (q.M + bm - 1) / bm, tiles_n = (q.N + bn - 1) / bn;
-        for (int g0 = 0; g0 < tiles_m; g0 += GROUP_M) {
-            const int g1 = std::min(tiles_m, g0 + GROUP_M);
+        for (size_t g0 = 0; g0 < bands.size(); g0 += GROUP_M) {
+            const size_t g1 = std::min(bands.size(), g0 + GROUP_M);
             for (int tn = 0; tn < tiles_n; ++tn)
-                for (int tm = g0; tm < g1; ++tm)
-                    tiles.push_back(HostTile{DevTile{i, tm * bm, tn * bn, shape}, cost});
+                for (size_t b = g0; b < g1; ++b)
+                    tiles.push_back(HostTile{DevTile{i, bands[b].m0, tn * ops.bn, bands[b].shape},
+                                             ((q.K + ops.bk - 1) / ops.bk + 2) * (long)(bands[b].shape ? ops.bm1 : ops.bm)});
         }
     }
     std::stable_sort(tiles.begin(), tiles.end(), [](const HostTile &a, const HostTile &b) { return a.cost > b.cost; });
@@ -613,15 +629,15 @@ bool parse_t(char c, bool *t) {
     return false;
 }
 
+// FP32 and FP32-MFMA plans: 64x64 tiles (variant 1, which deals K to groups
+// in small plans).  Large FP32 GEMM plans, where the drain of the last tiles no
+// longer shows, take the mixed 128x128 / 64x128 tiles: us on those against 64x64
+// by thousands of K columns of 64x64 tiles on a CU, 349: 8675 / 9025 (512 im2col
+// shapes), 86: 2434 / 2454, 34: 1251 / 1010.
 int default_variant(const ugemm_grouped_plan *p) {
-    // Most of the work in large-N problems: 128 x 128 tiles; otherwise 64 x 64.
-    double big = 0, all = 0;
-    for (const DevProblem &q : p->probs) {
-        const double f = 2.0 * q.M * q.N * q.K;
-        all += f;
-        if (q.M >= 128 && q.N >= 128) big += f;
-    }
-    return (all == 0 || big >= 0.5 * all) ? 0 : 1;
+    double work = 0;   // K columns of 64x64 tiles
+    for (const DevProblem &q : p->probs) work += (double)((q.M + 63) / 64) * ((q.N + 63) / 64) * q.K;
+    return p->mode == UGEMM_MODE_FP32 && !p->conv && work >= 80000.0 * device_cu_count() ? kMixed : 1;
 }
 
 // Uploads the problem table, picks the tile variant (forced, tuned, or by
@@ -724,7 +740,6 @@ int ugemm_hip_conv_grouped_plan_create_mode(ugemm_grouped_plan_t **plan, int cou
     int rc = ensure_device();
     if (rc) return rc;
     std::vector<int> hcol(count), wcol(count);
-    long ktab_total = 0;
     for (int i = 0; i < count; ++i) {
         const ugemm_conv_problem_t &c = convs[i];
         rc = conv_shape(c.ich, c.w, c.h, c.k, c.pad, c.stride, c.ch, &hcol[i], &wcol[i]);
@@ -732,29 +747,10 @@ int ugemm_hip_conv_grouped_plan_create_mode(ugemm_grouped_plan_t **plan, int cou
         if (!c.in || !c.weights || !c.out) return fail(UGEMM_ERR_ARG, "grouped conv: problem %d: NULL buffer", i);
         if (c.act != UGEMM_ACT_NONE && c.act != UGEMM_ACT_LEAKY_RELU)
             return fail(UGEMM_ERR_ARG, "grouped conv: problem %d: bad activation %d", i, c.act);
-        ktab_total += (long)c.ich * c.k * c.k;
-    }
-    // im2col offset tables: k = (ch*kh + i)*kw + j -> {ch*H*W + i*W + j, (i << 16) | j}.
-    std::vector<int2> ktab((size_t)std::max<long>(1, ktab_total));
-    std::vector<long> kofs(count);
-    long at = 0;
-    for (int i = 0; i < count; ++i) {
-        const ugemm_conv_problem_t &c = convs[i];
-        kofs[i] = at;
-        for (int q = 0; q < c.ich * c.k * c.k; ++q) {
-            const int ci = q / (c.k * c.k), r = q - ci * c.k * c.k, ki = r / c.k, kj = r - ki * c.k;
-            ktab[at++] = make_int2(ci * c.h * c.w + ki * c.w + kj, (ki << 16) | kj);
-        }
     }
     ugemm_grouped_plan *p = new ugemm_grouped_plan();
     p->mode = mode;
     p->conv = true;
-    hipError_t e;
-    if ((e = hipMalloc(&p->d_ktab, ktab.size() * sizeof(int2))) != hipSuccess ||
-        (e = hipMemcpy(p->d_ktab, ktab.data(), ktab.size() * sizeof(int2), hipMemcpyHostToDevice)) != hipSuccess) {
-        ugemm_hip_grouped_plan_destroy(p);
-        return hip_fail(e, "grouped conv: offset tables");
-    }
     for (int i = 0; i < count; ++i) {
         const ugemm_conv_problem_t &c = convs[i];
         const int K = c.ich * c.k * c.k, N = hcol[i] * wcol[i];
@@ -773,7 +769,7 @@ int ugemm_hip_conv_grouped_plan_create_mode(ugemm_grouped_plan_t **plan, int cou
         d.epi.bias_rows = 1;
         d.epi.act = c.act;
         d.epi.slope = c.slope;
-        d.cd = ConvDesc{c.in, p->d_ktab + kofs[i], c.h, c.w, wcol[i], c.stride, c.pad};
+        d.cd = conv_desc(c.in, nullptr, c.h, c.w, wcol[i], c.k, c.stride, c.pad);
         p->probs.push_back(d);
         p->flops += 2.0 * c.ch * N * K;
     }
@@ -796,7 +792,6 @@ void ugemm_hip_grouped_plan_destroy(ugemm_grouped_plan_t *p) {
     if (p->cap_stream) (void)hipStreamSynchronize(p->cap_stream);
     release_schedule(p);
     (void)hipFree(p->d_probs);
-    (void)hipFree(p->d_ktab);
     if (p->cap_stream) (void)hipStreamDestroy(p->cap_stream);
     delete p;
 }

@@ -28,12 +28,29 @@ __host__ __device__ inline float apply_epilogue(const Epilogue &e, float v, int 
 // never materialised): element (k, n) of the K x N matrix, K = ich*kh*kw,
 // N = hcol*wcol, is in[c*H*W + (ho*stride - pad + i)*W + (wo*stride - pad + j)]
 // for k = (c*kh + i)*kw + j, n = ho*wcol + wo, and 0 outside the image.
+// The FP32 tiles find c, i and j from k by multiplication (q = x / d is
+// (x * m) >> s for x < 2^31, conv_magic); the split forms' preparation reads
 // ktab[k] = {c*H*W + i*W + j, (i << 16) | j}, built on the device per call.
 struct ConvDesc {
     const float *in;
-    const int2 *ktab;
+    const int2 *ktab;              // split forms only
     int H, W, wcol, stride, pad;
+    int k, kk, k0;                 // taps per side, taps, first k of a split-K chunk
+    unsigned m_kk, m_k;
+    int s_kk, s_k;
 };
+inline void conv_magic(int d, unsigned *m, int *s) {
+    int l = 0;
+    while ((1LL << l) < d) ++l;    // 2^(l-1) < d <= 2^l: m * d - 2^(31+l) is in (0, 2^l]
+    *s = 31 + l;
+    *m = (unsigned)((1ULL << (31 + l)) / (unsigned)d + 1);
+}
+inline ConvDesc conv_desc(const float *in, const int2 *ktab, int H, int W, int wcol, int k, int stride, int pad) {
+    ConvDesc cd{in, ktab, H, W, wcol, stride, pad, k, k * k, 0, 0, 0, 0, 0};
+    conv_magic(cd.kk, &cd.m_kk, &cd.s_kk);
+    conv_magic(cd.k, &cd.m_k, &cd.s_k);
+    return cd;
+}
 
 // A problem of a grouped split-form plan: its prepared planes (blocked
 // layout, NP planes of Mp x Kp and Np x Kp) and C; and one C tile of it.

@@ -626,23 +626,26 @@ static int run_conv(const float *d_in, int ich, int w, int h, const float *d_wei
     if (mode == UGEMM_MODE_FP8_BLOCK) return fail(UGEMM_ERR_UNSUPPORTED, "conv: the FP8 form is not provided");
     if (!d_in || !d_weights || !d_out) return fail(UGEMM_ERR_ARG, "conv: NULL buffer");
     const int K = ich * k * k;
+    Gemm<float> g{ch, hcol * wcol, K, 1.0f, 0.0f, d_weights, K, nullptr, 0, d_out, (long)hcol * wcol, false, false};
+    g.epi = epi;
+    const int v = forced_variant(mode);
+    if (k == 1 && stride == 1 && pad == 0) {
+        // The column matrix is the image itself: a plain GEMM.
+        g.B = d_in;
+        g.ldb = (long)h * w;
+        return run_sgemm(g, mode, v, s);
+    }
+    g.splits = forced_splits(mode);
+    ConvDesc cd = conv_desc(d_in, nullptr, h, w, wcol, k, stride, pad);
+    if (mode == UGEMM_MODE_FP32) return launch_conv_fp32(g, cd, v, s);
+    if (mode == UGEMM_MODE_FP32_MFMA) return launch_conv_m32(g, cd, v, s);
     void *ws = nullptr;
     rc = stream_alloc(&ws, (size_t)K * sizeof(int2), s);
     if (rc) return rc;
-    int2 *ktab = (int2 *)ws;
-    hipLaunchKernelGGL(conv_ktab_kernel, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, s, ktab, K, k, h, w);
+    cd.ktab = (int2 *)ws;
+    hipLaunchKernelGGL(conv_ktab_kernel, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, s, (int2 *)ws, K, k, h, w);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) rc = hip_fail(e, "conv: offset table");
-    if (!rc) {
-        Gemm<float> g{ch, hcol * wcol, K, 1.0f, 0.0f, d_weights, K, nullptr, 0, d_out, (long)hcol * wcol, false, false};
-        g.epi = epi;
-        g.splits = forced_splits(mode);
-        const ConvDesc cd{d_in, ktab, h, w, wcol, stride, pad};
-        const int v = forced_variant(mode);
-        rc = mode == UGEMM_MODE_FP32        ? launch_conv_fp32(g, cd, v, s)
-             : mode == UGEMM_MODE_FP32_MFMA ? launch_conv_m32(g, cd, v, s)
-                                            : launch_mfma_conv(g, cd, mode, v, s);
-    }
+    rc = e == hipSuccess ? launch_mfma_conv(g, cd, mode, v, s) : hip_fail(e, "conv: offset table");
     const int rc2 = stream_free(ws, s);
     return rc ? rc : rc2;
 }

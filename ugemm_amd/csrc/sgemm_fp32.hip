@@ -34,7 +34,7 @@ __global__ __launch_bounds__(CF::THREADS, CF::MINB) void sgemm_fp32_kernel(int M
 // Split-K as in sgemm_fp32_kernel: the chunk's rows of the offset table
 // (absolute image offsets) and its weight columns.
 template <class CF>
-__global__ __launch_bounds__(CF::NT) void conv_fp32_kernel(int M, int N, int K, float alpha,
+__global__ __launch_bounds__(CF::THREADS) void conv_fp32_kernel(int M, int N, int K, float alpha,
                                                            const float *__restrict__ A, long lda, float beta,
                                                            float *__restrict__ C, long ldc, int tiles_m, int tiles_n,
                                                            Epilogue epi, ConvDesc cd, int kc, float *__restrict__ ws) {
@@ -44,7 +44,7 @@ __global__ __launch_bounds__(CF::NT) void conv_fp32_kernel(int M, int N, int K, 
     const bool part = gridDim.y > 1;
     const int k0 = part ? (int)blockIdx.y * kc : 0;
     ConvDesc cz = cd;
-    cz.ktab = cd.ktab + k0;
+    cz.k0 = k0;
     fp32_tile<CF, false, false, true>(M, N, part ? min(kc, K - k0) : K, part ? 1.0f : alpha, A + k0, lda, nullptr, 0,
                                       part ? 0.0f : beta, part ? ws + (long)blockIdx.y * M * N : C,
                                       part ? (long)N : ldc, tm * CF::BM, tn * CF::BN, lds, part ? Epilogue() : epi, cz);
@@ -63,6 +63,7 @@ using V5 = Fp32Cfg<128, 256, 16, 8, 16, 2>;
 using V1K4 = Fp32Cfg<64, 64, 16, 4, 4, 1, 4>;
 using V1S8 = Fp32Cfg<32, 32, 16, 4, 4, 1, 8>;
 using V1S16 = Fp32Cfg<32, 32, 16, 4, 4, 1, 16>;
+using V1C8 = Fp32Cfg<32, 64, 16, 4, 4, 1, 8>;   // convolutions
 
 const char *kNames[] = {"fp32_128x128x16_t8x8", "fp32_64x64x16_t4x4", "fp32_128x64x16_t8x4",
                         "fp32_64x128x16_t4x8", "fp32_256x128x16_t16x8", "fp32_128x256x16_t8x16"};
@@ -140,7 +141,7 @@ int launch_conv_cfg(const Gemm<float> &g, const ConvDesc &cd, hipStream_t s) {
         const int rc = stream_alloc((void **)&ws, (size_t)splits * g.M * g.N * sizeof(float), s);
         if (rc) return rc;
     }
-    dim3 grid((unsigned)nblk, (unsigned)splits), block(CF::NT);
+    dim3 grid((unsigned)nblk, (unsigned)splits), block(CF::THREADS);
     timing_begin(s);
     hipLaunchKernelGGL((conv_fp32_kernel<CF>), grid, block, 0, s, g.M, g.N, g.K, g.alpha, g.A, g.lda, g.beta, g.C,
                        g.ldc, tiles_m, tiles_n, g.epi, cd, kc, ws);
@@ -153,6 +154,22 @@ int launch_conv_cfg(const Gemm<float> &g, const ConvDesc &cd, hipStream_t s) {
         if (!rc) rc = rc2;
     }
     return rc;
+}
+
+// Variant 1 with the automatic split count, as launch_small: 8 groups of 32x64
+// tiles for the smallest grids, else as deal_k has it.
+int launch_conv_small(const Gemm<float> &g, const ConvDesc &cd, hipStream_t s) {
+    const long cus = device_cu_count();
+    const long t32 = (long)((g.M + 31) / 32) * ((g.N + 63) / 64), t64 = (long)((g.M + 63) / 64) * ((g.N + 63) / 64);
+    if (g.splits != 0 || t64 > 4 * cus) return launch_conv_cfg<V1>(g, cd, s);
+    Gemm<float> h = g;
+    h.splits = 1;
+    if (t32 <= cus && t32 * g.K <= cus * 2048) {
+        if (g.K > 768) h.splits = (int)std::max(1L, std::min({cus / t32, g.K / 256L, 16L}));
+        return launch_conv_cfg<V1C8>(h, cd, s);
+    }
+    return deal_k(t64, g.K, 40.0, 2, sizeof(*g.C) * g.M * g.N, &h.splits) ? (h.splits = 1, launch_conv_cfg<V1K4>(h, cd, s))
+                                                                        : launch_conv_cfg<V1>(h, cd, s);
 }
 
 }  // namespace
@@ -188,12 +205,13 @@ int fp32_pick_variant(const Gemm<float> &g) {
 }
 
 int launch_conv_fp32(const Gemm<float> &g, const ConvDesc &cd, int variant, hipStream_t s) {
-    // Convolutions are compiled for the four 8x8-or-smaller tiles.
-    if (variant < 0) variant = fp32_pick_variant(g);
+    // Convolutions are compiled for the four 8x8-or-smaller tiles; 64x64 is the
+    // fastest of them at every size tried (the gather, not the FMAs, sets the pace).
+    if (variant < 0) variant = 1;
     if (variant >= 4) variant = 0;
     switch (variant) {
         case 0: return launch_conv_cfg<V0>(g, cd, s);
-        case 1: return launch_conv_cfg<V1>(g, cd, s);
+        case 1: return launch_conv_small(g, cd, s);
         case 2: return launch_conv_cfg<V2>(g, cd, s);
         case 3: return launch_conv_cfg<V3>(g, cd, s);
         default: return fail(UGEMM_ERR_ARG, "conv: no variant %d", variant);

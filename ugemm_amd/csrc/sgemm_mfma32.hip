@@ -45,17 +45,16 @@ __global__ __launch_bounds__(CF::THREADS, CF::MINB) void sgemm_mfma32_kernel(
 // (ConvDesc).  Split-K: the chunk's rows of the offset table and its weight
 // columns, as in the GEMM kernel.
 template <class CF>
-__global__ __launch_bounds__(CF::NT, CF::MINB) void conv_mfma32_kernel(
+__global__ __launch_bounds__(CF::THREADS, CF::MINB) void conv_mfma32_kernel(
     int M, int N, int K_, const float *__restrict__ A_, long lda, float *__restrict__ C_, long ldc_, int tiles_m,
     int tiles_n, Epilogue epi, ConvDesc cd, int kc, float *__restrict__ ws) {
-    constexpr int kLds = 2 * (CF::template stage<true, CF::BM>() + CF::template stage<false, CF::BN>());
-    __shared__ __attribute__((aligned(16))) float lds[kLds];
+    __shared__ __attribute__((aligned(16))) float lds[CF::template lds_floats<false, false>()];
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
     const bool part = gridDim.y > 1;
     const int k0 = part ? (int)blockIdx.y * kc : 0;
     ConvDesc cz = cd;
-    cz.ktab = cd.ktab + k0;
+    cz.k0 = k0;
     m32_tile<CF, false, false, true>(M, N, part ? min(kc, K_ - k0) : K_, 1.0f, A_ + k0, lda, nullptr, 0, 0.0f,
                                      part ? ws + (long)blockIdx.y * M * N : C_, part ? (long)N : ldc_, tm * CF::BM,
                                      tn * CF::BN, lds, part ? Epilogue() : epi, cz);
@@ -71,6 +70,7 @@ using V5 = M32Cfg<128, 128, 32, 2, 2, 2>;
 using V3K4 = M32Cfg<64, 64, 16, 2, 2, 1, 4>;
 using V3S8 = M32Cfg<32, 32, 16, 1, 1, 1, 8>;
 using V3S16 = M32Cfg<32, 32, 16, 1, 1, 1, 16>;
+using V3C8 = M32Cfg<32, 64, 16, 1, 2, 1, 8>;   // convolutions
 
 const char *kNames[] = {"f32_mfma_128x128x16_w2x2", "f32_mfma_256x128x16_w4x2", "f32_mfma_128x256x16_w2x4",
                         "f32_mfma_64x64x16_w2x2",   "f32_mfma_256x256x16_w2x4", "f32_mfma_128x128x32_w2x2"};
@@ -141,7 +141,7 @@ int launch_conv_cfg(const Gemm<float> &g, const ConvDesc &cd, hipStream_t s) {
         if (rc) return rc;
     }
     timing_begin(s);
-    hipLaunchKernelGGL((conv_mfma32_kernel<CF>), dim3((unsigned)nblk, (unsigned)splits), dim3(CF::NT), 0, s, g.M,
+    hipLaunchKernelGGL((conv_mfma32_kernel<CF>), dim3((unsigned)nblk, (unsigned)splits), dim3(CF::THREADS), 0, s, g.M,
                        g.N, g.K, g.A, g.lda, g.C, g.ldc, tiles_m, tiles_n, g.epi, cd, kc, ws);
     timing_end(s);
     hipError_t e = hipGetLastError();
@@ -152,6 +152,21 @@ int launch_conv_cfg(const Gemm<float> &g, const ConvDesc &cd, hipStream_t s) {
         if (!rc) rc = rc2;
     }
     return rc;
+}
+
+// Variant 3 with the automatic split count, as the FP32 kernel's.
+int launch_conv_small(const Gemm<float> &g, const ConvDesc &cd, hipStream_t s) {
+    const long cus = device_cu_count();
+    const long t32 = (long)((g.M + 31) / 32) * ((g.N + 63) / 64), t64 = (long)((g.M + 63) / 64) * ((g.N + 63) / 64);
+    if (g.splits != 0 || t64 > 4 * cus) return launch_conv_cfg<V3>(g, cd, s);
+    Gemm<float> h = g;
+    h.splits = 1;
+    if (t32 <= cus && t32 * g.K <= cus * 2048) {
+        if (g.K > 768) h.splits = (int)std::max(1L, std::min({cus / t32, g.K / 256L, 16L}));
+        return launch_conv_cfg<V3C8>(h, cd, s);
+    }
+    return deal_k(t64, g.K, 40.0, 2, sizeof(*g.C) * g.M * g.N, &h.splits) ? (h.splits = 1, launch_conv_cfg<V3K4>(h, cd, s))
+                                                                        : launch_conv_cfg<V3>(h, cd, s);
 }
 
 }  // namespace
@@ -173,12 +188,12 @@ int m32_pick_variant(const Gemm<float> &g) {
 
 // g: the convolution as a GEMM (alpha 1, beta 0, A the weights, B unused).
 int launch_conv_m32(const Gemm<float> &g, const ConvDesc &cd, int variant, hipStream_t s) {
-    if (variant < 0) variant = m32_pick_variant(g);
+    if (variant < 0) variant = 3;   // the fastest at every size tried: the gather sets the pace
     switch (variant) {
         case 0: return launch_conv_cfg<V0>(g, cd, s);
         case 1: return launch_conv_cfg<V1>(g, cd, s);
         case 2: return launch_conv_cfg<V2>(g, cd, s);
-        case 3: return launch_conv_cfg<V3>(g, cd, s);
+        case 3: return launch_conv_small(g, cd, s);
         case 4: return launch_conv_cfg<V4>(g, cd, s);
         case 5: return launch_conv_cfg<V5>(g, cd, s);
         default: return fail(UGEMM_ERR_ARG, "conv fp32 mfma: no variant %d", variant);
