@@ -147,6 +147,11 @@ int m32_pick_variant(const Gemm<float> &g);
 int launch_m32(const Gemm<float> &g, int variant, hipStream_t s);
 int launch_conv_m32(const Gemm<float> &g, const ConvDesc &cd, int variant, hipStream_t s);
 
+// Split forms in one launch (split_small.hip): the tile (32 or 64) that suits
+// the automatic choice for g, or 0 where the plane-streaming path is better.
+int split_small_tile(const Gemm<float> &g, int mode);
+int launch_split_small(const Gemm<float> &g, int mode, int tile, hipStream_t s);
+
 int mfma_variant_count(int mode);
 const char *mfma_variant_name(int mode, int v);
 int mfma_pick_variant(const Gemm<float> &g, int mode);

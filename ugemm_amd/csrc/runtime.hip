@@ -398,7 +398,9 @@ static int choose_variant(const Gemm<float> &g, int mode, int *splits) {
         case UGEMM_MODE_FP32: return fp32_pick_variant(g);
         case UGEMM_MODE_FP32_MFMA: return m32_pick_variant(g);
         case UGEMM_MODE_FP8_BLOCK: return -1;   // launch_fp8 picks by grid size
-        default: return mfma_pick_variant(g, mode);
+        default:
+            // Small grids in one launch: variant 3's automatic choice.
+            return *splits == 0 && split_small_tile(g, mode) ? 3 : mfma_pick_variant(g, mode);
     }
 }
 
