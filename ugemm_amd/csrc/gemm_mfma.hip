@@ -1545,27 +1545,135 @@ const char *mfma_variant_name(int mode, int v) {
     }
 }
 
-int mfma_pick_variant(const Gemm<float> &g, int mode) {
+// The estimate behind the choice on grids of fewer than one 256-row tile a CU,
+// in us, fitted to splits 1-16 of variants 3, 7 and the large tile over 31
+// shapes (sides 33..15277, K 186..42112; rms 7-11% a form).  The CU with the
+// most blocks sets the time: `most` blocks of `us` per 1000 of K, of which
+// latency stretches few (`lat`; up to `occ` share a CU), and `block` each for
+// the first loads and the epilogue.  Partial sums cost a second launch and
+// their bytes, the preparation its bytes (FP16X3 reads an operand twice, once
+// for the row maxima), and an operand that the core splits spares it that for
+// `fused` times the core.  A copy moves 4.8 bytes a ps.
+namespace {
+struct PickTile {
+    int variant, bm, bn;
+    double us, lat, occ, block;
+};
+struct PickForm {
+    PickTile tile[3];
+    double prep, fused;
+};
+const PickForm &pick_form(int np) {
+    static const PickForm forms[3] = {
+        {{{3, 64, 64, 1.5, 6.0, 4, 0.4}, {7, 128, 128, 8.0, 0.3, 2, 2.0}, {5, 256, 256, 22, 0.1, 1, 12}}, 1.5, 1.9},
+        {{{3, 64, 64, 4.4, 1.9, 4, 0.4}, {7, 128, 128, 13.5, 0.3, 2, 2.0}, {6, 256, 256, 43, 0.1, 1, 15}}, 1.8, 1.5},
+        {{{3, 64, 64, 8.7, 0.9, 4, 1.2}, {7, 128, 128, 28.0, 0.1, 2, 3.0}, {6, 256, 128, 49, 0.1, 1, 8}}, 2.5, 1.3}};
+    return forms[np - 1];
+}
+
+// The operand (at most one) that the core splits itself: run_cfg's rule.
+void fused_operand(const Gemm<float> &g, int variant, long tm, long tn, bool *fa, bool *fb) {
+    const bool eight = variant == 4 || variant == 6 || variant == 7;
+    *fa = eight && tn <= 2;
+    *fb = eight && tm <= 2;
+    if (*fa && *fb) (g.M >= g.N ? *fb : *fa) = false;
+}
+
+// Microseconds of g on tile t with S splits; *ws receives the workspace bytes.
+double pick_cost(const Gemm<float> &g, int np, bool scaled, bool fusable, const PickForm &f, const PickTile &t, int S,
+                 size_t *ws) {
+    const double cus = (double)device_cu_count(), per_us = 4.8e6;
+    const long tm = (g.M + t.bm - 1) / t.bm, tn = (g.N + t.bn - 1) / t.bn, kc = ((g.K + S - 1) / S + 31) / 32 * 32;
+    bool fa = false, fb = false;
+    if (fusable) fused_operand(g, t.variant, tm, tn, &fa, &fb);
+    const long ra = tm * t.bm, rb = tn * t.bn;
+    const double left = scaled ? 0.5 : 0.0;   // of a fused operand's preparation: its row maxima
+    const double prep = ((fa ? left : 1.0) * ra + (fb ? left : 1.0) * rb) * g.K;
+    // Two rows a thread of a row-contiguous operand (256-row tiles) are loaded
+    // together: at an odd pitch, off their alignment, the core took 1.5-1.9 times as long.
+    const bool off = t.bm == 256 && ((fa && g.ta && (g.lda & 1)) || (fb && !g.tb && (g.ldb & 1)));
+    const double most = std::ceil(tm * tn * S / cus);
+    double us = t.us * (fa || fb ? f.fused : 1.0) * (off ? 1.8 : 1.0) * kc / 1000.0 * (1.0 + t.lat / std::min(most, t.occ));
+    us = (us + t.block) * most + (scaled ? 2.5 : f.prep) * prep * 4 / per_us;
+    const double sums = S > 1 ? 4.0 * S * g.M * g.N : 0.0;
+    if (S > 1) us += 2.5 + 0.9 * sums / per_us;
+    *ws = ((fa ? 0 : ra) + (fb ? 0 : rb)) * (size_t)round_up(g.K, 64) * 2 * np + (scaled ? (ra + rb) * 4 : 0) + 512 +
+          (size_t)sums;
+    return us;
+}
+
+// What the choice by the grid alone (mfma_fixed_variant) takes: its split count and workspace.
+double fixed_cost(const Gemm<float> &g, int np, bool scaled, bool fusable, const PickForm &f, int fixed, size_t *ws) {
+    for (const PickTile &t : f.tile) {
+        if (t.variant != fixed) continue;
+        int kc;
+        const long tiles = (long)((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn);
+        const int S = split_count(0, tiles, (int)round_up(g.K, 64), 32, &kc, fixed == 3 ? 2 : 1);
+        return pick_cost(g, np, scaled, fusable, f, t, S, ws);
+    }
+    *ws = 0;
+    return 0;
+}
+
+// Grids of fewer 256-row tiles than CUs, without a split count.  128 x 128
+// tiles: the 8-wave streamed V7 (2048^3: 12-24% faster per call than the
+// 4-wave V1, whose one wave per SIMD hides no latency).
+int mfma_fixed_variant(const Gemm<float> &g) {
+    return (long)((g.M + 127) / 128) * ((g.N + 127) / 128) >= device_cu_count() / 2 ? 7 : 3;
+}
+}  // namespace
+
+bool mfma_planes_fit_scratch(const Gemm<float> &g, int mode) {
+    const int np = planes_of(mode);
+    for (const int v : {3, mfma_fixed_variant(g)}) {
+        size_t ws;
+        fixed_cost(g, np, mode == UGEMM_MODE_FP16X3, true, pick_form(np), v, &ws);
+        if (ws <= UGEMM_HIP_NOALLOC_SCRATCH_BYTES) return true;
+    }
+    return false;
+}
+
+int mfma_pick_variant(const Gemm<float> &g, int mode, bool fusable, int *splits) {
     const long cus = device_cu_count();
     const int np = planes_of(mode);
     // Largest tile whose grid still gives every CU work; there, the
     // multi-wave variant measured fastest for the form.
     const long big_m = 256, big_n = (np == 3) ? 128 : 256;
-    const long tiles_big = ((g.M + big_m - 1) / big_m) * ((g.N + big_n - 1) / big_n);
-    if (tiles_big >= cus) {
-        // A skinny side whose operand (either layout) the 8-wave variant
-        // splits in the core (no preparation pass): V4.  Otherwise two and
-        // three planes run fastest on the streamed V6, one plane on the
-        // 16-wave V5.
-        const long tm = (g.M + big_m - 1) / big_m, tn = (g.N + big_n - 1) / big_n;
-        const bool fuse = np <= 2 && (tn <= 2 || tm <= 2);
-        return fuse ? 4 : (np >= 2 ? 6 : 5);
+    const long tm = (g.M + big_m - 1) / big_m, tn = (g.N + big_n - 1) / big_n;
+    // A skinny side whose operand (either layout) the 8-wave variant
+    // splits in the core (no preparation pass): V4.  Otherwise two and
+    // three planes run fastest on the streamed V6, one plane on the
+    // 16-wave V5.
+    const int big = fusable && np <= 2 && (tn <= 2 || tm <= 2) ? 4 : (np >= 2 ? 6 : 5);
+    if (tm * tn >= cus) return big;
+    const int fixed = mfma_fixed_variant(g);
+    if (*splits > 0 || g.K <= 0) return fixed;
+    // Fewer: tile and splits together.  493x2304x34854 BF16X3 ran 288 blocks
+    // of V3 in 877 us, one wave a SIMD and two blocks on a few CUs; V6 in 12
+    // splits takes 285.  1024x1024x4096 54 and 47 (V7 in 4), 64x6272x6592 91
+    // and 53 (V7 in 8, which splits B in the core), 5120x111x6405 93 and 48.
+    // Near ties stay with the fixed choice and its own split count.  What that
+    // runs within the scratch of the no-allocation entry stays within it, and
+    // there the calls that it refuses stay refused: one choice for both entries.
+    const bool scaled = mode == UGEMM_MODE_FP16X3;
+    const PickForm &f = pick_form(np);
+    size_t ws, fixed_ws;
+    double best = 0.92 * fixed_cost(g, np, scaled, fusable, f, fixed, &fixed_ws);
+    const bool fits = fixed_ws <= UGEMM_HIP_NOALLOC_SCRATCH_BYTES;
+    if (!fits && stream_alloc_is_static()) return fixed;
+    int v = fixed;
+    for (PickTile t : f.tile) {
+        if (t.bm == 256) t.variant = big;
+        for (int S = 1; S <= 16 && (S == 1 || (g.K / S >= 256 && (size_t)S * g.M * g.N * 4 <= (64u << 20))); ++S) {
+            const double c = pick_cost(g, np, scaled, fusable, f, t, S, &ws);
+            if (c < best && (!fits || ws <= UGEMM_HIP_NOALLOC_SCRATCH_BYTES)) {
+                best = c;
+                v = t.variant;
+                *splits = S;
+            }
+        }
     }
-    // 128 x 128 tiles: the 8-wave streamed V7 (2048^3: 12-24% faster per
-    // call than the 4-wave V1, whose one wave per SIMD hides no latency).
-    const long t128 = (long)((g.M + 127) / 128) * ((g.N + 127) / 128);
-    if (t128 >= cus / 2) return 7;
-    return 3;
+    return v;
 }
 
 // ---------------------------------------------------------------------------
@@ -1716,13 +1824,13 @@ int launch_mfma_conv(const Gemm<float> &g, const ConvDesc &cd, int mode, int var
     // No operand is split in the core here (the im2col operand is gathered
     // into planes), so the picker's fusing variant gives way to the
     // plane-streaming one.
-    int v = variant >= 0 ? variant : mfma_pick_variant(g, mode);
-    if (variant < 0 && v == 4) v = planes_of(mode) == 2 ? 6 : 5;
+    Gemm<float> gs = g;
+    const int v = variant >= 0 ? variant : mfma_pick_variant(g, mode, false, &gs.splits);
     switch (mode) {
-        case UGEMM_MODE_BF16X1: return launch_np_conv<1>(g, cd, v, s);
-        case UGEMM_MODE_BF16X3: return launch_np_conv<2>(g, cd, v, s);
-        case UGEMM_MODE_BF16X6: return launch_np_conv<3>(g, cd, v, s);
-        case UGEMM_MODE_FP16X3: return launch_np_conv<2, FmtF16>(g, cd, v, s);
+        case UGEMM_MODE_BF16X1: return launch_np_conv<1>(gs, cd, v, s);
+        case UGEMM_MODE_BF16X3: return launch_np_conv<2>(gs, cd, v, s);
+        case UGEMM_MODE_BF16X6: return launch_np_conv<3>(gs, cd, v, s);
+        case UGEMM_MODE_FP16X3: return launch_np_conv<2, FmtF16>(gs, cd, v, s);
         default: return fail(UGEMM_ERR_UNSUPPORTED, "conv: mode %d is not provided", mode);
     }
 }

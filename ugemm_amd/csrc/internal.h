@@ -154,7 +154,11 @@ int launch_split_small(const Gemm<float> &g, int mode, int tile, hipStream_t s);
 
 int mfma_variant_count(int mode);
 const char *mfma_variant_name(int mode, int v);
-int mfma_pick_variant(const Gemm<float> &g, int mode);
+// The automatic variant; with *splits == 0 also the split count to run it with
+// (0 left: that variant's own rule).  fusable: the core may split an operand.
+int mfma_pick_variant(const Gemm<float> &g, int mode, bool fusable, int *splits);
+// The planes of variant 3, or of the choice by the grid alone, fit the static scratch.
+bool mfma_planes_fit_scratch(const Gemm<float> &g, int mode);
 int launch_mfma(const Gemm<float> &g, int mode, int variant, hipStream_t s);
 // Grouped split-form plans: tile shape of a variant, and the launch of
 // the preparation (jobs) then the core (one block per tile).
@@ -269,6 +273,8 @@ void release_staging();
 // Stream-ordered workspace for the operand-preparation kernels: allocated
 // from the device's default memory pool on stream s (which keeps freed
 // blocks for reuse), released in stream order after the consuming kernel.
+// This thread is in a no-allocation call: stream_alloc gives from the static scratch.
+bool stream_alloc_is_static();
 int stream_alloc(void **ptr, size_t bytes, hipStream_t s);
 int stream_free(void *ptr, hipStream_t s);
 

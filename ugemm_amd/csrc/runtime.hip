@@ -203,6 +203,8 @@ static void ws_release_all() {
         if (b.p && !b.busy) ws_drop(b);
 }
 
+bool stream_alloc_is_static() { return t_arena != nullptr; }
+
 int stream_alloc(void **ptr, size_t bytes, hipStream_t s) {
     *ptr = nullptr;
     if (bytes == 0) return UGEMM_OK;
@@ -400,7 +402,7 @@ static int choose_variant(const Gemm<float> &g, int mode, int *splits) {
         case UGEMM_MODE_FP8_BLOCK: return -1;   // launch_fp8 picks by grid size
         default:
             // Small grids in one launch: variant 3's automatic choice.
-            return *splits == 0 && split_small_tile(g, mode) ? 3 : mfma_pick_variant(g, mode);
+            return *splits == 0 && split_small_tile(g, mode) ? 3 : mfma_pick_variant(g, mode, true, splits);
     }
 }
 

@@ -226,8 +226,10 @@ int launch_np(const Gemm<float> &g, int tile, hipStream_t s) {
 //   1615x2637x35 TN (1092 of 64x64) 37.2 / 71 / 31.9;  15.9 / 36.8 / 25.7
 // So 32x32 tiles up to two workgroups a CU while the scan of K is short, 64x64
 // up to one; FP16X3, whose planes cost three more launches, further where K
-// is short.
+// is short.  A no-allocation call whose planes exceed the static scratch keeps
+// the planes, and is refused as ever.
 int split_small_tile(const Gemm<float> &g, int mode) {
+    if (stream_alloc_is_static() && !mfma_planes_fit_scratch(g, mode)) return 0;
     const bool scaled = mode == UGEMM_MODE_FP16X3;
     const long cus = device_cu_count();
     const long t32 = (long)((g.M + 31) / 32) * ((g.N + 31) / 32), t64 = (long)((g.M + 63) / 64) * ((g.N + 63) / 64);
