@@ -49,17 +49,14 @@
 namespace ugemm {
 namespace {
 
+// row_inf (scaled formats): the row's largest magnitude is infinite.
 template <int NP, class FMT>
-__device__ __forceinline__ void write_planes(typename FMT::E *dst, long plane_stride, const float (&x)[8]) {
-    typename FMT::E o[NP][8];
-    split_vec<NP, 8>(x, o);
+__device__ __forceinline__ void write_planes(typename FMT::E *dst, long plane_stride, const float (&x)[8],
+                                             bool row_inf = false) {
+    typename FMT::V8 w[NP];
+    split8<NP, FMT>(x, __any(split_special(FMT(), x, row_inf)), w);
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
-        typename FMT::V8 w;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) w[j] = o[p][j];
-        *reinterpret_cast<typename FMT::V8 *>(dst + p * plane_stride) = w;
-    }
+    for (int p = 0; p < NP; ++p) *reinterpret_cast<typename FMT::V8 *>(dst + p * plane_stride) = w[p];
 }
 
 // Plane layout written by the preparation kernels ("k-tile blocked"): plane
@@ -93,12 +90,14 @@ __device__ __forceinline__ void prep_kcont_chunk(const float *__restrict__ X, lo
 #pragma unroll
         for (int j = 0; j < 8; ++j) x[j] = (r < rows && k + j < K) ? p[j] : 0.0f;
     }
+    bool inf = false;
     if constexpr (FMT::SCALED) {
         const int e = -row_exp(amax[r]);
+        inf = row_is_inf(amax[r]);
 #pragma unroll
         for (int j = 0; j < 8; ++j) x[j] = ldexpf(x[j], e);
     }
-    write_planes<NP, FMT>(out + blocked_offset(r, k, rows_pad), plane_stride, x);
+    write_planes<NP, FMT>(out + blocked_offset(r, k, rows_pad), plane_stride, x, inf);
 }
 
 template <int NP, class FMT>
@@ -153,7 +152,7 @@ __device__ __forceinline__ void prep_kcont_tile(const float *__restrict__ X, lon
 #pragma unroll
             for (int j = 0; j < 8; ++j) x[i][j] = ldexpf(x[i][j], e);
         }
-        write_planes<NP, FMT>(out + blocked_offset(r, k, rows_pad), plane_stride, x[i]);
+        write_planes<NP, FMT>(out + blocked_offset(r, k, rows_pad), plane_stride, x[i], row_is_inf(am[i]));
     }
 }
 
@@ -224,7 +223,8 @@ __device__ __forceinline__ void prep_kcont_rowscaled_pair(const float *__restric
         if (kt >= ktiles) break;
 #pragma unroll
         for (int j = 0; j < 8; ++j) x[i][j] = ldexpf(x[i][j], e);
-        write_planes<NP, FMT>(out + blocked_offset(r, kt * 32 + cc * 8, rows_pad), plane_stride, x[i]);
+        write_planes<NP, FMT>(out + blocked_offset(r, kt * 32 + cc * 8, rows_pad), plane_stride, x[i],
+                              row_is_inf(bits));
     }
 }
 
@@ -287,7 +287,7 @@ __device__ __forceinline__ void prep_rcont_tile(const float *__restrict__ X, lon
 #pragma unroll
             for (int j = 0; j < 8; ++j) x[j] = ldexpf(x[j], e);
         }
-        write_planes<NP, FMT>(out + blocked_offset(r, k, rows_pad), plane_stride, x);
+        write_planes<NP, FMT>(out + blocked_offset(r, k, rows_pad), plane_stride, x, row_is_inf(am[i]));
     }
 }
 
@@ -515,12 +515,14 @@ __global__ __launch_bounds__(256) void split_prep_im2col(ConvDesc cd, int N, int
         float x[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) x[j] = im2col_at(cd, r, k + j, N, K);
+        bool inf = false;
         if constexpr (FMT::SCALED) {
             const int e = -row_exp(amax[r]);
+            inf = row_is_inf(amax[r]);
 #pragma unroll
             for (int j = 0; j < 8; ++j) x[j] = ldexpf(x[j], e);
         }
-        write_planes<NP, FMT>(out + blocked_offset(r, k, rows_pad), plane_stride, x);
+        write_planes<NP, FMT>(out + blocked_offset(r, k, rows_pad), plane_stride, x, inf);
     }
 }
 
@@ -696,51 +698,50 @@ __global__ __launch_bounds__(CF::NT) void split_nt_core(int M_, int N_, int Kp_,
     V8 pa[FA ? 1 : A_CH], pb[FB ? 1 : B_CH];
     float fa[FA ? FA_CH : 1][8], fb[FB ? FB_CH : 1][8];
     // Row-contiguous source: rows [r, r+RW) of k-lines k .. k+7 into v[i][j]
-    // (row r+i, k+j); zeros outside rows x K.  RW is 1 or 2 (stage rows per
-    // thread).  full: the whole stage lies inside rows x K (uniform over the
-    // block): unguarded loads, no per-element branches.
-    auto load_rc = [&](const float *X, long ld, int rows, int r, int k, auto &v, bool full) {
+    // (row r+i, k+j).  RW is 1 or 2 (stage rows per thread).  Rows past the
+    // last read it in their place, without a branch: nothing stores their
+    // results.  kin: the stage ends inside K (uniform); else values past K are 0.
+    // (Guards on rows and k, a branch and a wait each, made the tiles at the
+    // edge up to twice as long: 32767x512x1024 TN BF16X3 took 225 us, now 117.)
+    auto load_rc = [&](const float *X, long ld, int rows, int r, int k, auto &v, bool kin) {
         constexpr int RW = std::extent<std::remove_reference_t<decltype(v)>>::value;
-        if (full) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                if constexpr (RW == 2) {
-                    const f32x2u x = *reinterpret_cast<const f32x2u *>(X + (long)(k + j) * ld + r);
-                    v[0][j] = x.x;
-                    v[1][j] = x.y;
-                } else {
-                    v[0][j] = X[(long)(k + j) * ld + r];
-                }
-            }
-            return;
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float *p = X + (long)(k + j) * ld + r;
-            if constexpr (RW == 2) {
-                if (k + j < K && r + 2 <= rows) {
-                    const f32x2u x = *reinterpret_cast<const f32x2u *>(p);
-                    v[0][j] = x.x;
-                    v[1][j] = x.y;
-                } else {
-                    v[0][j] = (k + j < K && r < rows) ? p[0] : 0.0f;
-                    v[1][j] = (k + j < K && r + 1 < rows) ? p[1] : 0.0f;
-                }
+        const bool pair = RW == 2 && (!GR || rows > 1);   // one problem: run_cfg fuses no single row
+        const float *p = X + min(r, rows - (pair ? 2 : 1));   // the last row alone is a pair's second: store_stage
+        auto line = [&](const float *q, int j) {
+            if (pair) {
+                const f32x2u x = *reinterpret_cast<const f32x2u *>(q);
+                v[0][j] = x.x;
+                v[RW - 1][j] = x.y;
             } else {
-                v[0][j] = (k + j < K && r < rows) ? p[0] : 0.0f;
+                v[0][j] = v[RW - 1][j] = *q;
             }
+        };
+        if (kin) {
+            p += (long)k * ld;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) line(p + (long)j * ld, j);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) line(p + (long)min(k + j, K - 1) * ld, j);
+#pragma unroll
+            for (int i = 0; i < RW; ++i)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v[i][j] = k + j < K ? v[i][j] : 0.0f;
         }
     };
-    // 8 floats of row `row`, k in [k, k+8), zeros outside rows x K.
-    auto load8 = [&](const float *X, long ld, int rows, int row, int k, float (&v)[8], bool full) {
-        const float *p = X + (long)row * ld + k;
-        if (full || (row < rows && k + 8 <= K)) {
-            const f32x4u x0 = *reinterpret_cast<const f32x4u *>(p);
-            const f32x4u x1 = *reinterpret_cast<const f32x4u *>(p + 4);
+    // 8 floats of row `row`, k in [k, k+8), likewise.
+    auto load8 = [&](const float *X, long ld, int rows, int row, int k, float (&v)[8], bool kin) {
+        const float *p = X + (long)min(row, rows - 1) * ld;
+        if (kin) {
+            const f32x4u x0 = *reinterpret_cast<const f32x4u *>(p + k);
+            const f32x4u x1 = *reinterpret_cast<const f32x4u *>(p + k + 4);
             v[0] = x0.x; v[1] = x0.y; v[2] = x0.z; v[3] = x0.w; v[4] = x1.x; v[5] = x1.y; v[6] = x1.z; v[7] = x1.w;
         } else {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = (row < rows && k + j < K) ? p[j] : 0.0f;
+            for (int j = 0; j < 8; ++j) {
+                const float x = p[min(k + j, K - 1)];
+                v[j] = k + j < K ? x : 0.0f;
+            }
         }
     };
     // Plane copy, chunk c (A chunks first): global -> registers, and
@@ -765,81 +766,96 @@ __global__ __launch_bounds__(CF::NT) void split_nt_core(int M_, int N_, int Kp_,
         const int k0 = kt * BK;
         const bool kin = k0 + BK <= K;
         if constexpr (FA == FUSE_RCONT) {
-            load_rc(Af, lda, M, m0 + (t % (BM / FA_CH)) * FA_CH, k0 + (t / (BM / FA_CH)) * 8, fa,
-                    kin && m0 + BM <= M);
+            load_rc(Af, lda, M, m0 + (t % (BM / FA_CH)) * FA_CH, k0 + (t / (BM / FA_CH)) * 8, fa, kin);
         } else if constexpr (FA == FUSE_KCONT) {
-            const bool full = kin && m0 + BM <= M;
 #pragma unroll
             for (int i = 0; i < FA_CH; ++i) {
                 const int f = t + CF::NT * i, r = f >> 2, c = (f & 3) ^ ((r >> 1) & 3);
-                load8(Af, lda, M, m0 + r, k0 + c * 8, fa[i], full);
+                load8(Af, lda, M, m0 + r, k0 + c * 8, fa[i], kin);
             }
         } else {
 #pragma unroll
             for (int i = 0; i < A_CH; ++i) load_chunk(kt, i);
         }
         if constexpr (FB == FUSE_RCONT) {
-            load_rc(Bf, ldb, N, n0 + (t % (BN / FB_CH)) * FB_CH, k0 + (t / (BN / FB_CH)) * 8, fb,
-                    kin && n0 + BN <= N);
+            load_rc(Bf, ldb, N, n0 + (t % (BN / FB_CH)) * FB_CH, k0 + (t / (BN / FB_CH)) * 8, fb, kin);
         } else if constexpr (FB == FUSE_KCONT) {
-            const bool full = kin && n0 + BN <= N;
 #pragma unroll
             for (int i = 0; i < FB_CH; ++i) {
                 const int f = t + CF::NT * i, r = f >> 2, c = (f & 3) ^ ((r >> 1) & 3);
-                load8(Bf, ldb, N, n0 + r, k0 + c * 8, fb[i], full);
+                load8(Bf, ldb, N, n0 + r, k0 + c * 8, fb[i], kin);
             }
         } else {
 #pragma unroll
             for (int i = 0; i < B_CH; ++i) load_chunk(kt, A_CH + i);
         }
     };
-    // Split one fused chunk (scaled formats: times 2^-e of its row) into its
-    // NP plane chunks at plane offset f * 8 of the operand's LDS region.
-    auto store_fused = [&](E *region, int plane, const unsigned *amax, int row, int f, float (&v)[8]) {
+    // Scaled formats: the exponents of this thread's fused rows, read once (at
+    // each stage, past a barrier, the load stood in front of the split).
+    int ea[FA ? FA_CH : 1], eb[FB ? FB_CH : 1];
+    bool row_inf = false;   // of any of the wave's fused rows
+    auto scales = [&](const unsigned *amax, int mode, int ch, int rows, int r0, auto &e) {
+#pragma unroll
+        for (int i = 0; i < ch; ++i) {
+            const unsigned bits = amax[r0 + (mode == FUSE_RCONT ? (t % (rows / ch)) * ch + i : (t + CF::NT * i) >> 2)];
+            e[i] = -row_exp(bits);
+            row_inf |= row_is_inf(bits);
+        }
+    };
+    if constexpr (FMT::SCALED && FA != FUSE_NONE) scales(amax_a, FA, FA_CH, BM, m0, ea);
+    if constexpr (FMT::SCALED && FB != FUSE_NONE) scales(amax_b, FB, FB_CH, BN, n0, eb);
+    if constexpr (FMT::SCALED) row_inf = __any(row_inf);
+    // Split one fused chunk (scaled formats: times 2^e) into its NP plane
+    // chunks at plane offset f * 8 of the operand's LDS region.
+    auto store_fused = [&](E *region, int plane, int e, int f, float (&v)[8]) {
         if constexpr (FMT::SCALED) {
-            const int e = -row_exp(amax[row]);
 #pragma unroll
             for (int j = 0; j < 8; ++j) v[j] = ldexpf(v[j], e);
         }
-        E o[NP][8];
-        split_vec<NP, 8>(v, o);
+        V8 w[NP];
+        split8<NP, FMT>(v, FMT::SCALED ? row_inf : __any(split_special(FMT(), v, false)), w);
 #pragma unroll
-        for (int p = 0; p < NP; ++p) {
-            V8 w;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) w[j] = o[p][j];
-            *reinterpret_cast<V8 *>(region + p * plane + f * 8) = w;
-        }
+        for (int p = 0; p < NP; ++p) *reinterpret_cast<V8 *>(region + p * plane + f * 8) = w[p];
     };
     auto store_stage = [&](int buf) {
         E *a_reg = lds + buf * STAGE, *b_reg = a_reg + NP * CF::A_PLANE;
         if constexpr (FA == FUSE_RCONT) {
+            if (FA_CH == 2 && (M & 1) && m0 + BM > M) {   // uniform: the tile at the edge of odd rows
+                const bool last = m0 + (t % (BM / FA_CH)) * FA_CH == M - 1;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) fa[0][j] = last ? fa[FA_CH - 1][j] : fa[0][j];
+            }
 #pragma unroll
             for (int i = 0; i < FA_CH; ++i) {
                 const int r = (t % (BM / FA_CH)) * FA_CH + i, f = r * 4 + ((t / (BM / FA_CH)) ^ ((r >> 1) & 3));
-                store_fused(a_reg, CF::A_PLANE, amax_a, m0 + r, f, fa[i]);
+                store_fused(a_reg, CF::A_PLANE, FMT::SCALED ? ea[i] : 0, f, fa[i]);
             }
         } else if constexpr (FA == FUSE_KCONT) {
 #pragma unroll
             for (int i = 0; i < FA_CH; ++i) {
                 const int f = t + CF::NT * i;
-                store_fused(a_reg, CF::A_PLANE, amax_a, m0 + (f >> 2), f, fa[i]);
+                store_fused(a_reg, CF::A_PLANE, FMT::SCALED ? ea[i] : 0, f, fa[i]);
             }
         } else {
 #pragma unroll
             for (int i = 0; i < A_CH; ++i) store_chunk(buf, i);
         }
         if constexpr (FB == FUSE_RCONT) {
+            if (FB_CH == 2 && (N & 1) && n0 + BN > N) {   // uniform: the tile at the edge of odd rows
+                const bool last = n0 + (t % (BN / FB_CH)) * FB_CH == N - 1;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) fb[0][j] = last ? fb[FB_CH - 1][j] : fb[0][j];
+            }
 #pragma unroll
             for (int i = 0; i < FB_CH; ++i) {
                 const int r = (t % (BN / FB_CH)) * FB_CH + i, f = r * 4 + ((t / (BN / FB_CH)) ^ ((r >> 1) & 3));
-                store_fused(b_reg, CF::B_PLANE, amax_b, n0 + r, f, fb[i]);
+                store_fused(b_reg, CF::B_PLANE, FMT::SCALED ? eb[i] : 0, f, fb[i]);
             }
         } else if constexpr (FB == FUSE_KCONT) {
 #pragma unroll
             for (int i = 0; i < FB_CH; ++i) {
                 const int f = t + CF::NT * i;
-                store_fused(b_reg, CF::B_PLANE, amax_b, n0 + (f >> 2), f, fb[i]);
+                store_fused(b_reg, CF::B_PLANE, FMT::SCALED ? eb[i] : 0, f, fb[i]);
             }
         } else {
 #pragma unroll
@@ -1331,8 +1347,8 @@ int run_cfg(const Gemm<float> &g, hipStream_t s) {
     // operand is fused per call (the larger, when both qualify).
     constexpr int RW_A = CF::BM * CF::CPR / CF::NT, RW_B = CF::BN * CF::CPR / CF::NT;
     constexpr bool RC_A = RW_A == 1 || RW_A == 2, RC_B = RW_B == 1 || RW_B == 2;
-    bool fa = CF::FUSABLE && Np / CF::BN <= 2 && (!g.ta || RC_A);
-    bool fb = CF::FUSABLE && Mp / CF::BM <= 2 && (g.tb || RC_B);
+    bool fa = CF::FUSABLE && Np / CF::BN <= 2 && (!g.ta || (RC_A && g.M >= RW_A));
+    bool fb = CF::FUSABLE && Mp / CF::BM <= 2 && (g.tb || (RC_B && g.N >= RW_B));
     if (fa && fb) (g.M >= g.N ? fb : fa) = false;
     const int fa_mode = !fa ? FUSE_NONE : (g.ta ? FUSE_RCONT : FUSE_KCONT);
     const int fb_mode = !fb ? FUSE_NONE : (g.tb ? FUSE_KCONT : FUSE_RCONT);
@@ -1589,11 +1605,8 @@ double pick_cost(const Gemm<float> &g, int np, bool scaled, bool fusable, const 
     const long ra = tm * t.bm, rb = tn * t.bn;
     const double left = scaled ? 0.5 : 0.0;   // of a fused operand's preparation: its row maxima
     const double prep = ((fa ? left : 1.0) * ra + (fb ? left : 1.0) * rb) * g.K;
-    // Two rows a thread of a row-contiguous operand (256-row tiles) are loaded
-    // together: at an odd pitch, off their alignment, the core took 1.5-1.9 times as long.
-    const bool off = t.bm == 256 && ((fa && g.ta && (g.lda & 1)) || (fb && !g.tb && (g.ldb & 1)));
     const double most = std::ceil(tm * tn * S / cus);
-    double us = t.us * (fa || fb ? f.fused : 1.0) * (off ? 1.8 : 1.0) * kc / 1000.0 * (1.0 + t.lat / std::min(most, t.occ));
+    double us = t.us * (fa || fb ? f.fused : 1.0) * kc / 1000.0 * (1.0 + t.lat / std::min(most, t.occ));
     us = (us + t.block) * most + (scaled ? 2.5 : f.prep) * prep * 4 / per_us;
     const double sums = S > 1 ? 4.0 * S * g.M * g.N : 0.0;
     if (S > 1) us += 2.5 + 0.9 * sums / per_us;

@@ -85,7 +85,8 @@ __global__ __launch_bounds__(64 * KG) void split_small_kernel(int M, int N, int 
         }
     };
 
-    int ea[FM], eb[FN];   // scaled formats: exponents to subtract
+    int ea[FM], eb[FN];     // scaled formats: exponents to add
+    bool row_inf = false;   // and whether a row's largest magnitude is infinite
     const int mine = w < steps ? (steps - 1 - w) / KG + 1 : 0;   // this wave's steps: w + KG * u, u < mine
     if constexpr (FMT::SCALED) {
         if (t < BM + BN) smax[t] = 0u;
@@ -120,9 +121,16 @@ __global__ __launch_bounds__(64 * KG) void split_small_kernel(int M, int N, int 
         }
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < FM; ++i) ea[i] = -row_exp(smax[i * 16 + fr]);
+        for (int i = 0; i < FM; ++i) {
+            ea[i] = -row_exp(smax[i * 16 + fr]);
+            row_inf |= row_is_inf(smax[i * 16 + fr]);
+        }
 #pragma unroll
-        for (int j = 0; j < FN; ++j) eb[j] = -row_exp(smax[BM + j * 16 + fr]);
+        for (int j = 0; j < FN; ++j) {
+            eb[j] = -row_exp(smax[BM + j * 16 + fr]);
+            row_inf |= row_is_inf(smax[BM + j * 16 + fr]);
+        }
+        row_inf = __any(row_inf);
     } else if (mine > 0) {
         load(w);
     }
@@ -133,26 +141,33 @@ __global__ __launch_bounds__(64 * KG) void split_small_kernel(int M, int N, int 
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
     for (int u = 0; u < mine; ++u) {
-        V8 pa[NP][FM], pb[NP][FN];
-        auto split = [&](float (&x)[8], int e, auto set) {
+        // One answer for all fragments: a branch for the step.  Three planes
+        // have no registers for both ways (spilling, 700x700x700 TT took 28.6
+        // us instead of 17.8).
+        bool special = NP == 3 || (FMT::SCALED && row_inf);
+        if constexpr (!FMT::SCALED && NP == 2) {
+#pragma unroll
+            for (int i = 0; i < FM; ++i) special |= split_special(FMT(), ra[i], false);
+#pragma unroll
+            for (int j = 0; j < FN; ++j) special |= split_special(FMT(), rb[j], false);
+            special = __any(special);
+        }
+        V8 pa[FM][NP], pb[FN][NP];
+        auto split = [&](float (&x)[8], int e, bool sp, V8 (&w)[NP]) {
             if constexpr (FMT::SCALED) {
 #pragma unroll
                 for (int q = 0; q < 8; ++q) x[q] = ldexpf(x[q], e);
             }
-            typename FMT::E o[NP][8];
-            split_vec<NP, 8>(x, o);
-#pragma unroll
-            for (int p = 0; p < NP; ++p) {
-                V8 v;
-#pragma unroll
-                for (int q = 0; q < 8; ++q) v[q] = o[p][q];
-                set(p, v);
-            }
+            split8<NP, FMT>(x, sp, w);
         };
+        auto split_all = [&](bool sp) {
 #pragma unroll
-        for (int i = 0; i < FM; ++i) split(ra[i], FMT::SCALED ? ea[i] : 0, [&](int p, const V8 &v) { pa[p][i] = v; });
+            for (int i = 0; i < FM; ++i) split(ra[i], FMT::SCALED ? ea[i] : 0, sp, pa[i]);
 #pragma unroll
-        for (int j = 0; j < FN; ++j) split(rb[j], FMT::SCALED ? eb[j] : 0, [&](int p, const V8 &v) { pb[p][j] = v; });
+            for (int j = 0; j < FN; ++j) split(rb[j], FMT::SCALED ? eb[j] : 0, sp, pb[j]);
+        };
+        if (special) split_all(true);
+        else split_all(false);
         if (u + 1 < mine) load(w + KG * (u + 1));
         __builtin_amdgcn_sched_barrier(0);   // the loads stay in front of the MFMAs
 #pragma unroll
@@ -161,7 +176,7 @@ __global__ __launch_bounds__(64 * KG) void split_small_kernel(int M, int N, int 
             for (int i = 0; i < FM; ++i)
 #pragma unroll
                 for (int j = 0; j < FN; ++j)
-                    acc[i][j] = FMT::mfma(pa[Products<NP>::a[q]][i], pb[Products<NP>::b[q]][j], acc[i][j]);
+                    acc[i][j] = FMT::mfma(pa[i][Products<NP>::a[q]], pb[j][Products<NP>::b[q]], acc[i][j]);
     }
 
     // Every wave's sums into LDS, then one value per thread and turn.
