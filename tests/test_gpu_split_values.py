@@ -84,3 +84,36 @@ def test_special_values(mode, ta, tb):
             ug.force_splits(mode, 0)
             dA.free()
             dB.free()
+
+
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
+@pytest.mark.parametrize("K", [64, 65, 200, 300, 513, 1100, 2048, 2049, 8192, 8200])
+def test_row_scales(K, ta, tb):
+    """FP16X3's preparation: pairs of whole rows on 16 .. 256 threads, maxima
+    in parts and combined, columns by 64 and by 256, with and without an operand
+    that the core splits; wide data, so that a wrong scale shows."""
+    mode = ug.MODE_FP16X3
+    g = orc.rng(K)
+    for M, N in [(70, 333), (600, 130)] + ([(64, 20000)] if K in (200, 2049) else []):
+        A, B = orc.wide_range(g, (M, K)).astype(np.float32), orc.wide_range(g, (N, K)).astype(np.float32)
+        a, b = np.ascontiguousarray(A.T if ta == "T" else A), np.ascontiguousarray(B if tb == "T" else B.T)
+        exact = A.astype(np.float64) @ B.astype(np.float64).T
+        scale = np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64).T
+        dA, dB = hip.DeviceArray.from_host(a), hip.DeviceArray.from_host(b)
+        try:
+            for variant in (3, 7):
+                ug.force_variant(mode, variant)
+                ug.force_splits(mode, 1)
+                print(f"K {K} {ta}{tb} {M}x{N} variant {variant}", flush=True)
+                dC = hip.DeviceArray.from_host(np.zeros((M, N), np.float32))
+                ug.sgemm_dev("R", ta, tb, M, N, K, 1.0, dA, a.shape[1], dB, b.shape[1], 0.0, dC, N, mode=mode)
+                hip.synchronize()
+                got = dC.download()
+                dC.free()
+                ok, worst = orc.check_bound(got, exact, scale, orc.tolerance(K + 2, extra=MODE_EXTRA[mode]))
+                assert ok, worst
+        finally:
+            ug.force_variant(mode, -1)
+            ug.force_splits(mode, 0)
+            dA.free()
+            dB.free()

@@ -70,45 +70,9 @@ __device__ __forceinline__ long blocked_offset(int r, int k, int rows_pad) {
     return ((long)(k >> 5) * rows_pad + r) * 32 + ((((k >> 3) & 3) ^ ((r >> 1) & 3)) << 3);
 }
 
-// Source element (r, k) of the operand: KCONT ? X[r*ld + k] : X[k*ld + r];
-// zeros outside rows x K.  KCONT version: one thread per 8 k of one row
-// (chunk f of the rows_pad x k_pad/8 chunks).
-// FMT::SCALED: row r is multiplied by 2^-row_exp(amax[r]) before splitting.
-template <int NP, class FMT>
-__device__ __forceinline__ void prep_kcont_chunk(const float *__restrict__ X, long ld, int rows, int K, typename FMT::E *__restrict__ out, long plane_stride, int rows_pad,
-                                                 int k_pad, const unsigned *__restrict__ amax, long f) {
-    const long chunks_per_row = k_pad / 8;
-    const int r = (int)(f / chunks_per_row);
-    const int k = (int)(f - (long)r * chunks_per_row) * 8;
-    float x[8];
-    const float *p = X + (long)r * ld + k;
-    if (r < rows && k + 8 <= K) {
-        const f32x4u a = *reinterpret_cast<const f32x4u *>(p);
-        const f32x4u b = *reinterpret_cast<const f32x4u *>(p + 4);
-        x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = (r < rows && k + j < K) ? p[j] : 0.0f;
-    }
-    bool inf = false;
-    if constexpr (FMT::SCALED) {
-        const int e = -row_exp(amax[r]);
-        inf = row_is_inf(amax[r]);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = ldexpf(x[j], e);
-    }
-    write_planes<NP, FMT>(out + blocked_offset(r, k, rows_pad), plane_stride, x, inf);
-}
-
-template <int NP, class FMT>
-__global__ __launch_bounds__(256) void split_prep_kcont(const float *__restrict__ X, long ld, int rows, int K,
-                                                        typename FMT::E *__restrict__ out,
-                                                        long plane_stride, int rows_pad, int k_pad,
-                                                        const unsigned *__restrict__ amax) {
-    const long total = (long)rows_pad * (k_pad / 8);
-    for (long f = (long)blockIdx.x * blockDim.x + threadIdx.x; f < total; f += (long)gridDim.x * blockDim.x)
-        prep_kcont_chunk<NP, FMT>(X, ld, rows, K, out, plane_stride, rows_pad, k_pad, amax, f);
-}
+// Source element (r, k) of the operand: X[r*ld + k] (k-contiguous) or
+// X[k*ld + r] (row-contiguous); zeros outside rows x K.  FMT::SCALED: row r is
+// multiplied by 2^-row_exp(amax[r]) before splitting.
 
 // k-contiguous source, 2-D blocks: block (bx, by) covers rows [64 bx, +64)
 // and k [128 by, +128) (four 32-wide k tiles).  Chunk f = t + 256 i of a
@@ -156,15 +120,6 @@ __device__ __forceinline__ void prep_kcont_tile(const float *__restrict__ X, lon
     }
 }
 
-template <int NP, class FMT>
-__global__ __launch_bounds__(256) void split_prep_kcont_tiles(const float *__restrict__ X, long ld, int rows, int K,
-                                                              typename FMT::E *__restrict__ out,
-                                                              long plane_stride, int rows_pad, int k_pad,
-                                                              const unsigned *__restrict__ amax) {
-    prep_kcont_tile<NP, FMT>(X, ld, rows, K, out, plane_stride, rows_pad, k_pad, amax, blockIdx.x * 64,
-                             blockIdx.y * 128);
-}
-
 // FP16X3, k-contiguous source with k_pad <= 8192: the row maximum and the
 // split in one pass.  Block b reads rows r0 = 2b and r0 + 1 once into
 // registers, reduces each row's largest magnitude (amax[r], as the separate
@@ -177,15 +132,25 @@ __global__ __launch_bounds__(256) void split_prep_kcont_tiles(const float *__res
 // in K tile t / 8 of each 32-tile pass (at most 8 passes, k_pad <= 8192).
 // Each row's maximum is reduced over the lanes that hold it (shuffles that
 // keep bit 2 of the lane fixed), then over the waves.
+// lanes (16 .. 256, a power of two): threads to a pair of rows.  Rows of fewer
+// than 32 K tiles leave the rest of the block to further pairs (row_lanes;
+// 30564x448x49: 85 us a call before, 38 now).
+inline int row_lanes(int k_pad) {   // 8 a K tile; k_pad is a multiple of 64
+    int lanes = 16;
+    while (lanes < 256 && lanes * 4 < k_pad) lanes *= 2;
+    return lanes;
+}
+
 template <int NP, class FMT>
 __device__ __forceinline__ void prep_kcont_rowscaled_pair(const float *__restrict__ X, long ld, int rows, int K,
                                                           typename FMT::E *__restrict__ out,
                                                           long plane_stride, int rows_pad, int k_pad,
-                                                          unsigned *__restrict__ amax, int r0) {
+                                                          unsigned *__restrict__ amax, int r0,
+                                                          int lanes = 256) {
     static_assert(FMT::SCALED, "row scales");
     constexpr int PASSES = 8;   // 8 passes x 32 K tiles x 32 = 8192
-    const int t = threadIdx.x;
-    const int ktl = t >> 3, rr = (t >> 2) & 1, cc = t & 3, r = r0 + rr;
+    const int t = threadIdx.x & (lanes - 1), group = threadIdx.x / lanes;
+    const int ktl = t >> 3, rr = (t >> 2) & 1, cc = t & 3, r = r0 + 2 * group + rr;
     const int ktiles = k_pad / 32;
     float x[PASSES][8];
     float m = 0.0f;
@@ -208,12 +173,16 @@ __device__ __forceinline__ void prep_kcont_rowscaled_pair(const float *__restric
     m = fmaxf(m, __shfl_xor(m, 1));
     m = fmaxf(m, __shfl_xor(m, 2));
     m = fmaxf(m, __shfl_xor(m, 8));
-    m = fmaxf(m, __shfl_xor(m, 16));
-    m = fmaxf(m, __shfl_xor(m, 32));
-    __shared__ float wmax[4][2];
-    if ((t & 63) < 8 && (t & 3) == 0) wmax[t >> 6][rr] = m;
-    __syncthreads();
-    m = fmaxf(fmaxf(wmax[0][rr], wmax[1][rr]), fmaxf(wmax[2][rr], wmax[3][rr]));
+    if (lanes > 16) m = fmaxf(m, __shfl_xor(m, 16));
+    if (lanes > 32) m = fmaxf(m, __shfl_xor(m, 32));
+    if (lanes > 64) {   // uniform: 2 or 4 waves a group
+        __shared__ float wmax[4][2];
+        if ((t & 63) < 8 && (t & 3) == 0) wmax[threadIdx.x >> 6][rr] = m;
+        __syncthreads();
+        const int w0 = group * (lanes >> 6);
+        m = fmaxf(wmax[w0][rr], wmax[w0 + 1][rr]);
+        if (lanes == 256) m = fmaxf(m, fmaxf(wmax[2][rr], wmax[3][rr]));
+    }
     const unsigned bits = m > 0.0f ? __float_as_uint(m) : 0u;
     if (t < 8 && (t & 3) == 0) amax[r] = bits;
     const int e = -row_exp(bits);
@@ -228,29 +197,33 @@ __device__ __forceinline__ void prep_kcont_rowscaled_pair(const float *__restric
     }
 }
 
-template <int NP, class FMT>
-__global__ __launch_bounds__(256) void split_prep_kcont_rowscaled(const float *__restrict__ X, long ld, int rows,
-                                                                  int K, typename FMT::E *__restrict__ out,
-                                                                  long plane_stride, int rows_pad, int k_pad,
-                                                                  unsigned *__restrict__ amax) {
-    prep_kcont_rowscaled_pair<NP, FMT>(X, ld, rows, K, out, plane_stride, rows_pad, k_pad, amax,
-                                       (int)blockIdx.x * 2);
-}
+// Partial row maxima of a row-contiguous operand, at most (FP16X3).
+constexpr int kAmaxParts = 16;
 
 // Row-contiguous source (X[k*ld + r]): the 64 x 64 tile (rows r0.., k k0..)
 // transposed through LDS (tile[64][65], 256 threads).
 template <int NP, class FMT>
 __device__ __forceinline__ void prep_rcont_tile(const float *__restrict__ X, long ld, int rows, int K, typename FMT::E *__restrict__ out, long plane_stride, int rows_pad,
                                                 int k_pad, const unsigned *__restrict__ amax, int r0, int k0,
-                                                float (*tile)[65]) {
+                                                float (*tile)[65], const unsigned *__restrict__ parts = nullptr,
+                                                int nparts = 0) {
     const int t = threadIdx.x;
-    // Scaled formats: this thread's two row maxima, loaded before the tile.
-    unsigned am[2] = {0u, 0u};
+    // Scaled formats: this thread's two row maxima, loaded before the tile; or
+    // (parts) its share of one row's, put together behind the tile's barrier.
+    unsigned am[2] = {0u, 0u}, pm[kAmaxParts / 4];
+    __shared__ unsigned pmax[FMT::SCALED ? 4 : 1][FMT::SCALED ? 64 : 1];
     if constexpr (FMT::SCALED) {
+        if (nparts) {
+            const int r = min(r0 + (t & 63), rows - 1);   // repeats change no maximum; past the rows it is not used
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int r = r0 + (t + i * 256) / 8;
-            am[i] = r < rows_pad ? amax[r] : 0u;
+            for (int i = 0; i < kAmaxParts / 4; ++i)
+                pm[i] = parts[(long)min((t >> 6) + 4 * i, nparts - 1) * rows_pad + r];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int r = r0 + (t + i * 256) / 8;
+                am[i] = r < rows_pad ? amax[r] : 0u;
+            }
         }
     }
     // Read: 64 k-lines of 64 r each, as 16 float4 per line (coalesced along r).
@@ -271,7 +244,18 @@ __device__ __forceinline__ void prep_rcont_tile(const float *__restrict__ X, lon
 #pragma unroll
         for (int j = 0; j < 4; ++j) tile[kk][rr + j] = v[j];
     }
+    if constexpr (FMT::SCALED) {
+        if (nparts) pmax[t >> 6][t & 63] = max(max(pm[0], pm[1]), max(pm[2], pm[3]));
+    }
     __syncthreads();
+    if constexpr (FMT::SCALED) {
+        if (nparts) {
+            auto row_max = [&](int r) { return max(max(pmax[0][r], pmax[1][r]), max(pmax[2][r], pmax[3][r])); };
+#pragma unroll
+            for (int i = 0; i < 2; ++i) am[i] = row_max((t + i * 256) / 8);
+            if (k0 == 0 && t < 64 && r0 + t < rows_pad) const_cast<unsigned *>(amax)[r0 + t] = row_max(t);
+        }
+    }
     // Write: 64 rows of 8 chunks of 8 k.
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -289,16 +273,6 @@ __device__ __forceinline__ void prep_rcont_tile(const float *__restrict__ X, lon
         }
         write_planes<NP, FMT>(out + blocked_offset(r, k, rows_pad), plane_stride, x, row_is_inf(am[i]));
     }
-}
-
-template <int NP, class FMT>
-__global__ __launch_bounds__(256) void split_prep_rcont(const float *__restrict__ X, long ld, int rows, int K,
-                                                        typename FMT::E *__restrict__ out,
-                                                        long plane_stride, int rows_pad, int k_pad,
-                                                        const unsigned *__restrict__ amax) {
-    __shared__ float tile[64][65];
-    prep_rcont_tile<NP, FMT>(X, ld, rows, K, out, plane_stride, rows_pad, k_pad, amax, blockIdx.x * 64,
-                             blockIdx.y * 64, tile);
 }
 
 // block_job[b]: the job of preparation block b (one load, where a search of
@@ -337,7 +311,7 @@ __global__ __launch_bounds__(256) void grouped_split_prep(const PrepJob *__restr
     }
 }
 
-// Both operands of one GEMM in one launch (formats without row scales):
+// Both operands of one GEMM in one launch (scaled formats: their maxima known):
 // blocks [0, b.block0) prepare a, the rest b, one tile each (64-row x 128-k
 // tiles of a k-contiguous operand, 64 x 64 transposing tiles of a
 // row-contiguous one; nbx blocks along the rows).  One launch instead of
@@ -345,7 +319,6 @@ __global__ __launch_bounds__(256) void grouped_split_prep(const PrepJob *__restr
 // (2048^3 BF16x3: 263 against 256 TF/s per call).
 template <int NP, class FMT>
 __global__ __launch_bounds__(256) void split_prep_pair(PrepJob a, PrepJob b) {
-    static_assert(!FMT::SCALED, "row-scaled formats compute their maxima first");
     __shared__ float tile[64][65];
     const bool second = (int)blockIdx.x >= b.block0;
     const PrepJob &j = second ? b : a;
@@ -354,10 +327,10 @@ __global__ __launch_bounds__(256) void split_prep_pair(PrepJob a, PrepJob b) {
     const int r0 = (lb % j.nbx) * 64;
     if (j.kcont)
         prep_kcont_tile<NP, FMT>(j.X, j.ld, j.rows, j.K, out, j.plane_stride, j.rows_pad, j.k_pad,
-                                 nullptr, r0, (lb / j.nbx) * 128);
+                                 j.amax, r0, (lb / j.nbx) * 128);
     else
         prep_rcont_tile<NP, FMT>(j.X, j.ld, j.rows, j.K, out, j.plane_stride, j.rows_pad, j.k_pad,
-                                 nullptr, r0, (lb / j.nbx) * 64, tile);
+                                 j.amax, r0, (lb / j.nbx) * 64, tile, j.parts, j.nparts);
 }
 
 // Largest magnitude of every plane row (row r of op(A), column r of op(B))
@@ -368,12 +341,13 @@ __global__ void fill_zero_u32(unsigned *__restrict__ p, long n) {
 }
 
 // k-contiguous source: block b covers row b / kchunks, k in [2048 * (b % kchunks), +2048).
+// One chunk a row: stored, not combined, and the block may lie past the rows (0).
 __device__ __forceinline__ void row_amax_kcont_block(const float *__restrict__ X, long ld, int rows, int K, long kchunks, unsigned *__restrict__ amax, long b) {
     const int r = (int)(b / kchunks);
     const int k = (int)(b % kchunks) * 2048 + threadIdx.x * 8;
     const float *p = X + (long)r * ld + k;
     float m = 0.0f;
-    if (k + 8 <= K) {
+    if (r < rows && k + 8 <= K) {
         const f32x4u a = *reinterpret_cast<const f32x4u *>(p);
         const f32x4u c = *reinterpret_cast<const f32x4u *>(p + 4);
         m = fmaxf(fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))),
@@ -381,7 +355,7 @@ __device__ __forceinline__ void row_amax_kcont_block(const float *__restrict__ X
     } else {
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-            if (k + j < K) m = fmaxf(m, fabsf(p[j]));
+            if (r < rows && k + j < K) m = fmaxf(m, fabsf(p[j]));
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
@@ -390,47 +364,48 @@ __device__ __forceinline__ void row_amax_kcont_block(const float *__restrict__ X
     __syncthreads();
     if (threadIdx.x == 0) {
         m = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-        if (r < rows && m > 0.0f) atomicMax(&amax[r], __float_as_uint(m));
+        if (kchunks == 1) {
+            amax[r] = m > 0.0f ? __float_as_uint(m) : 0u;
+        } else if (r < rows && m > 0.0f) {
+            atomicMax(&amax[r], __float_as_uint(m));
+        }
     }
 }
 
-__global__ __launch_bounds__(256) void row_amax_kcont(const float *__restrict__ X, long ld, int rows, int K,
-                                                      long kchunks, unsigned *__restrict__ amax) {
-    row_amax_kcont_block(X, ld, rows, K, kchunks, amax, blockIdx.x);
-}
-
 // Row-contiguous source (X[k*ld + r]): block b covers columns r in
-// [256 * (b % cblocks), +256) and k in [S * (b / cblocks), +S), S =
-// kAmaxRcontSpan,
-// cblocks = ceil(rows / 256): consecutive blocks read neighbouring 1 KB row
-// segments (blocks that shared columns and differed only in k read addresses
-// a power-of-two multiple of the row pitch apart, which crowd the same HBM
-// channels).
-__device__ __forceinline__ void row_amax_rcont_block(const float *__restrict__ X, long ld, int rows, int K, long kblocks, unsigned *__restrict__ amax, long b) {
-    const long cblocks = (rows + 255) / 256;
-    constexpr int SPAN = kAmaxRcontSpan;
-    const int c0 = (int)(b % cblocks) * 256, k0 = (int)(b / cblocks) * SPAN;
-    (void)kblocks;
-    const int cg = threadIdx.x & 63, kp = threadIdx.x >> 6;
+// [4 CG (b % cblocks), +4 CG) and k in [S * (b / cblocks), +S), S =
+// kAmaxRcontSpan, cblocks = ceil(rows / (4 CG)): consecutive blocks read
+// neighbouring row segments (blocks that shared columns and differed only in
+// k read addresses a power-of-two multiple of the row pitch apart, which crowd
+// the same HBM channels).  CG = 64: 1 KB segments; CG = 16, four times the
+// blocks, for operands that would leave CUs idle.  PARTS: row b / cblocks of
+// the partial maxima (rows_pad long) instead of combined ones.
+template <int CG, bool PARTS = false>
+__device__ __forceinline__ void row_amax_rcont_block(const float *__restrict__ X, long ld, int rows, int K,
+                                                     unsigned *__restrict__ amax, long b, long rows_pad = 0) {
+    constexpr int COLS = 4 * CG, KP = 256 / CG, SPAN = kAmaxRcontSpan, PER = SPAN / KP, BATCH = PER < 16 ? PER : 16;
+    const long cblocks = (rows + COLS - 1) / COLS;
+    const int c0 = (int)(b % cblocks) * COLS, k0 = (int)(b / cblocks) * SPAN;
+    const int cg = threadIdx.x % CG, kp = threadIdx.x / CG;
     const int c = c0 + cg * 4;
     float m[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (c + 4 <= rows && k0 + SPAN <= K) {
-        // Whole block: SPAN/4 independent 16-byte loads per thread, issued 16 at
+        // Whole block: PER independent 16-byte loads per thread, issued 16 at
         // a time into registers before any is used (the compiler otherwise
         // waits after every second load, which leaves HBM idle).
         const float *p = X + (long)(k0 + kp) * ld + c;
-        for (int kb = 0; kb < SPAN / 4; kb += 16) {
-            f32x4u v[16];
+        for (int kb = 0; kb < PER; kb += BATCH) {
+            f32x4u v[BATCH];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = *reinterpret_cast<const f32x4u *>(p + (long)(kb + i) * 4 * ld);
+            for (int i = 0; i < BATCH; ++i) v[i] = *reinterpret_cast<const f32x4u *>(p + (long)(kb + i) * KP * ld);
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
+            for (int i = 0; i < BATCH; ++i) {
                 m[0] = fmaxf(m[0], fabsf(v[i].x)); m[1] = fmaxf(m[1], fabsf(v[i].y));
                 m[2] = fmaxf(m[2], fabsf(v[i].z)); m[3] = fmaxf(m[3], fabsf(v[i].w));
             }
         }
     } else {
-        for (int kk = kp; kk < SPAN && k0 + kk < K; kk += 4) {
+        for (int kk = kp; kk < SPAN && k0 + kk < K; kk += KP) {
             const float *p = X + (long)(k0 + kk) * ld + c;
             if (c + 4 <= rows) {
                 const f32x4u a = *reinterpret_cast<const f32x4u *>(p);
@@ -443,48 +418,63 @@ __device__ __forceinline__ void row_amax_rcont_block(const float *__restrict__ X
             }
         }
     }
-    __shared__ float sm[4][256];
+    __shared__ float sm[KP][COLS];
 #pragma unroll
     for (int j = 0; j < 4; ++j) sm[kp][cg * 4 + j] = m[j];
     __syncthreads();
     const int t = threadIdx.x, col = c0 + t;
-    const float v = fmaxf(fmaxf(sm[0][t], sm[1][t]), fmaxf(sm[2][t], sm[3][t]));
-    if (col < rows && v > 0.0f) atomicMax(&amax[col], __float_as_uint(v));
+    if (t >= COLS || col >= rows) return;
+    float v = sm[0][t];
+#pragma unroll
+    for (int i = 1; i < KP; ++i) v = fmaxf(v, sm[i][t]);
+    if constexpr (PARTS) amax[(b / cblocks) * rows_pad + col] = v > 0.0f ? __float_as_uint(v) : 0u;
+    else if (v > 0.0f) atomicMax(&amax[col], __float_as_uint(v));
 }
 
-__global__ __launch_bounds__(256) void row_amax_rcont(const float *__restrict__ X, long ld, int rows, int K,
-                                                      long kblocks, unsigned *__restrict__ amax) {
-    row_amax_rcont_block(X, ld, rows, K, kblocks, amax, blockIdx.x);
+// Before the planes of one FP16X3 GEMM, in one launch for both operands, so
+// that their passes over HBM overlap: `none`, or whole rows of a k-contiguous
+// operand to planes and maxima (prep_kcont_rowscaled_pair), or only its row
+// maxima, or those of a row-contiguous operand (columns by 256 or 64, combined
+// or in parts).
+enum ScaleKind { SCALE_NONE, SCALE_SPLIT_ROWS, SCALE_KCONT, SCALE_RCONT, SCALE_RCONT_NARROW, SCALE_PARTS,
+                 SCALE_PARTS_NARROW };
+struct ScaleJob {
+    const float *X;
+    long ld, plane_stride, chunks;   // chunks: of 2048 a row; SCALE_SPLIT_ROWS: lanes
+    void *out;
+    unsigned *amax, *parts;
+    int kind, rows, rows_pad, k_pad, blocks;
+};
+template <int NP, class FMT>
+__global__ __launch_bounds__(256) void split_scales(ScaleJob a, ScaleJob b, int K) {
+    const bool second = (int)blockIdx.x >= a.blocks;
+    const ScaleJob &j = second ? b : a;
+    const int lb = (int)blockIdx.x - (second ? a.blocks : 0);
+    switch (j.kind) {
+        case SCALE_SPLIT_ROWS:
+            prep_kcont_rowscaled_pair<NP, FMT>(j.X, j.ld, j.rows, K, static_cast<typename FMT::E *>(j.out),
+                                               j.plane_stride, j.rows_pad, j.k_pad, j.amax,
+                                               lb * (int)(512 / j.chunks), (int)j.chunks);
+            break;
+        case SCALE_KCONT: row_amax_kcont_block(j.X, j.ld, j.rows, K, j.chunks, j.amax, lb); break;
+        case SCALE_RCONT: row_amax_rcont_block<64>(j.X, j.ld, j.rows, K, j.amax, lb); break;
+        case SCALE_RCONT_NARROW: row_amax_rcont_block<16>(j.X, j.ld, j.rows, K, j.amax, lb); break;
+        case SCALE_PARTS: row_amax_rcont_block<64, true>(j.X, j.ld, j.rows, K, j.parts, lb, j.rows_pad); break;
+        case SCALE_PARTS_NARROW: row_amax_rcont_block<16, true>(j.X, j.ld, j.rows, K, j.parts, lb, j.rows_pad); break;
+        default: break;
+    }
 }
 
 // Row maxima of the operands of a grouped FP16X3 plan: job j (PrepJob with
 // out = its maxima, nbx = K chunks per row (k-contiguous: 2048 wide) or per
 // 256-column block (row-contiguous: kAmaxRcontSpan deep)), blocks as in the kernels above.
-// FP16X3 with k-contiguous op(A) (K <= 8192) and row-contiguous op(B): A's
-// fused row maximum + split (one block per two padded rows of A) and B's column
-// maxima (row_amax_rcont blocks, combined with atomicMax into zeroed maxima)
-// in one launch, so that the two passes over HBM overlap.  Blocks below
-// b_blocks scan B; the others split rows 2 (blockIdx.x - b_blocks) and the
-// next of A.
-template <int NP, class FMT>
-__global__ __launch_bounds__(256) void split_prep_rowscaled_a_amax_b(
-    const float *__restrict__ A, long lda, int rows_a, int K, typename FMT::E *__restrict__ out_a,
-    long plane_a, int rows_pad_a, int k_pad, unsigned *__restrict__ amax_a, const float *__restrict__ B, long ldb,
-    int rows_b, long kblocks_b, unsigned *__restrict__ amax_b, int b_blocks) {
-    if ((int)blockIdx.x < b_blocks)
-        row_amax_rcont_block(B, ldb, rows_b, K, kblocks_b, amax_b, blockIdx.x);
-    else
-        prep_kcont_rowscaled_pair<NP, FMT>(A, lda, rows_a, K, out_a, plane_a, rows_pad_a, k_pad, amax_a,
-                                           ((int)blockIdx.x - b_blocks) * 2);
-}
-
 __global__ __launch_bounds__(256) void grouped_row_amax(const PrepJob *__restrict__ jobs,
                                                         const int *__restrict__ block_job) {
     const PrepJob j = jobs[block_job[blockIdx.x]];
     const long lb = (long)blockIdx.x - j.block0;
     unsigned *amax = static_cast<unsigned *>(j.out);
     if (j.kcont) row_amax_kcont_block(j.X, j.ld, j.rows, j.K, j.nbx, amax, lb);
-    else row_amax_rcont_block(j.X, j.ld, j.rows, j.K, j.nbx, amax, lb);
+    else row_amax_rcont_block<64>(j.X, j.ld, j.rows, j.K, amax, lb);
 }
 
 // Implicit im2col operand of a convolution (ConvDesc): element (n, k) of the
@@ -1235,59 +1225,109 @@ int planes_of(int mode) {
 
 static long round_up(long x, long a) { return (x + a - 1) / a * a; }
 
-// Scaled formats: amax (rows_pad entries, zeroed by the caller) receives the
-// per-row largest magnitudes before the split reads them.
-// split == false: only the row maxima (scaled formats); the core splits the
-// operand itself while staging it.
+// One operand of a GEMM to prepare: its source, its planes (out null: the core
+// splits it, only the row maxima are wanted), row maxima (scaled formats) and,
+// if there is room for them, partial maxima (kAmaxParts rows of rows_pad).
+struct Side {
+    const float *X;
+    long ld;
+    bool kcont;
+    int rows, rows_pad;
+    void *out;
+    long plane_stride;
+    unsigned *amax, *parts;
+};
+bool side_in_parts(bool kcont, bool planes, int K) {
+    return !kcont && planes && (K + kAmaxRcontSpan - 1) / kAmaxRcontSpan <= kAmaxParts;
+}
+
+// Planes and row maxima of up to two operands in the fewest launches, each
+// 4-5 us of a call: the BF16 forms one.  FP16X3 one where every operand is
+// k-contiguous with K <= 8192 (row maximum and split of whole rows together);
+// else the maxima of both (or the whole rows of one) in one and the remaining
+// planes in another.  Row-contiguous operands with K <= 2048 hand partial
+// maxima over; longer ones, and those split in the core, combine them in
+// memory, which a fill clears first (a kernel, not a memset: callers may capture
+// this call in a graph).
+// us a call, one preparation an operand and a fill before / now: 655x4518x667 TN
+// 68 / 43, 543x128x3603 TT 46 / 34, 700x3000x1000 NN 52 / 46, 2048^3 NT 79 / 76.
 template <int NP, class FMT>
-int prep_operand(const float *X, long ld, bool kcont, int rows, int K, typename FMT::E *out, long plane_stride,
-                 int rows_pad, int k_pad, unsigned *amax, hipStream_t s, bool split = true, bool amax_done = false) {
+int prep_operands(Side a, Side b, int K, int k_pad, bool zeroed, hipStream_t s) {
+    bool rows_done[2] = {false, false};
+    Side *sides[2] = {&a, &b};
     if constexpr (FMT::SCALED) {
-        if (amax_done) goto planes;   // the row maxima were computed by an earlier launch
-        if (split && kcont && rows > 0 && K > 0 && k_pad <= 8192 && rows_pad % 2 == 0) {
-            // Row maxima and planes in one pass (one block per two padded rows).
-            hipLaunchKernelGGL((split_prep_kcont_rowscaled<NP, FMT>), dim3((unsigned)(rows_pad / 2)), dim3(256), 0, s, X,
-                               ld, rows, K, out, plane_stride, rows_pad, k_pad, amax);
-            UGEMM_HIP_TRY(hipGetLastError());
-            return UGEMM_OK;
-        }
-        if (rows > 0 && K > 0) {
-            if (kcont) {
-                const long kchunks = (K + 2047) / 2048;
-                hipLaunchKernelGGL(row_amax_kcont, dim3((unsigned)(rows * kchunks)), dim3(256), 0, s, X, ld, rows, K,
-                                   kchunks, amax);
+        ScaleJob jobs[2] = {};
+        bool combine = false;
+        for (int i = 0; i < 2; ++i) {
+            Side &d = *sides[i];
+            ScaleJob &j = jobs[i];
+            if (!d.X) continue;
+            j.X = d.X;
+            j.ld = d.ld;
+            j.plane_stride = d.plane_stride;
+            j.out = d.out;
+            j.amax = d.amax;
+            j.parts = d.parts;
+            j.rows = d.rows;
+            j.rows_pad = d.rows_pad;
+            j.k_pad = k_pad;
+            long blocks;
+            if (d.kcont && d.out && k_pad <= 8192) {
+                j.kind = SCALE_SPLIT_ROWS;
+                j.chunks = row_lanes(k_pad);
+                blocks = d.rows_pad / (512 / j.chunks);
+                rows_done[i] = true;
+            } else if (d.kcont) {
+                j.kind = SCALE_KCONT;
+                j.chunks = (K + 2047) / 2048;
+                blocks = j.chunks == 1 ? d.rows_pad : d.rows * j.chunks;
+                combine |= j.chunks > 1;
             } else {
-                const long kblocks = (K + kAmaxRcontSpan - 1) / kAmaxRcontSpan, cblocks = (rows + 255) / 256;
-                hipLaunchKernelGGL(row_amax_rcont, dim3((unsigned)(cblocks * kblocks)), dim3(256), 0, s, X, ld, rows,
-                                   K, kblocks, amax);
+                const long kblocks = (K + kAmaxRcontSpan - 1) / kAmaxRcontSpan;
+                const bool parts = d.parts != nullptr, narrow = kblocks * ((d.rows + 255) / 256) < device_cu_count();
+                j.kind = parts ? (narrow ? SCALE_PARTS_NARROW : SCALE_PARTS) : (narrow ? SCALE_RCONT_NARROW : SCALE_RCONT);
+                blocks = kblocks * (narrow ? (d.rows + 63) / 64 : (d.rows + 255) / 256);
+                combine |= !parts;
             }
+            if (blocks > 0x7fffffffL) return fail(UGEMM_ERR_ARG, "too many row blocks");
+            j.blocks = (int)blocks;
         }
+        if (combine && !zeroed)   // the maxima of both operands, one array
+            hipLaunchKernelGGL(fill_zero_u32, dim3((unsigned)std::min<long>((a.rows_pad + b.rows_pad + 255) / 256, 1024)),
+                               dim3(256), 0, s, a.amax, (long)a.rows_pad + b.rows_pad);
+        // The scans first: whole rows keep a block busier.
+        const bool swap = jobs[0].kind == SCALE_SPLIT_ROWS;
+        const long blocks = (long)jobs[0].blocks + jobs[1].blocks;
+        if (blocks > 0x7fffffffL) return fail(UGEMM_ERR_ARG, "too many row blocks");
+        hipLaunchKernelGGL((split_scales<NP, FMT>), dim3((unsigned)blocks), dim3(256), 0, s, jobs[swap], jobs[!swap], K);
     }
-    if (!split) {
-        UGEMM_HIP_TRY(hipGetLastError());
-        return UGEMM_OK;
+    PrepJob jobs[2] = {};
+    long blocks = 0;
+    for (int i = 0; i < 2; ++i) {
+        const Side &d = *sides[i];
+        PrepJob &j = jobs[i];
+        j.block0 = (int)blocks;
+        if (!d.X || !d.out || rows_done[i]) continue;
+        j.X = d.X;
+        j.ld = d.ld;
+        j.out = d.out;
+        j.plane_stride = d.plane_stride;
+        j.rows = d.rows;
+        j.K = K;
+        j.rows_pad = d.rows_pad;
+        j.k_pad = k_pad;
+        j.kcont = d.kcont;
+        j.nbx = d.rows_pad / 64;
+        j.amax = d.amax;
+        j.parts = d.parts;
+        j.nparts = d.parts ? (K + kAmaxRcontSpan - 1) / kAmaxRcontSpan : 0;
+        blocks += (long)j.nbx * (d.kcont ? (k_pad + 127) / 128 : k_pad / 64);
+        if (blocks > 0x7fffffffL) return fail(UGEMM_ERR_ARG, "too many preparation blocks");
     }
-planes:
-    if (kcont && rows_pad % 64 == 0 && (k_pad + 127) / 128 < 65536) {
-        dim3 grid((unsigned)(rows_pad / 64), (unsigned)((k_pad + 127) / 128));
-        hipLaunchKernelGGL((split_prep_kcont_tiles<NP, FMT>), grid, dim3(256), 0, s, X, ld, rows, K, out,
-                           plane_stride, rows_pad, k_pad, (const unsigned *)amax);
-    } else if (kcont) {
-        const long total = (long)rows_pad * (k_pad / 8);
-        // One chunk per thread (the grid-stride loop only matters beyond 2^28
-        // chunks): a grid capped at 8192 blocks, four chunks per thread, ran
-        // 13% slower at 8192^3 (fewer loads in flight).
-        long blocks = (total + 255) / 256;
-        if (blocks > (1L << 20)) blocks = 1L << 20;
-        hipLaunchKernelGGL((split_prep_kcont<NP, FMT>), dim3((unsigned)blocks), dim3(256), 0, s, X, ld, rows, K,
-                           out, plane_stride, rows_pad, k_pad, (const unsigned *)amax);
-    } else {
-        dim3 grid((unsigned)((rows_pad + 63) / 64), (unsigned)((k_pad + 63) / 64));
-        hipLaunchKernelGGL((split_prep_rcont<NP, FMT>), grid, dim3(256), 0, s, X, ld, rows, K, out, plane_stride,
-                           rows_pad, k_pad, (const unsigned *)amax);
-    }
-    UGEMM_HIP_TRY(hipGetLastError());
-    return UGEMM_OK;
+    if (blocks > 0)
+        hipLaunchKernelGGL((split_prep_pair<NP, FMT>), dim3((unsigned)blocks), dim3(256), 0, s, jobs[0], jobs[1]);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? UGEMM_OK : hip_fail(e, "split preparation");
 }
 
 // Split-K count of the core's grid, with *kc the K chunk (whole 32-wide K tiles).
@@ -1361,72 +1401,29 @@ int run_cfg(const Gemm<float> &g, hipStream_t s) {
         return fail(UGEMM_ERR_ARG, "too many row blocks");
     int kc;
     const int splits = core_splits<CF>(g, tiles_m, tiles_n, (int)Kp, &kc);
-    const size_t ws_off = splitk_ws_offset(a_bytes + b_bytes + amax_bytes);
+    // Partial maxima only where they don't take the call beyond the scratch of
+    // the no-allocation entry.
+    const size_t base = a_bytes + b_bytes + amax_bytes, sums = splitk_ws_bytes(splits, g);
+    size_t a_parts = FMT::SCALED && side_in_parts(!g.ta, !fa, g.K) ? (size_t)kAmaxParts * Mp * sizeof(unsigned) : 0;
+    size_t b_parts = FMT::SCALED && side_in_parts(g.tb, !fb, g.K) ? (size_t)kAmaxParts * Np * sizeof(unsigned) : 0;
+    if (splitk_ws_offset(base) + sums <= UGEMM_HIP_NOALLOC_SCRATCH_BYTES &&
+        splitk_ws_offset(base + a_parts + b_parts) + sums > UGEMM_HIP_NOALLOC_SCRATCH_BYTES)
+        a_parts = b_parts = 0;
+    const size_t ws_off = splitk_ws_offset(base + a_parts + b_parts);
     void *ws = nullptr;
-    int rc = stream_alloc(&ws, ws_off + splitk_ws_bytes(splits, g), s);
+    int rc = stream_alloc(&ws, ws_off + sums, s);
     if (rc) return rc;
     E *Ap = (E *)ws, *Bp = (E *)((char *)ws + a_bytes);
     unsigned *amax_a = FMT::SCALED ? (unsigned *)((char *)ws + a_bytes + b_bytes) : nullptr;
     unsigned *amax_b = FMT::SCALED ? amax_a + Mp : nullptr;
+    unsigned *parts_a = a_parts ? (unsigned *)((char *)ws + base) : nullptr;
+    unsigned *parts_b = b_parts ? (unsigned *)((char *)ws + base + a_parts) : nullptr;
     float *part = splits > 1 ? (float *)((char *)ws + ws_off) : nullptr;
-    if (FMT::SCALED) {
-        // A fill kernel rather than a memset: callers may capture this call in a graph.
-        hipLaunchKernelGGL(fill_zero_u32, dim3((unsigned)std::min<long>((Mp + Np + 255) / 256, 1024)), dim3(256), 0,
-                           s, amax_a, Mp + Np);
-    }
-    // FP16X3 NN (A k-contiguous with K <= 8192, B row-contiguous, both on
-    // planes): A's fused row maximum + split and B's column maxima in one
-    // launch, then B's split; otherwise one preparation per operand.
-    bool merged = false;
-    if constexpr (FMT::SCALED) {
-        if (!fa && !fb && !g.ta && !g.tb && g.M > 0 && g.N > 0 && g.K > 0 && Kp <= 8192) {
-            const long kblocks = (g.K + kAmaxRcontSpan - 1) / kAmaxRcontSpan, cblocks = (g.N + 255) / 256;
-            hipLaunchKernelGGL((split_prep_rowscaled_a_amax_b<NP, FMT>), dim3((unsigned)(cblocks * kblocks + Mp / 2)),
-                               dim3(256), 0, s, g.A, g.lda, g.M, g.K, Ap, a_plane, (int)Mp, (int)Kp, amax_a,
-                               g.B, g.ldb, g.N, kblocks, amax_b, (int)(cblocks * kblocks));
-            const hipError_t e = hipGetLastError();
-            rc = e == hipSuccess ? UGEMM_OK : hip_fail(e, "split preparation");
-            if (!rc) rc = prep_operand<NP, FMT>(g.B, g.ldb, false, g.N, g.K, Bp, b_plane, (int)Np, (int)Kp, amax_b, s,
-                                                true, true);
-            merged = true;
-        }
-    }
-    if constexpr (!FMT::SCALED) {
-        if (!fa && !fb) {
-            // Both operands on planes: one preparation launch.
-            auto job = [&](const float *X, long ld, bool kcont, int rows, E *out, long plane, long rows_pad,
-                           int block0) {
-                PrepJob j{};
-                j.X = X;
-                j.ld = ld;
-                j.out = out;
-                j.plane_stride = plane;
-                j.rows = rows;
-                j.K = g.K;
-                j.rows_pad = (int)rows_pad;
-                j.k_pad = (int)Kp;
-                j.kcont = kcont;
-                j.block0 = block0;
-                j.nbx = (int)(rows_pad / 64);
-                j.amax = nullptr;
-                return j;
-            };
-            const long ka = !g.ta ? (Kp + 127) / 128 : (Kp + 63) / 64, kb = g.tb ? (Kp + 127) / 128 : (Kp + 63) / 64;
-            const long blocks_a = Mp / 64 * ka, blocks = blocks_a + Np / 64 * kb;
-            if (Mp % 64 == 0 && Np % 64 == 0 && blocks <= 0x7fffffffL) {
-                const PrepJob ja = job(g.A, g.lda, !g.ta, g.M, Ap, a_plane, Mp, 0);
-                const PrepJob jb = job(g.B, g.ldb, g.tb, g.N, Bp, b_plane, Np, (int)blocks_a);
-                hipLaunchKernelGGL((split_prep_pair<NP, FMT>), dim3((unsigned)blocks), dim3(256), 0, s, ja, jb);
-                const hipError_t e = hipGetLastError();
-                rc = e == hipSuccess ? UGEMM_OK : hip_fail(e, "split preparation");
-                merged = true;
-            }
-        }
-    }
-    if (!merged) {
-        rc = prep_operand<NP, FMT>(g.A, g.lda, !g.ta, g.M, g.K, Ap, a_plane, (int)Mp, (int)Kp, amax_a, s, !fa);
-        if (!rc) rc = prep_operand<NP, FMT>(g.B, g.ldb, g.tb, g.N, g.K, Bp, b_plane, (int)Np, (int)Kp, amax_b, s, !fb);
-    }
+    const Side sa = {g.A, g.lda, !g.ta, g.M, (int)Mp, fa ? nullptr : Ap, a_plane, amax_a, parts_a};
+    const Side sb = {g.B, g.ldb, (bool)g.tb, g.N, (int)Np, fb ? nullptr : Bp, b_plane, amax_b, parts_b};
+    // The BF16 forms need nothing of an operand that the core splits.
+    if (FMT::SCALED || !fa || !fb)
+        rc = prep_operands<NP, FMT>(sa, sb, g.K, (int)Kp, false, s);
     if (!rc) {
         const unsigned *ma = amax_a, *mb = amax_b;
 #define UGEMM_CORE(FA_, FB_) \
@@ -1494,7 +1491,8 @@ int run_cfg_conv(const Gemm<float> &g, const ConvDesc &cd, hipStream_t s) {
     if (FMT::SCALED)
         hipLaunchKernelGGL(fill_zero_u32, dim3((unsigned)std::min<long>((Mp + Np + 255) / 256, 1024)), dim3(256), 0,
                            s, amax_a, Mp + Np);
-    rc = prep_operand<NP, FMT>(g.A, g.lda, true, g.M, g.K, Ap, a_plane, (int)Mp, (int)Kp, amax_a, s);
+    rc = prep_operands<NP, FMT>(Side{g.A, g.lda, true, g.M, (int)Mp, Ap, a_plane, amax_a, nullptr}, Side{}, g.K,
+                                (int)Kp, true, s);
     if (!rc) {
         constexpr int KSPAN = 32;   // short spans: enough blocks for small images
         if (FMT::SCALED)

@@ -608,19 +608,25 @@ int default_split_variant(const ugemm_grouped_plan *p) {
     // than re-splitting (512 im2col-shaped problems, M = 32..512,
     // N = 49..3136, K = 144..4608: 4.1 ms, against 4.7 for the 4-wave
     // split-B variant and 5.8 with planes, for BF16x3).
-    double big = 0, all = 0, rows_w = 0;
+    // Plans whose 128 x 128 tiles leave a third of the CUs idle: 64 x 64 (us,
+    // 64 x 64 / 128 x 128 split-B, FP16X3 and BF16X3: 28 tiles, K 1266 76 / 87 and
+    // 54 / 65, 71 tiles, K 1845 102 / 127 and 80 / 98, 157 tiles, K 1180 99 / 117
+    // and 77 / 92; 180 tiles, K 2163 195 / 182 and 155 / 138).
+    double big = 0, all = 0, rows_w = 0, tiles = 0;
     int n_t = 0, n_n = 0;
     for (const DevProblem &q : p->probs) {
         const double f = 2.0 * q.M * q.N * q.K;
         all += f;
         if (q.M >= 128 && q.N >= 128) big += f;
         rows_w += f * ((q.M + 127) / 128);
+        if (q.K > 0) tiles += (double)((q.M + 127) / 128) * ((q.N + 127) / 128);
         if (q.M > 0 && q.N > 0) ((q.layout & 2) ? n_t : n_n)++;
     }
-    if (all == 0 || big < 0.5 * all) return 3;
+    if (all == 0 || big < 0.5 * all || 3 * tiles <= 2.0 * device_cu_count()) return 3;
     const int split_b = mfma_variant_count(p->mode) + 2;   // split-B on the 8-wave streamed 128 x 128
     if (!(n_t && n_n) && rows_w <= 4.0 * all && mfma_grouped_splits_b(p->mode, split_b)) return split_b;
-    return 1;
+    // Planes for both: the same tiles on eight waves (20 problems, BF16X3 218 us on four, 207 now; BF16X6 317 and 260).
+    return 7;
 }
 
 bool parse_t(char c, bool *t) {

@@ -94,6 +94,10 @@ struct PrepJob {
     int kcont;
     int block0, nbx;
     const unsigned *amax;   // FP16X3: the operand's row maxima (row scales), else null
+    // FP16X3, row-contiguous, one GEMM: nparts > 0: the maxima come as nparts
+    // rows of rows_pad partial maxima, and the blocks of k tile 0 write amax.
+    const unsigned *parts;
+    int nparts;
 };
 // FP16X3 grouped plans: the row-maximum jobs (out = maxima), the job of
 // each of their blocks, and the maxima buffer of all problems, zeroed before
