@@ -1,0 +1,55 @@
+"""gemv 'N' over its three ways: one thread a row, 16 waves to 64 rows in one
+launch, and in chunks of columns; rows around 64, columns around 128, the
+bounds of the choice and ragged chunks; strides, a padded leading dimension,
+beta == 0 not reading y.  Against FP64 sums (numpy.longdouble for FP64), bound
+by the length of the sum; repeated calls give the same bits."""
+import numpy as np
+import pytest
+
+import ugemm_amd as ug
+from ugemm_amd import hip
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(1, 1), (1, 128), (63, 127), (64, 128), (65, 129), (300, 768), (130, 769), (1000, 1024), (200, 1025),
+         (70, 1300), (3, 20000), (192, 17216), (4097, 333), (33000, 130), (4095, 2000), (16500, 4100)]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("beta,incx,incy,pad", [(0.0, 1, 1, 0), (0.5, 2, 3, 5)])
+def test_gemv_n(dtype, beta, incx, incy, pad):
+    wide = np.float64 if dtype == np.float32 else np.longdouble
+    eps = np.finfo(dtype).eps
+    for M, N in SIZES:
+        if M * N > 2e7 and (pad or dtype == np.float32):
+            continue
+        g = orc.rng(M + N)
+        A = orc.uniform(g, (N, M + pad)).astype(dtype)
+        A[:, M:] = np.nan
+        x = np.full(N * incx, np.nan, dtype)
+        x[::incx] = orc.uniform(g, (N,)).astype(dtype)
+        y0 = np.full(M * incy, np.nan, dtype)
+        if beta:
+            y0[::incy] = orc.uniform(g, (M,)).astype(dtype)
+        dA, dx = hip.DeviceArray.from_host(A), hip.DeviceArray.from_host(x)
+        got = []
+        print(f"{np.dtype(dtype).name} {M}x{N} beta {beta}", flush=True)
+        for _ in range(2):
+            dy = hip.DeviceArray.from_host(y0)
+            ug.gemv_dev("N", M, N, 1.5, dA, M + pad, dx, incx, beta, dy, incy, double=dtype == np.float64)
+            hip.synchronize()
+            got.append(dy.download())
+            dy.free()
+        dA.free()
+        dx.free()
+        assert got[0].tobytes() == got[1].tobytes()
+        a, xs = A[:, :M], x[::incx]
+        want = 1.5 * (xs.astype(wide) @ a.astype(wide))
+        bound = 1.5 * (np.abs(xs).astype(wide) @ np.abs(a).astype(wide))
+        if beta:
+            want = want + beta * y0[::incy].astype(wide)
+            bound = bound + beta * np.abs(y0[::incy])
+        assert np.all(np.abs(got[0][::incy] - want) <= (N + 4) * eps * bound)
+        if incy > 1:
+            assert np.all(np.isnan(np.delete(got[0], np.s_[::incy])))

@@ -15,9 +15,10 @@
 // here x uses incx.  Increments must be >= 1.  beta == 0 does not read y.
 //
 // gemv 'N' (column-major walk, A[m + n*lda] contiguous in m): threads own
-// rows m and stream down the columns; N is split over up to 64 blocks in y's
-// grid dimension, each writing a partial sum per row, and a second kernel
-// adds the partials in a fixed order (deterministic, no atomics).
+// rows m and stream down the columns, one thread a row or the 16 waves of a
+// block in turn; N is split over blocks in y's grid dimension where rows are
+// few, each writing a partial sum per row, and a second kernel adds the partials
+// in a fixed order (deterministic, no atomics).
 // gemv 'T' (A[n + m*lda] contiguous in n): one wave per output row, lanes
 // stride along n, then a wave reduction (fixed shuffle order).
 #include <algorithm>
@@ -112,15 +113,66 @@ __global__ __launch_bounds__(256) void gemv_n_kernel(int M, int N, int chunk, T 
     }
 }
 
+// The sum of 16 values of LDS, one a wave, by wave order: lane's row.
 template <typename T>
-__global__ __launch_bounds__(256) void gemv_n_reduce(int M, int splits, T alpha, const T *__restrict__ partial, T beta,
-                                                     T *__restrict__ y, long incy) {
-    const int m = blockIdx.x * 256 + threadIdx.x;
-    if (m >= M) return;
+__device__ __forceinline__ T waves_sum(T (*part)[64], int lane) {
+    T s = part[0][lane];
+#pragma unroll
+    for (int w = 1; w < 16; ++w) s += part[w][lane];
+    return s;
+}
+
+// The same by 16 waves: block (bx, by) covers rows [64*bx, +64), wave w the
+// columns by*chunk + w, + 16, ..., eight loads in flight; the waves' sums are
+// added through LDS.
+template <typename T>
+__global__ __launch_bounds__(1024) void gemv_n_waves(int M, int N, int chunk, T alpha, const T *__restrict__ A, long lda,
+                                                     const T *__restrict__ x, long incx, T beta, T *__restrict__ y,
+                                                     long incy, T *__restrict__ partial) {
+    __shared__ T part[16][64];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m = blockIdx.x * 64 + lane;
+    const int n1 = min(N, ((int)blockIdx.y + 1) * chunk);
+    const T *p = A + min(m, M - 1);   // rows past the last read it; nothing is stored for them
+    T s[8] = {};
+    int n = blockIdx.y * chunk + w;
+    for (; n + 112 < n1; n += 128) {
+        T a[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a[j] = p[(long)(n + 16 * j) * lda];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s[j] = fma(a[j], x[(long)(n + 16 * j) * incx], s[j]);
+    }
+    for (; n < n1; n += 16) s[0] = fma(p[(long)n * lda], x[(long)n * incx], s[0]);
+    part[w][lane] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+    __syncthreads();
+    if (w || m >= M) return;
+    const T v = waves_sum(part, lane);
+    if (partial) {
+        partial[(long)blockIdx.y * M + m] = v;
+    } else {
+        T *py = y + (long)m * incy;
+        *py = beta == T(0) ? alpha * v : fma(alpha, v, beta * *py);
+    }
+}
+
+// 64 rows a block, the partials dealt to 16 waves (one thread a row added up
+// to 64 of them one after the other).
+template <typename T>
+__global__ __launch_bounds__(1024) void gemv_n_reduce(int M, int splits, T alpha, const T *__restrict__ partial, T beta,
+                                                      T *__restrict__ y, long incy) {
+    __shared__ T part[16][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int m = blockIdx.x * 64 + lane;
     T s = 0;
-    for (int k = 0; k < splits; ++k) s += partial[(long)k * M + m];
+    if (m < M)
+        for (int k = w; k < splits; k += 16) s += partial[(long)k * M + m];
+    part[w][lane] = s;
+    __syncthreads();
+    if (w || m >= M) return;
+    const T v = waves_sum(part, lane);
     T *py = y + (long)m * incy;
-    *py = beta == T(0) ? alpha * s : fma(alpha, s, beta * *py);
+    *py = beta == T(0) ? alpha * v : fma(alpha, v, beta * *py);
 }
 
 // gemv 'T': 4 waves per block, one row m per wave.
@@ -215,28 +267,35 @@ int gemv(char trans, int M, int N, T alpha, const T *A, int lda, const T *x, int
         return UGEMM_OK;
     }
     // 'N': enough blocks to cover the chip -- split N when M alone is too small.
+    // 16 waves to 64 rows, in one launch while a wave's columns are few (its
+    // loads are a chain of N / 128 latencies); else N in chunks of blocks.  One
+    // thread a row where the columns are too few for that, and for matrices
+    // that keep HBM busy either way.  us, thread a row / waves, one launch /
+    // waves, chunks, FP32: 128x256 9.9 / 6.5 / 10.0, 1000x1000 9.7 / 8.9 / 9.7,
+    // 720x3068 11.7 / 23.1 / 9.5, 192x17216 26.8 / 109 / 9.4, 4096x4096 15.5 /
+    // 27.6 / 14.6, 20000x5000 77 / 83 / 83; FP64: 384x742 10.2 / 8.8 / 10.2,
+    // 1000x1000 11.1 / 11.9 / 10.1, 8192x8192 89 / 115 / 97.
     const int cus = device_cu_count();
-    const int mblocks = (M + 255) / 256;
-    int splits = std::max(1, std::min(64, (4 * cus + mblocks - 1) / mblocks));
-    splits = std::min(splits, std::max(1, N / 64));
+    const bool waves = N >= 128 && (M < 4096 || (double)M * N * sizeof(T) <= (double)(256u << 20));
+    const int rows = waves ? 64 : 256, mblocks = (M + rows - 1) / rows;
+    int splits;
+    if (waves) splits = N <= (sizeof(T) == 4 ? 1024 : 768) ? 1 : std::min({256, 2 * cus / mblocks, N / 128});
+    else splits = std::min({64, (4 * cus + mblocks - 1) / mblocks, N / 64});
+    splits = std::max(1, splits);
     const int chunk = (N + splits - 1) / splits;
     splits = (N + chunk - 1) / chunk;
-    if (splits == 1) {
-        hipLaunchKernelGGL(gemv_n_kernel<T>, dim3((unsigned)mblocks, 1), dim3(256), 0, s, M, N, chunk, alpha, A,
-                           (long)lda, x, (long)incx, beta, y, (long)incy, (T *)nullptr);
-        UGEMM_HIP_TRY(hipGetLastError());
-        return UGEMM_OK;
-    }
     void *ws = nullptr;
-    int rc = stream_alloc(&ws, (size_t)splits * M * sizeof(T), s);
-    if (rc) return rc;
-    hipLaunchKernelGGL(gemv_n_kernel<T>, dim3((unsigned)mblocks, (unsigned)splits), dim3(256), 0, s, M, N, chunk, alpha,
-                       A, (long)lda, x, (long)incx, beta, y, (long)incy, (T *)ws);
-    hipLaunchKernelGGL(gemv_n_reduce<T>, dim3((unsigned)mblocks), dim3(256), 0, s, M, splits, alpha, (const T *)ws, beta,
-                       y, (long)incy);
-    hipError_t e = hipGetLastError();
-    rc = e == hipSuccess ? UGEMM_OK : hip_fail(e, "gemv launch");
-    const int rc2 = stream_free(ws, s);
+    if (splits > 1)
+        if (const int rc = stream_alloc(&ws, (size_t)splits * M * sizeof(T), s)) return rc;
+    hipLaunchKernelGGL(waves ? gemv_n_waves<T> : gemv_n_kernel<T>, dim3((unsigned)mblocks, (unsigned)splits),
+                       dim3(waves ? 1024 : 256), 0, s, M, N, chunk, alpha, A, (long)lda, x, (long)incx, beta, y,
+                       (long)incy, (T *)ws);
+    if (splits > 1)
+        hipLaunchKernelGGL(gemv_n_reduce<T>, dim3((unsigned)((M + 63) / 64)), dim3(1024), 0, s, M, splits, alpha,
+                           (const T *)ws, beta, y, (long)incy);
+    const hipError_t e = hipGetLastError();
+    const int rc = e == hipSuccess ? UGEMM_OK : hip_fail(e, "gemv launch");
+    const int rc2 = splits > 1 ? stream_free(ws, s) : UGEMM_OK;
     return rc ? rc : rc2;
 }
 
