@@ -492,7 +492,7 @@ __device__ __forceinline__ float im2col_at(const ConvDesc &cd, int n, int k, int
 }
 
 // Planes of the im2col operand, gathered straight from the image (no im2col
-// matrix in HBM): one thread per 8 k of one pixel n, as split_prep_kcont.
+// matrix in HBM): one thread per 8 k of one pixel n.
 template <int NP, class FMT>
 __global__ __launch_bounds__(256) void split_prep_im2col(ConvDesc cd, int N, int K, typename FMT::E *__restrict__ out,
                                                          long plane_stride, int rows_pad, int k_pad,
