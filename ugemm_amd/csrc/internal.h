@@ -142,6 +142,14 @@ int device_cu_count();
 // Variant tables: each family exposes a count, names, and a launcher.
 int fp32_variant_count();
 const char *fp32_variant_name(int v);
+// A tile shape's price: us per 128x128 of C (any unit common to the shapes), and
+// the latency of a CU's tiles, in tiles.  cheapest_tile: the shape whose fullest
+// CU is done first, or v unless one is 5% ahead; bits of skip leave shapes out.
+struct TileCost {
+    int bm, bn;
+    double us, lone;
+};
+int cheapest_tile(const TileCost *c, int n, unsigned skip, int v, int M, int N);
 int fp32_pick_variant(const Gemm<float> &g);
 int launch_fp32(const Gemm<float> &g, int variant, hipStream_t s);
 // FP32 SGEMM on FP32 MFMA (sgemm_mfma32.hip).

@@ -191,17 +191,27 @@ int fp32_pick_variant(const Gemm<float> &g) {
     const int cus = device_cu_count();
     const long t128x256 = (long)((g.M + 127) / 128) * ((g.N + 255) / 256);
     const long t256x128 = (long)((g.M + 255) / 256) * ((g.N + 127) / 128);
-    if (!g.ta && !g.tb && t256x128 >= 2L * cus) return 4;
-    if (t128x256 >= 2L * cus) return 5;
     const long t128 = (long)((g.M + 127) / 128) * ((g.N + 127) / 128);
-    if (t128 >= 2L * cus) return 0;
-    if (2 * t128x256 >= cus && g.K >= 1024 && g.splits != 1) return 5;
-    const long t64 = (long)((g.M + 63) / 64) * ((g.N + 63) / 64);
-    if (t64 > 2L * cus) {
-        if (g.M >= 4 * g.N) return 2;
-        if (g.N >= 4 * g.M) return 3;
+    const bool nn = !g.ta && !g.tb;
+    int v;
+    if (nn && t256x128 >= 2L * cus) v = 4;
+    else if (t128x256 >= 2L * cus) v = 5;
+    else if (t128 >= 2L * cus) v = 0;
+    else if (2 * t128x256 >= cus && g.K >= 1024 && g.splits != 1) return 5;
+    else {
+        const long t64 = (long)((g.M + 63) / 64) * ((g.N + 63) / 64);
+        v = t64 > 2L * cus && g.M >= 4 * g.N ? 2 : t64 > 2L * cus && g.N >= 4 * g.M ? 3 : 1;
     }
-    return 1;
+    if (t128 <= cus) return v;
+    // The CU with one tile more than the others sets the time: 583 tiles of
+    // 128x128 (6662x1408x2930 NT) are three on some CUs and two on most, 890 us,
+    // where 1166 of 128x64 are five and four, 756.  So another shape where the
+    // tiles of its fullest CU are 5% cheaper (us per 128x128 and 1000 of K, a
+    // lone tile's latency in tiles; fitted to all six over 60 sizes).  Over those
+    // sizes (sides 720..16384, K 256..5800) 1.11 times as fast on average.
+    static const TileCost cost[6] = {{128, 128, 85, 0.27}, {64, 64, 95, 0.9},   {128, 64, 87, 0.75},
+                                     {64, 128, 87, 0.75},  {256, 128, 82, 0.23}, {128, 256, 82, 0.2}};
+    return cheapest_tile(cost, 6, 1 << (nn ? 5 : 4), v, g.M, g.N);
 }
 
 int launch_conv_fp32(const Gemm<float> &g, const ConvDesc &cd, int variant, hipStream_t s) {

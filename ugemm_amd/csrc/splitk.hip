@@ -86,6 +86,21 @@ bool deal_k(long tiles, int K, double us_per_k1000, int grouped, size_t c_bytes,
     return tiles <= grouped * cus && groups <= best;
 }
 
+int cheapest_tile(const TileCost *c, int n, unsigned skip, int v, int M, int N) {
+    const long cus = device_cu_count();
+    auto tiles = [&](const TileCost &t) { return (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn); };
+    auto us = [&](const TileCost &t) { return t.us * t.bm * t.bn * ((double)((tiles(t) + cus - 1) / cus) + t.lone); };
+    double best = 0.95 * us(c[v]);
+    for (int i = 0; i < n; ++i) {
+        if (skip >> i & 1 || tiles(c[i]) <= cus) continue;   // at most one tile a CU: split counts decide
+        if (const double t = us(c[i]); t < best) {
+            best = t;
+            v = i;
+        }
+    }
+    return v;
+}
+
 int launch_splitk_reduce_f32(int M, int N, int splits, float alpha, const float *ws, float beta, float *C, long ldc,
                              const Epilogue &epi, hipStream_t s) {
     return reduce<float>(M, N, splits, alpha, ws, beta, C, ldc, epi, s);
