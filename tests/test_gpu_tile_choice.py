@@ -43,3 +43,43 @@ def test_tile_choice(mode, ta, tb):
         ok, worst = orc.check_bound(got[0][:, :N], want, scale, orc.tolerance(K + 2))
         assert ok, f"{M}x{N}x{K}: {worst:.3g}"
         assert np.array_equal(got[0][:, N:], c0[:, N:], equal_nan=True)
+
+
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
+def test_tile_choice_fp64(ta, tb):
+    for M, N, K in [(2050, 2049, 33), (770, 5500, 50), (6240, 808, 40)]:
+        case = Case("R", ta, tb, M, N, K, 1.5, 0.5, seed=M, dtype=np.float64, pad=1)
+        dA, dB, dC = (hip.DeviceArray.from_host(x) for x in (case.A, case.B, case.C0))
+        print(f"fp64 {ta}{tb} {M}x{N}x{K}", flush=True)
+        ug.dgemm_dev("R", ta, tb, M, N, K, 1.5, dA, case.lda, dB, case.ldb, 0.5, dC, case.ldc)
+        hip.synchronize()
+        got = dC.download()
+        for d in (dA, dB, dC):
+            d.free()
+        Aop = case.A[:, :M].T if ta == "T" else case.A[:, :K]
+        Bop = case.B[:, :K].T if tb == "T" else case.B[:, :N]
+        want = 1.5 * (Aop @ Bop) + 0.5 * case.C0[:, :N]
+        scale = 1.5 * (np.abs(Aop) @ np.abs(Bop)) + 0.5 * np.abs(case.C0[:, :N])
+        # Both sides are FP64 sums of K products: twice the bound of one.
+        assert np.all(np.abs(got[:, :N] - want) <= 2 * (K + 4) * np.finfo(np.float64).eps * scale)
+        assert np.array_equal(got[:, N:], case.C0[:, N:])
+
+
+@pytest.mark.parametrize("mode", [ug.MODE_BF16X1, ug.MODE_BF16X3, ug.MODE_FP16X3])
+def test_large_tiles_a_little_over(mode):
+    """17 x 16 tiles of 256x256: the automatic choice and the large tile give the same bits."""
+    M, N, K = 4200, 4090, 70
+    case = Case("R", "N", "T", M, N, K, 1.0, 0.0, seed=mode)
+    dA, dB = hip.DeviceArray.from_host(case.A), hip.DeviceArray.from_host(case.B)
+    got = []
+    for variant in (-1, 6):
+        ug.force_variant(mode, variant)
+        dC = hip.DeviceArray.from_host(np.full((M, N), np.nan, np.float32))
+        ug.sgemm_dev("R", "N", "T", M, N, K, 1.0, dA, K, dB, K, 0.0, dC, N, mode=mode)
+        hip.synchronize()
+        got.append(dC.download())
+        dC.free()
+    ug.force_variant(mode, -1)
+    dA.free()
+    dB.free()
+    assert got[0].tobytes() == got[1].tobytes()

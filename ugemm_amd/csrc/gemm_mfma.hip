@@ -1656,7 +1656,18 @@ int mfma_pick_variant(const Gemm<float> &g, int mode, bool fusable, int *splits)
     // three planes run fastest on the streamed V6, one plane on the
     // 16-wave V5.
     const int big = fusable && np <= 2 && (tn <= 2 || tm <= 2) ? 4 : (np >= 2 ? 6 : 5);
-    if (tm * tn >= cus) return big;
+    if (tm * tn >= cus) {
+        // A few tiles more than CUs: the second round is nearly empty, and V7's
+        // 128x128 tiles, 1.4 times as dear by area, come out ahead (us, V6 or V5 /
+        // V7, 289 tiles: 4200x4200x2048 BF16X3 294 / 244, FP16X3 325 / 262, BF16X1
+        // 139 / 129; 360 tiles, 5000x4500x1500 222 / 210, 384 287 / 293).  Not for
+        // three planes, whose large tile is half as wide.  Same bits.
+        const double t128 = (double)((g.M + 127) / 128) * ((g.N + 127) / 128);
+        if (np <= 2 && big != 4 && !stream_alloc_is_static() &&
+            1.4 * 0.25 * std::ceil(t128 / cus) < 0.95 * ((tm * tn + cus - 1) / cus))
+            return 7;
+        return big;
+    }
     const int fixed = mfma_fixed_variant(g);
     if (*splits > 0 || g.K <= 0) return fixed;
     // Fewer: tile and splits together.  493x2304x34854 BF16X3 ran 288 blocks
