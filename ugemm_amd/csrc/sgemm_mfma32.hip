@@ -125,6 +125,10 @@ int launch_small(const Gemm<float> &g, hipStream_t s) {
         return launch_cfg<V3S16>(h, s);
     }
     if (t32 <= 2 * cus && g.K <= 2048) return launch_cfg<V3S8>(h, s);
+    // One tile a CU and a K of a few steps: a chain of latencies that deal_k,
+    // fitted to longer ones, prices too low (us, one group / four: 4440x192x128
+    // 11.1 / 8.8, 1000x1000x200 15.3 / 11.3, 4440x192x256 16.5 / 11.9, K 64 8.5 / 8.5).
+    if (t64 <= cus && g.K > 64 && g.K <= 512) return launch_cfg<V3K4>(h, s);
     return deal_k(t64, g.K, 21.0, 2, sizeof(*g.C) * g.M * g.N, &h.splits) ? (h.splits = 1, launch_cfg<V3K4>(h, s)) : launch_cfg<V3>(h, s);
 }
 
