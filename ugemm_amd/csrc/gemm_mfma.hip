@@ -687,10 +687,16 @@ __global__ __launch_bounds__(CF::NT) void split_nt_core(int M_, int N_, int Kp_,
                   "row-contiguous fusion: one or two rows per thread");
     V8 pa[FA ? 1 : A_CH], pb[FB ? 1 : B_CH];
     float fa[FA ? FA_CH : 1][8], fb[FB ? FB_CH : 1][8];
+    // A grouped problem with K == 0 or alpha == 0 (handed over with K = 0) still
+    // gets the two K tiles of its zero planes, but has no line of B to read in
+    // the place of one past K, and B may be NULL: the stage is zeros, without a
+    // load.  Uniform over the block.  A single GEMM never gets here with K == 0.
+    const bool no_k = GR && K == 0;
     // Row-contiguous source: rows [r, r+RW) of k-lines k .. k+7 into v[i][j]
     // (row r+i, k+j).  RW is 1 or 2 (stage rows per thread).  Rows past the
     // last read it in their place, without a branch: nothing stores their
-    // results.  kin: the stage ends inside K (uniform); else values past K are 0.
+    // results.  kin: the stage ends inside K (uniform); else values past K are 0
+    // (K >= 1: the last line of K is read in their place).
     // (Guards on rows and k, a branch and a wait each, made the tiles at the
     // edge up to twice as long: 32767x512x1024 TN BF16X3 took 225 us, now 117.)
     auto load_rc = [&](const float *X, long ld, int rows, int r, int k, auto &v, bool kin) {
@@ -710,6 +716,9 @@ __global__ __launch_bounds__(CF::NT) void split_nt_core(int M_, int N_, int Kp_,
             p += (long)k * ld;
 #pragma unroll
             for (int j = 0; j < 8; ++j) line(p + (long)j * ld, j);
+        } else if (no_k) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[0][j] = v[RW - 1][j] = 0.0f;
         } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j) line(p + (long)min(k + j, K - 1) * ld, j);
@@ -726,6 +735,9 @@ __global__ __launch_bounds__(CF::NT) void split_nt_core(int M_, int N_, int Kp_,
             const f32x4u x0 = *reinterpret_cast<const f32x4u *>(p + k);
             const f32x4u x1 = *reinterpret_cast<const f32x4u *>(p + k + 4);
             v[0] = x0.x; v[1] = x0.y; v[2] = x0.z; v[3] = x0.w; v[4] = x1.x; v[5] = x1.y; v[6] = x1.z; v[7] = x1.w;
+        } else if (no_k) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = 0.0f;
         } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {

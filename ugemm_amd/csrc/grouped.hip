@@ -520,7 +520,7 @@ int build_split_schedule(ugemm_grouped_plan *p, int v) {
         if (!split_b) add_job(q.B, q.ldb, tb, q.N, q.K, (int)Np, (int)Kp, bo, b_plane, am_b);
         GroupedSplitProblem g{};
         if (split_b) {
-            // FP32 B read by the core; K == 0 (alpha == 0) reads nothing.
+            // FP32 B read by the core; with K == 0 (alpha == 0: B may be NULL) it loads nothing.
             g.Bf = q.B;
             g.ldb = q.ldb;
             g.K = q.K;
