@@ -109,3 +109,18 @@ def test_finish_gives_the_blocks_back_and_calls_go_on(calls):
     ug.finish()
     rounds(calls[:3], 6, True, wrong)
     assert not wrong, wrong[:5]
+
+
+def test_more_live_streams_than_kept_blocks(calls):
+    """70 streams alive at once, three rounds of calls on all of them before
+    any is waited for: streams without a kept block allocate as they go."""
+    streams = [hip.Stream() for _ in range(70)]
+    picked = [calls[i % len(calls)] for i in range(len(streams))]
+    outs = [hip.DeviceArray(c.case.C0.shape, np.float32) for c in picked]
+    for _ in range(3):
+        for c, out, s in zip(picked, outs, streams):
+            c.run(out, s)
+    for c, out, s in zip(picked, outs, streams):
+        s.synchronize()
+        assert out.download().tobytes() == c.want
+        s.destroy()
