@@ -124,3 +124,21 @@ def test_more_live_streams_than_kept_blocks(calls):
         s.synchronize()
         assert out.download().tobytes() == c.want
         s.destroy()
+
+
+def test_finish_beside_running_calls(calls):
+    """finish() while calls still run on the caller's stream: their blocks are
+    given back only behind them, so other streams' calls change nothing."""
+    s, others = hip.Stream(), [hip.Stream() for _ in range(4)]
+    outs = [hip.DeviceArray(c.case.C0.shape, np.float32) for c in calls]
+    more = [hip.DeviceArray(calls[5].case.C0.shape, np.float32) for _ in others]
+    for c, out in zip(calls, outs):
+        c.run(out, s)
+    ug.finish()
+    for o, out in zip(others, more):
+        calls[5].run(out, o)
+    hip.synchronize()
+    assert [out.download().tobytes() == c.want for c, out in zip(calls, outs)] == [True] * len(calls)
+    assert all(out.download().tobytes() == calls[5].want for out in more)
+    for o in others + [s]:
+        o.destroy()

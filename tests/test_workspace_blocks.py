@@ -92,3 +92,18 @@ def test_large_blocks_never_wait(fake):
         once(200 * MIB, 101)                      # beyond a kept block's size
         assert count()[2] == 0 and size("bytes").value == 4 * 120 * MIB
         """)
+
+
+def test_idle_blocks_are_released_after_a_wait_and_kept_if_refused(fake):
+    run(fake, """
+        release = L._ZN5ugemm22release_idle_workspaceEv
+        a, b = once(3 * MIB, 101), once(4 * MIB, 0)
+        p = call(MIB, 102)                        # in use: stays
+        counter("refuse").value = 1
+        assert release() == 0 and once(3 * MIB, 101) == a and once(4 * MIB, 0) == b
+        c = call(9 * MIB, 101)                    # a is not replaced: the call has memory of its own
+        counter("refuse").value = 0
+        assert free(c, 101) == 0 and once(2 * MIB, 101) == a
+        assert release() == 2 and size("bytes").value == MIB
+        assert free(p, 102) == 0 and release() == 1 and size("bytes").value == 0
+        """)

@@ -284,11 +284,17 @@ void release_staging();
 // ---- device scratch (runtime.hip) ----
 // Stream-ordered workspace for the operand-preparation kernels: allocated
 // from the device's default memory pool on stream s (which keeps freed
-// blocks for reuse), released in stream order after the consuming kernel.
-// This thread is in a no-allocation call: stream_alloc gives from the static scratch.
-bool stream_alloc_is_static();
+// blocks for reuse) or kept from the stream's last call, released in stream
+// order after the consuming kernel.
 int stream_alloc(void **ptr, size_t bytes, hipStream_t s);
 int stream_free(void *ptr, hipStream_t s);
+// This thread is in a no-allocation call: stream_alloc gives from the static scratch.
+bool stream_alloc_is_static();
+// Frees the kept blocks that no call is using, after a wait for their devices
+// (hipFree itself does not wait for kernels that use such memory); a block
+// whose device cannot be waited for, or whose free is refused (another thread
+// captures a graph), is kept.  Returns how many were freed.
+int release_idle_workspace();
 
 }  // namespace ugemm
 

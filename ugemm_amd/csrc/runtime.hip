@@ -163,10 +163,10 @@ static thread_local ScratchArena *t_arena = nullptr;
 //
 // A block never goes to another stream.  Only its own stream's end says when it
 // may be written: hipFree does not wait for kernels that still use such memory
-// (0.8 us beside 9 ms of work on the stream), an event recorded behind the last use cannot be
-// asked once its stream is destroyed (hipEventQuery then fails for good), and a
-// wait for the device would make a call synchronous, or hang it beside a kernel
-// that waits for the host.  So streams that come when the places or the bytes
+// (0.8 us beside 9 ms of work on the stream), an event recorded behind the last
+// use cannot be asked once its stream is destroyed (hipEventQuery then fails for
+// good), and a wait for the device would make a call synchronous, or hang it
+// beside a kernel that waits for the host.  So streams that come when the places or the bytes
 // are taken, also by streams that are gone, allocate as if nothing were kept.
 // The last places and 128 MiB are the null streams'.  us of host time a call,
 // FP32 256x256x4096 over 40 streams in turn, kept / not: 7.5 / 20-24.
@@ -180,6 +180,7 @@ struct WsBlock {
 constexpr int kWsBlocks = 64, kWsNull = 8;
 constexpr size_t kWsMost = (size_t)128 << 20, kWsTotal = (size_t)512 << 20;   // a block; all blocks
 constexpr unsigned long long kNullStream = ~0ull;
+
 // Guards the three below.  A busy block is its call's alone; no HIP call is made
 // with the mutex held.
 static std::mutex g_ws_mu;
@@ -209,24 +210,44 @@ static void ws_clear(WsBlock &b) {
     b = WsBlock();
 }
 
-// Gives the idle blocks back to the runtime.  hipFree waits for the work that
-// may still use them.
-static void ws_release_idle() {
-    for (WsBlock &b : g_ws) {
-        {
-            std::lock_guard<std::mutex> lk(g_ws_mu);
-            if (!b.p || b.busy) continue;
-            b.busy = true;
+// A busy block that goes on as before.
+static void ws_keep(WsBlock &b) {
+    (void)hipGetLastError();
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    b.busy = false;
+}
+
+int release_idle_workspace() {
+    int home = 0, waited = -1, released = 0;
+    (void)hipGetDevice(&home);
+    bool mine[kWsBlocks];   // busy from here on: no further call writes them
+    {
+        std::lock_guard<std::mutex> lk(g_ws_mu);
+        for (int i = 0; i < kWsBlocks; ++i) {
+            mine[i] = g_ws[i].p && !g_ws[i].busy;
+            g_ws[i].busy |= mine[i];
         }
-        (void)hipFree(b.p);
-        ws_clear(b);
     }
+    for (int i = 0; i < kWsBlocks; ++i) {
+        if (!mine[i]) continue;
+        WsBlock &b = g_ws[i];
+        if (waited != b.device && hipSetDevice(b.device) == hipSuccess && hipDeviceSynchronize() == hipSuccess)
+            waited = b.device;
+        if (waited == b.device && hipFree(b.p) == hipSuccess) {
+            ws_clear(b);
+            ++released;
+        } else {
+            ws_keep(b);
+        }
+    }
+    (void)hipSetDevice(home);
+    return released;
 }
 
 // A block for `bytes` on stream (device, id), now busy: an idle one of the
 // stream; or, with p null, a place for one of b->size bytes, free or with the
-// stream's own that is too small (*old: its memory); or null.
-static WsBlock *ws_take(size_t bytes, int device, unsigned long long id, void **old) {
+// stream's own that is too small (*old); or null.
+static WsBlock *ws_take(size_t bytes, int device, unsigned long long id, WsBlock *old) {
     const size_t size = (bytes + (1u << 20) - 1) >> 20 << 20;
     const bool null_stream = id == kNullStream;
     WsBlock *best = nullptr, *own = nullptr, *place = nullptr;
@@ -251,7 +272,7 @@ static WsBlock *ws_take(size_t bytes, int device, unsigned long long id, void **
     if (!place || g_ws_bytes - place->size + size > (null_stream ? kWsTotal : kWsTotal - kWsMost)) return nullptr;
     g_ws_used += !place->size;
     g_ws_bytes += size - place->size;
-    *old = place->p;
+    *old = *place;
     *place = WsBlock{nullptr, size, device, id, true};
     return place;
 }
@@ -273,13 +294,18 @@ int stream_alloc(void **ptr, size_t bytes, hipStream_t s) {
     }
     int device = 0;
     unsigned long long id = 0;
-    void *old = nullptr;
-    WsBlock *b = bytes <= kWsMost && ws_key(s, &device, &id) ? ws_take(bytes, device, id, &old) : nullptr;
+    WsBlock old, *b = bytes <= kWsMost && ws_key(s, &device, &id) ? ws_take(bytes, device, id, &old) : nullptr;
     if (b && b->p) {
         *ptr = b->p;
         return UGEMM_OK;
     }
-    if (old) (void)hipFreeAsync(old, s);   // this stream's: ordered after its last use
+    if (old.p && hipFreeAsync(old.p, s) != hipSuccess) {   // this stream's: ordered after its last use
+        (void)hipGetLastError();
+        std::lock_guard<std::mutex> lk(g_ws_mu);
+        g_ws_bytes += old.size - b->size;
+        *b = old;   // idle, as it was
+        b = nullptr;
+    }
     const hipError_t e = hipMallocAsync(ptr, b ? b->size : bytes, s);
     if (e != hipSuccess) {
         if (b) ws_clear(*b);
@@ -854,7 +880,7 @@ void ugemm_hip_finish(void) {
     if (!g_dev.ready) return;
     (void)hipSetDevice(g_dev.device);
     if (g_dev.stream) (void)hipStreamSynchronize(g_dev.stream);
-    ws_release_idle();
+    (void)release_idle_workspace();
     release_staging();
     if (g_dev.staging) (void)hipFree(g_dev.staging);
     if (g_dev.stream) (void)hipStreamDestroy(g_dev.stream);
