@@ -57,3 +57,5 @@ int hipFree(void *p) {
 int hipDeviceSynchronize(void) { return fake_working = 0; }
 int hipSetDevice(int device) { return device; }
 int hipGetLastError(void) { return 0; }
+int hipDeviceGetDefaultMemPool(void **pool, int device) { return *pool = NULL, device; }
+int hipMemPoolTrimTo(void *pool, size_t keep) { return pool || keep; }

@@ -107,3 +107,20 @@ def test_idle_blocks_are_released_after_a_wait_and_kept_if_refused(fake):
         assert release() == 2 and size("bytes").value == MIB
         assert free(p, 102) == 0 and release() == 1 and size("bytes").value == 0
         """)
+
+
+@pytest.mark.parametrize("large", [100, 300])
+def test_a_call_out_of_memory_takes_back_the_idle_blocks(fake, large):
+    """What fits without kept blocks fits beside them: of a size that is kept
+    and of one that is not."""
+    run(fake, f"""
+        size("limit").value = 350 * MIB
+        for s in (101, 102, 0):
+            once(100 * MIB, s)
+        p = call(MIB, 103)                        # in use: stays
+        q = call({large} * MIB, 104)
+        assert count()[2] == 3 and size("bytes").value == {large + 1} * MIB
+        call(400 * MIB, 105, status=-3)           # nothing left to give back
+        assert free(q, 104) == 0 and free(p, 103) == 0
+        once(100 * MIB, 101)
+        """)

@@ -188,6 +188,11 @@ static WsBlock g_ws[kWsBlocks];
 static int g_ws_used = 0;        // places
 static size_t g_ws_bytes = 0;
 
+static bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
 // The key of a stream that keeps blocks, or false.
 static bool ws_key(hipStream_t s, int *device, unsigned long long *id) {
     if (s == hipStreamPerThread || hipGetDevice(device) != hipSuccess) return false;
@@ -197,9 +202,7 @@ static bool ws_key(hipStream_t s, int *device, unsigned long long *id) {
     }
     typedef hipError_t (*GetId)(hipStream_t, unsigned long long *);
     static const GetId get_id = (GetId)dlsym(RTLD_DEFAULT, "hipStreamGetId");   // thread-safe initialisation
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (!get_id || hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return false;
-    return get_id(s, id) == hipSuccess;
+    return get_id && !capturing(s) && get_id(s, id) == hipSuccess;
 }
 
 // Frees a busy block's place (its memory is gone).
@@ -306,8 +309,17 @@ int stream_alloc(void **ptr, size_t bytes, hipStream_t s) {
         *b = old;   // idle, as it was
         b = nullptr;
     }
-    const hipError_t e = hipMallocAsync(ptr, b ? b->size : bytes, s);
+    hipError_t e = hipMallocAsync(ptr, b ? b->size : bytes, s);
+    if (e == hipErrorOutOfMemory && !capturing(s) && release_idle_workspace() > 0) {
+        // The idle blocks may be what is missing: free, and out of the pool.
+        (void)hipGetLastError();
+        hipMemPool_t pool;
+        if (hipGetDevice(&device) == hipSuccess && hipDeviceGetDefaultMemPool(&pool, device) == hipSuccess)
+            (void)hipMemPoolTrimTo(pool, 0);
+        e = hipMallocAsync(ptr, b ? b->size : bytes, s);
+    }
     if (e != hipSuccess) {
+        *ptr = nullptr;
         if (b) ws_clear(*b);
         return hip_fail(e, "hipMallocAsync(workspace)");
     }
