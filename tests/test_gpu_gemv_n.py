@@ -53,3 +53,22 @@ def test_gemv_n(dtype, beta, incx, incy, pad):
         assert np.all(np.abs(got[0][::incy] - want) <= (N + 4) * eps * bound)
         if incy > 1:
             assert np.all(np.isnan(np.delete(got[0], np.s_[::incy])))
+
+
+def test_gemv_n_of_nearly_2_to_the_31_columns():
+    """Chunk bounds beyond INT_MAX: one row of 2^31 - 100 ones (17 GB with x).
+    The blocks' sums are exact; at most 32 roundings follow, each by half a
+    step of the total (64) or less."""
+    N = 2 ** 31 - 100
+    ones, block = [hip.DeviceArray(N, np.float32) for _ in range(2)], np.ones(1 << 24, np.float32)
+    for d in ones:
+        hip.check(hip.lib().hipMemcpy(d.ptr, block.ctypes.data, block.nbytes, hip.H2D), "fill")
+        for at in range(block.size, N, block.size):
+            hip.check(hip.lib().hipMemcpy(d.at(at), d.ptr, 4 * min(block.size, N - at), hip.D2D), "fill")
+    dy = hip.DeviceArray(1, np.float32)
+    ug.gemv_dev("N", 1, N, 1.0, ones[0], 1, ones[1], 1, 0.0, dy, 1)
+    hip.synchronize()
+    got = float(dy.download()[0])
+    for d in ones:
+        d.free()
+    assert abs(got - N) <= 32 * 64, got

@@ -132,18 +132,18 @@ __global__ __launch_bounds__(1024) void gemv_n_waves(int M, int N, int chunk, T 
     __shared__ T part[16][64];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m = blockIdx.x * 64 + lane;
-    const int n1 = min(N, ((int)blockIdx.y + 1) * chunk);
+    const long n0 = (long)blockIdx.y * chunk, n1 = min((long)N, n0 + chunk);   // long: N may reach INT_MAX
     const T *p = A + min(m, M - 1);   // rows past the last read it; nothing is stored for them
     T s[8] = {};
-    int n = blockIdx.y * chunk + w;
+    long n = n0 + w;
     for (; n + 112 < n1; n += 128) {
         T a[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) a[j] = p[(long)(n + 16 * j) * lda];
+        for (int j = 0; j < 8; ++j) a[j] = p[(n + 16 * j) * lda];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) s[j] = fma(a[j], x[(long)(n + 16 * j) * incx], s[j]);
+        for (int j = 0; j < 8; ++j) s[j] = fma(a[j], x[(n + 16 * j) * incx], s[j]);
     }
-    for (; n < n1; n += 16) s[0] = fma(p[(long)n * lda], x[(long)n * incx], s[0]);
+    for (; n < n1; n += 16) s[0] = fma(p[n * lda], x[n * incx], s[0]);
     part[w][lane] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
     __syncthreads();
     if (w || m >= M) return;
@@ -282,8 +282,8 @@ int gemv(char trans, int M, int N, T alpha, const T *A, int lda, const T *x, int
     if (waves) splits = N <= (sizeof(T) == 4 ? 1024 : 768) ? 1 : std::min({256, 2 * cus / mblocks, N / 128});
     else splits = std::min({64, (4 * cus + mblocks - 1) / mblocks, N / 64});
     splits = std::max(1, splits);
-    const int chunk = (N + splits - 1) / splits;
-    splits = (N + chunk - 1) / chunk;
+    const int chunk = (int)(((long)N + splits - 1) / splits);
+    splits = (int)(((long)N + chunk - 1) / chunk);
     void *ws = nullptr;
     if (splits > 1)
         if (const int rc = stream_alloc(&ws, (size_t)splits * M * sizeof(T), s)) return rc;
