@@ -14,7 +14,8 @@ The dominant kernel's own average duration (the MFMA core, without the
 operand-preparation kernels) comes from the library's event hook
 (ugemm_hip_timing_*), recorded on the same stream.
 
-Also reported (one JSON line in total):
+Also reported (one JSON line in total, with the main figures; all of them in
+the [detail] line on stderr):
   * errors of every form vs an FP64 evaluation of 64 sampled rows;
   * config 2's grid: 2048^3, 4096^3, 8192^3 x NN/NT/TN for FP32, BF16x3 and
     FP16X3, each cell with its roofline fraction and errors;
@@ -883,6 +884,33 @@ def load_counters(form):
         return None
 
 
+# Left out of the printed line (whole, 28 KB: readers that keep the last 12 KB
+# of an output lost its start).  Every figure stands in the [detail] line on stderr.
+SECTIONS = ("config2_grid", "config3", "config4_batched", "config4_as_convolutions", "split_k", "blas12",
+            "host_pointer_path", "config5_precision_ladder")
+DETAIL = {"ms_median", "ms_min", "wall_s", "max_abs_err", "max_err_over_bound_scale", "core_kernel", "core_ms",
+          "frac_of_fp32_vector_peak"}
+SECTION_DETAIL = DETAIL | {"max_rel_err", "rms_abs_err", "core_tflops", "roofline_peak", "mfma_issue_frac", "note",
+                           "mfma_utilisation", "ms_per_call", "operands", "resident_operand_bytes", "gemms_per_s",
+                           "frac_of_single_large_gemm_rate"}
+
+
+def summary(line):
+    """The line with sections and forms cut to their main figures, numbers to five digits."""
+    def cut(x, drop):
+        if isinstance(x, dict):
+            return {k: cut(v, drop) for k, v in x.items() if k not in drop}
+        if isinstance(x, list):
+            return [cut(v, drop) for v in x]
+        return float(f"{x:.5g}") if isinstance(x, float) else x
+    out = dict(line, forms=cut(line["forms"], DETAIL))
+    out.update({k: cut(line[k], SECTION_DETAIL) for k in SECTIONS if k in line})
+    if "config2_grid" in out:   # 27 cells: rate and mean relative error of each
+        out["config2_grid"] = {k: [c["tflops"], c["mean_rel_err"]] if "mean_rel_err" in c else c
+                               for k, c in out["config2_grid"].items()}
+    return out
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -1047,7 +1075,8 @@ def main():
         del A5, B5, C5
     if not args.no_cpu:
         line["cpu_baseline"] = cpu_baseline(n, args.cpu_seconds, with_config1=not args.quick)
-    print(json.dumps(line), flush=True)
+    log("[detail] " + json.dumps(line))
+    print(json.dumps(summary(line)), flush=True)
 
 
 if __name__ == "__main__":
