@@ -33,8 +33,9 @@ constexpr int LDS_PAD = 4;   // floats; keeps rows 16-byte aligned
 // start at even registers, the fragments' as well as these, so a(i), b(j) and
 // acc(i, j) could share a bank only if one quad started an odd distance from
 // another in j: the rotation rules that out.  Left to the register allocator,
-// 1-13% of the FMAs of a kernel had the conflict, and any change of the code
-// around the loop moved that share.
+// 3-14% of the FMAs of a GEMM or convolution kernel had the conflict (counted in
+// the assembly of each, 60 kernels; none has it now), and any change of the
+// code around the loop moved that share.
 template <int TM, int TN>
 __device__ __forceinline__ void pin_step(float (&acc)[TM][TN]) {
     typedef float quad __attribute__((ext_vector_type(4)));

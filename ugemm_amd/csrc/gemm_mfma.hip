@@ -1711,8 +1711,9 @@ int mfma_pick_variant(const Gemm<float> &g, int mode, bool fusable, int *splits)
 }
 
 // ---------------------------------------------------------------------------
-// Grouped split-form plans (grouped.hip): any variant (no operand is split
-// in the core here); the FP16 form adds the row-maximum pass.
+// Grouped split-form plans (grouped.hip): any variant, on planes of both
+// operands, or those that split B in the core; the FP16 form adds the row-maximum
+// pass.
 namespace {
 template <class CF, int FB = FUSE_NONE>
 int grouped_core(const PrepJob *jobs, const int *block_job, int prep_blocks, const GroupedSplitProblem *probs,

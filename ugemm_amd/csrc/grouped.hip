@@ -164,7 +164,7 @@ using G1K8 = Fp32Cfg<32, 64, 16, 4, 4, 1, 8>;
 // problem's last rows where it covers them.
 constexpr int kNumVariants = 5, kMixed = 4;
 // The same five tile choices on the FP32 matrix cores (UGEMM_MODE_FP32_MFMA
-// plans), 4 waves each; variant 4 mixes GM0 and GM3 per problem.
+// plans), 4 waves a group; variant 4 mixes GM0 and GM3 likewise.
 using GM0 = M32Cfg<128, 128, 16, 2, 2>;
 using GM1 = M32Cfg<64, 64, 16, 2, 2>;
 using GM2 = M32Cfg<128, 64, 16, 2, 2>;
@@ -206,9 +206,9 @@ VariantOps variant_ops(int mode, int v, int groups) {
 }
 
 const char *kGroupedNames[] = {"fp32_128x128x16_t8x8", "fp32_64x64x16_t4x4", "fp32_128x64x16_t8x4",
-                               "fp32_64x128x16_t4x8", "fp32_mixed_128x128_or_64x128_per_problem"};
+                               "fp32_64x128x16_t4x8", "fp32_mixed_128x128_64x128_last_rows"};
 const char *kGroupedM32Names[] = {"f32_mfma_128x128x16_w2x2", "f32_mfma_64x64x16_w2x2", "f32_mfma_128x64x16_w2x2",
-                                  "f32_mfma_64x128x16_w2x2", "f32_mfma_mixed_128x128_or_64x128_per_problem"};
+                                  "f32_mfma_64x128x16_w2x2", "f32_mfma_mixed_128x128_64x128_last_rows"};
 
 }  // namespace
 

@@ -31,8 +31,8 @@ __global__ __launch_bounds__(CF::THREADS, CF::MINB) void sgemm_fp32_kernel(int M
 // Implicit-GEMM convolution: C (M = output channels x N = output pixels) =
 // alpha * W (M x K, row-major weights) * im2col(in) + beta * C, then the
 // epilogue.  The column matrix is gathered in the tile loader (ConvDesc).
-// Split-K as in sgemm_fp32_kernel: the chunk's rows of the offset table
-// (absolute image offsets) and its weight columns.
+// Split-K as in sgemm_fp32_kernel: the chunk's weight columns, and cd.k0, from
+// which its k count (ConvRegs).
 template <class CF>
 __global__ __launch_bounds__(CF::THREADS) void conv_fp32_kernel(int M, int N, int K, float alpha,
                                                            const float *__restrict__ A, long lda, float beta,

@@ -42,8 +42,8 @@ __global__ __launch_bounds__(CF::THREADS, CF::MINB) void sgemm_mfma32_kernel(
 // Implicit-GEMM convolution on the FP32 matrix cores: C (M = output
 // channels x N = output pixels) = W (M x K, row-major weights) * im2col(in),
 // then the epilogue; the column matrix is gathered in the tile loader
-// (ConvDesc).  Split-K: the chunk's rows of the offset table and its weight
-// columns, as in the GEMM kernel.
+// (ConvDesc).  Split-K as in the GEMM kernel: the chunk's weight columns, and
+// cd.k0, from which its k count (ConvRegs).
 template <class CF>
 __global__ __launch_bounds__(CF::THREADS, CF::MINB) void conv_mfma32_kernel(
     int M, int N, int K_, const float *__restrict__ A_, long lda, float *__restrict__ C_, long ldc_, int tiles_m,
@@ -190,9 +190,8 @@ int m32_pick_variant(const Gemm<float> &g) {
     if (t128 <= cus) return v;
     // As fp32_pick_variant, over the same 60 sizes: 1.19 times as fast on
     // average as by the count of 256x128 tiles alone.
-    static const TileCost cost[6] = {{128, 128, 62, 0.47}, {256, 128, 58.5, 0.3}, {128, 256, 58.5, 0.3},
-                                     {64, 64, 70, 1.1},    {256, 256, 62, 0.1},   {128, 128, 68, 0.3}};
-    return cheapest_tile(cost, 6, 1 << 4 | 1 << 5, v, g.M, g.N);
+    static const TileCost cost[4] = {{128, 128, 62, 0.47}, {256, 128, 58.5, 0.3}, {128, 256, 58.5, 0.3}, {64, 64, 70, 1.1}};
+    return cheapest_tile(cost, 4, 0, v, g.M, g.N);
 }
 
 // g: the convolution as a GEMM (alpha 1, beta 0, A the weights, B unused).
