@@ -1683,8 +1683,8 @@ int mfma_pick_variant(const Gemm<float> &g, int mode, bool fusable, int *splits)
     const int fixed = mfma_fixed_variant(g);
     if (*splits > 0 || g.K <= 0) return fixed;
     // Fewer: tile and splits together.  493x2304x34854 BF16X3 ran 288 blocks
-    // of V3 in 877 us, one wave a SIMD and two blocks on a few CUs; V6 in 12
-    // splits takes 285.  1024x1024x4096 54 and 47 (V7 in 4), 64x6272x6592 91
+    // of V3 in 877 us, one wave a SIMD and two blocks on a few CUs; V4 in 14
+    // splits takes 270.  1024x1024x4096 54 and 47 (V7 in 4), 64x6272x6592 91
     // and 53 (V7 in 8, which splits B in the core), 5120x111x6405 93 and 48.
     // Near ties stay with the fixed choice and its own split count.  What that
     // runs within the scratch of the no-allocation entry stays within it, and

@@ -253,7 +253,16 @@ int launch_splitk_reduce_f64(int M, int N, int splits, double alpha, const doubl
 // grouped plans do not provide.
 int grouped_variant_count(int mode);
 
+// The built-in choice of a form (runtime.hip): its variant (-1: the launcher
+// picks), and with *splits == 0 the split count to run it with (0 left: the
+// variant's own rule).
+int automatic_variant(const Gemm<float> &g, int mode, int *splits);
+
 // ---- tuning (tune.hip) ----
+// What the tuner times for a product: the built-in choice first, whose split
+// count may be any, then every variant by itself and with set split counts.
+// variants and splits: room for most; the number of candidates.
+int tune_candidates(int mode, int ta, int tb, int M, int N, int K, int most, int *variants, int *splits);
 // Tuning-table key of grouped plans (variants = grouped_variant_count(mode)).
 constexpr int TUNE_KEY_GROUPED = 16;
 // ta, tb: layout flags (grouped keys: convolution flag, split form).

@@ -453,14 +453,7 @@ static int normalize(char major, char transa, char transb, int M, int N, int K, 
 
 // ---------------------------------------------------------------------------
 // Device-pointer execution of a normalised GEMM.
-// Variant and split-K count: forced (ugemm_hip_force_variant/_splits), else
-// the tuning table's entry for the shape bucket, else the built-in choice.
-static int choose_variant(const Gemm<float> &g, int mode, int *splits) {
-    int v = forced_variant(mode), tsplits = 0;
-    const int fs = forced_splits(mode);
-    if (v < 0) v = tuned_variant(mode, g.ta, g.tb, g.M, g.N, g.K, &tsplits);
-    *splits = fs > 0 ? fs : tsplits;
-    if (v >= 0) return v;
+int automatic_variant(const Gemm<float> &g, int mode, int *splits) {
     switch (mode) {
         case UGEMM_MODE_FP32: return fp32_pick_variant(g);
         case UGEMM_MODE_FP32_MFMA: return m32_pick_variant(g);
@@ -469,6 +462,17 @@ static int choose_variant(const Gemm<float> &g, int mode, int *splits) {
             // Small grids in one launch: variant 3's automatic choice.
             return *splits == 0 && split_small_tile(g, mode) ? 3 : mfma_pick_variant(g, mode, true, splits);
     }
+}
+
+// Variant and split-K count: forced (ugemm_hip_force_variant/_splits), else
+// the tuning table's entry for the shape bucket, else the built-in choice.
+static int choose_variant(const Gemm<float> &g, int mode, int *splits) {
+    int v = forced_variant(mode), tsplits = 0;
+    const int fs = forced_splits(mode);
+    if (v < 0) v = tuned_variant(mode, g.ta, g.tb, g.M, g.N, g.K, &tsplits);
+    *splits = fs > 0 ? fs : tsplits;
+    if (v >= 0) return v;
+    return automatic_variant(g, mode, splits);
 }
 
 int run_sgemm(const Gemm<float> &g, int mode, int variant, hipStream_t s) {
