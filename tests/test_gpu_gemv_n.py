@@ -72,3 +72,38 @@ def test_gemv_n_of_nearly_2_to_the_31_columns():
     for d in ones:
         d.free()
     assert abs(got - N) <= 32 * 64, got
+
+
+def plain_sums(A, x, chunk=64):
+    """A^T x by one thread a row: chunks of columns on four accumulators (one
+    rounding a multiply-add), the chunks' sums one after the other."""
+    wide = np.float64 if A.dtype == np.float32 else np.longdouble
+    y = np.zeros(A.shape[1], A.dtype)
+    for c in range(0, len(x), chunk):
+        s = [np.zeros_like(y) for _ in range(4)]
+        for n in range(c, min(c + chunk, len(x))):
+            i = (n - c) % 4
+            s[i] = (A[n].astype(wide) * wide(x[n]) + s[i]).astype(A.dtype)
+        y = y + ((s[0] + s[1]) + (s[2] + s[3]))
+    return y
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_gemv_n_sums_of_few_columns_are_no_less_exact(dtype):
+    """The waves' sums are added in pairs: the root mean square error over rows
+    of 128 to 250 columns stays below that of a thread's own sums."""
+    wide = np.float64 if dtype == np.float32 else np.longdouble
+    got = want = 0.0
+    for N in (128, 160, 200, 250):
+        for seed in range(5):
+            g = np.random.default_rng(1000 * N + seed)
+            A, x = g.standard_normal((N, 400)).astype(dtype), g.standard_normal(N).astype(dtype)
+            exact = x.astype(wide) @ A.astype(wide)
+            dA, dx, dy = hip.DeviceArray.from_host(A), hip.DeviceArray.from_host(x), hip.DeviceArray(400, dtype)
+            ug.gemv_dev("N", 400, N, 1.0, dA, 400, dx, 1, 0.0, dy, 1, double=dtype == np.float64)
+            hip.synchronize()
+            # Relative to sqrt(N), which the errors of both grow with.
+            got += float(np.sum((dy.download() - exact) ** 2)) / N
+            want += float(np.sum((plain_sums(A, x) - exact) ** 2)) / N
+    print(f"{np.dtype(dtype).name}: {np.sqrt(got / want):.3f} of the plain sums' error")
+    assert got <= want
